@@ -13,9 +13,10 @@
 // counter, atomic or cross-workgroup fence.  The (r,z)/(r,r) partials
 // alternate between two buffers by iteration parity, so iteration j still
 // sees rho_{j-2} for beta.  The stop test of ConjugateGradients::x runs at
-// the start of both kernels of the next iteration; once it holds, the
-// remaining launches are no-ops and workgroup 0 records the final state,
-// which the host reads every few iterations.  Results are deterministic.
+// the start of the next iteration's SpMV; once it holds, the remaining
+// launches are no-ops and workgroup 0 has recorded the final state, also
+// in pinned host memory, where the host looks once per batch of iterations.
+// Results are deterministic.
 //
 // SpMV of the recurrences (CG and flexible CG): tiles of consecutive rows (at
 // most 2048 nonzeros in FP64, 4096 in FP32); a workgroup forms a tile's
@@ -49,6 +50,12 @@ constexpr int kMaxParts = 2048;
 template <class T>
 constexpr int tile_nnz() { return sizeof(T) == 4 ? 4096 : 2048; }
 
+// workgroups of a SpMV launch: four per CU, so that a launch of more than
+// 1024 tiles walks them evenly with the next tile's loads in flight (per
+// iteration of Jacobi-PCG with one workgroup per tile, at most 2048: 29.8 us
+// at 64^3 and 68 us at 100^3; 1280: 29.5 and 71; 1024: 27.8 and 65.3; 768:
+// 27.8 and 65.8; 512: 29.1 and 71.6)
+constexpr int kSpmvGrid = 1024;
 constexpr int kVecParts = 512;    // workgroups of the vector kernels (max)
 constexpr int kBufLen = 2 * kVecParts + 8;   // rz[.], rr[.], finished flag
 
@@ -75,8 +82,9 @@ struct CgSolver {
   std::vector<DevArr> allocs;
   int *dia = nullptr, *dja = nullptr;
   int ntile = 0, ntile32 = 0;
-  int* dtile = nullptr;          // first row of each FP64 SpMV tile (ntile + 1)
-  int* dtile32 = nullptr;        // the same for the FP32 products
+  int4* dtile = nullptr;         // FP64 SpMV tiles: first row, row end, first
+                                 // nonzero, nonzeros
+  int4* dtile32 = nullptr;       // the same for the FP32 products
   double* da = nullptr;          // values as used by the solve
   float* da32 = nullptr;         // FP32 copy for the mixed-precision inner solve
   double *x = nullptr, *b = nullptr, *r = nullptr, *z = nullptr, *d = nullptr;
@@ -92,6 +100,8 @@ struct CgSolver {
   double* rzb = nullptr;         // 2 x kBufLen partials of (r,z), (r,r)
   CgState* st = nullptr;
   CgState* hst = nullptr;        // pinned host mirror
+  CgState* hpub = nullptr;       // pinned: the final state, written by the device
+  hipEvent_t ev[2] = {nullptr, nullptr};   // ends of the enqueued batches
   DevArr bcbuf;                  // Dirichlet rows/values of xg_cg_init_dev
   int pc = 0;
   bool ready = false;            // setup done
@@ -153,31 +163,51 @@ __device__ inline void put_part(double* part, int k, double v, double* sm) {
   if (threadIdx.x == 0) part[k] = s;
 }
 
-// The stop test of ConjugateGradients::x (ConjugateGradients.cpp:772-823)
-// after iteration it = j-1, from that iteration's (r,r) and finished flag.
-struct StopTest {
-  double rz, rr;
-  bool stop, converged;
-};
-
-__device__ inline StopTest stop_test(const double* __restrict__ buf, int nvp, int j,
-                                     long long maxit, double tol_nb, double* sm) {
-  StopTest s;
-  s.rz = sum_parts(buf, nvp, sm);
-  s.rr = sum_parts(buf + kVecParts, nvp, sm);
-  const bool finished = buf[2 * kVecParts] != 0.0;
-  const double normr = sqrt(s.rr);
-  s.stop = j >= 2 && (finished || normr < tol_nb || (long long)(j - 1) >= maxit);
-  s.converged = !(normr > tol_nb);
-  return s;
+// K sums at once, each as sum_parts takes it (the same order and tree, so the
+// same bits), with one exchange through LDS: v[k] holds this thread's part.
+template <int K>
+__device__ inline void block_sums_all(double v[K], double (*sm)[kCgThreads / 64]) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += __shfl_xor(v[k], o, 64);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < K; ++k) sm[k][threadIdx.x >> 6] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < kCgThreads / 64; ++w) s += sm[k][w];
+    v[k] = s;
+  }
 }
 
-__device__ inline void record_stop(CgState* st, int j, const StopTest& s) {
-  if (blockIdx.x == 0 && threadIdx.x == 0 && !st->done) {
+// this thread's part of sum_parts
+__device__ inline double part_of(const double* __restrict__ part, int n) {
+  double v = 0.0;
+  for (int i = threadIdx.x; i < n; i += kCgThreads) v += part[i];
+  return v;
+}
+
+// The stop of ConjugateGradients::x (ConjugateGradients.cpp:772-823) after
+// iteration j - 1: the final state for the later launches of the batch
+// (which become no-ops) and, in pinned memory, for the host.
+__device__ inline void record_stop(CgState* st, CgState* pub, int j, double rr, double normr,
+                                   double tol_nb) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const int conv = !(normr > tol_nb) ? 1 : 0;
     st->it = j - 1;
-    st->rr = s.rr;
-    st->converged = s.converged ? 1 : 0;
+    st->rr = rr;
+    st->converged = conv;
     st->done = 1;
+    volatile CgState* h = pub;
+    h->it = j - 1;
+    h->rr = rr;
+    h->converged = conv;
+    __threadfence_system();
+    h->done = 1;
   }
 }
 
@@ -254,48 +284,78 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_setup_final(
 // ConjugateGradients' CSR::mult); row(r, p_r, q_r) is called once per row,
 // by that thread (thread 0 for a row longer than a tile).  Every thread of
 // the workgroup calls this (it holds barriers).
-template <class T, class Row>
-__device__ inline void tiles_spmv(int ntile, const int* __restrict__ tile,
+//
+// Up to some 600,000 rows a launch has one tile per workgroup and its time
+// is a chain of dependent loads, not bytes: so the tile's record comes in
+// one load, a thread's whole share of the tile is in flight before anything
+// is waited for, and coef() -- the scalars, themselves sums over the last
+// kernel's partials -- runs while it is; on larger systems the next tile's
+// share is loaded while the current one's rows are summed.
+template <class T, class Coef, class Row>
+__device__ inline bool tiles_spmv(int ntile, const int4* __restrict__ tile,
                                   const int* __restrict__ ia, const int* __restrict__ ja,
-                                  const T* __restrict__ a, const T* __restrict__ zp, T bt,
-                                  T* prod, double* sm, Row row) {
+                                  const T* __restrict__ a, const T* __restrict__ zp,
+                                  T* prod, double* sm, Coef coef, Row row) {
   constexpr int kTileNnz = tile_nnz<T>();
+  constexpr int kShare = kTileNnz / kCgThreads;   // products of a thread
+  constexpr int kGather = 4;                      // gathers in flight
   const Pair<T>* zpp = reinterpret_cast<const Pair<T>*>(zp);
   const int t = threadIdx.x;
+  unsigned cc[kShare];
+  T av[kShare];
+  int4 W = make_int4(0, 0, 0, 0);
+  int e0 = 0, e1 = 0;
+  // loads past the end of the tile are of its last entry: no branch between
+  // the loads
+  auto fetch = [&](int ti) {
+    if (ti >= ntile) return;
+    W = tile[ti];
+    if (W.w > kTileNnz) return;
+    const unsigned last = (unsigned)max(W.w, 1) - 1;
+    const int* jt = ja + W.z;
+    const T* at = a + W.z;
+#pragma unroll
+    for (int u = 0; u < kShare; ++u) {
+      const unsigned kk = min((unsigned)(t + u * kCgThreads), last);
+      cc[u] = (unsigned)jt[kk];
+      av[u] = at[kk];
+    }
+    const unsigned r = min((unsigned)t, (unsigned)(W.y - W.x - 1));
+    const int* it = ia + W.x;
+    e0 = it[r] - W.z;
+    e1 = it[r + 1] - W.z;
+  };
+  fetch(blockIdx.x);
+  T bt;
+  if (!coef(bt)) return false;
   for (int ti = blockIdx.x; ti < ntile; ti += gridDim.x) {
-    const int r0 = tile[ti], r1 = tile[ti + 1];
-    const int k0 = ia[r0], nz = ia[r1] - k0;
+    const int r0 = W.x, r1 = W.y, k0 = W.z, nz = W.w;
     if (nz <= kTileNnz) {
-      for (int k = t; k < nz; k += 4 * kCgThreads) {
-        int cc[4];
-        T av[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int kk = k + u * kCgThreads;
-          cc[u] = kk < nz ? ja[k0 + kk] : 0;
-          av[u] = kk < nz ? a[k0 + kk] : T(0);
-        }
-        T zv[4], pv[4];
+      for (int u0 = 0; u0 < kShare; u0 += kGather) {
+        Pair<T> v[kGather];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const Pair<T> v = zpp[cc[u]];
-          zv[u] = v.z;
-          pv[u] = v.p;
-        }
+        for (int u = 0; u < kGather; ++u) v[u] = zpp[cc[u0 + u]];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int kk = k + u * kCgThreads;
-          if (kk < nz) prod[kk] = av[u] * (zv[u] + bt * pv[u]);
-        }
+        for (int u = 0; u < kGather; ++u)
+          prod[t + (u0 + u) * kCgThreads] = av[u0 + u] * (v[u].z + bt * v[u].p);
       }
+      const int f0 = e0, f1 = e1, r = r0 + t;
+      Pair<T> own = {};
+      if (r < r1) own = zpp[r];
+      fetch(ti + gridDim.x);
       __syncthreads();
-      const int r = r0 + t;
       if (r < r1) {
-        const int e0 = ia[r] - k0, e1 = ia[r + 1] - k0;
         T acc = T(0);
-        for (int k = e0; k < e1; ++k) acc += prod[k];
-        const Pair<T> v = zpp[r];
-        row(r, v.z + bt * v.p, acc);
+        for (int k = f0; k < f1; k += 8) {
+          T v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) v[u] = prod[min(k + u, kTileNnz - 1)];
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (k + u < f1) acc += v[u];
+        }
+        row(r, own.z + bt * own.p, acc);
       }
       __syncthreads();        // prod is the next tile's
     } else {
@@ -310,76 +370,133 @@ __device__ inline void tiles_spmv(int ntile, const int* __restrict__ tile,
         const Pair<T> v = zpp[r0];
         row(r0, v.z + bt * v.p, (T)sum);
       }
+      fetch(ti + gridDim.x);
     }
   }
+  return true;
 }
 
 // iteration j, first half: p_j = z + beta p_{j-1} (both read from the (z, p)
 // pairs the previous update wrote), q = A p_j, partials of
-// (p_j, q) (ConjugateGradients::next/qAp, :585-635)
+// (p_j, q) (ConjugateGradients::next/qAp, :585-635).  The stop test of
+// ConjugateGradients::x after iteration j - 1 runs here: every workgroup
+// takes the same sums and the first one records the stop, which the update
+// kernel of this iteration and all later launches of the batch read.
+// An iteration (this and k_cg_update) moves 12 nnz + 44 n bytes of matrix
+// and pairs and 76 n of vectors in FP64: 15 us at 64^3 (274,625 rows) at the
+// copy rate, 27.8 us measured (37 before the loads were put ahead of the
+// scalars); 65 us at 100^3, 81 before.
 template <class T>
 __global__ __launch_bounds__(kCgThreads) void k_cg_spmv(
-    int j, int ntile, const int* __restrict__ tile, const int* __restrict__ ia,
+    int j, int ntile, const int4* __restrict__ tile, const int* __restrict__ ia,
     const int* __restrict__ ja, const T* __restrict__ a, const T* __restrict__ zp,
     T* __restrict__ pnew, T* __restrict__ q,
     const double* __restrict__ rzb, int nvp, double* __restrict__ pq, CgState* st,
-    long long maxit, double tol_nb) {
+    CgState* pub, long long maxit, double tol_nb) {
   constexpr int kTileNnz = tile_nnz<T>();
-  __shared__ double sm[kCgThreads / 64];
+  __shared__ double sm[3][kCgThreads / 64];
   __shared__ T prod[kTileNnz];
-  // after the stop the partial sums of the two buffers are one update apart
-  // from each other no more: every later launch of the batch is a no-op
-  if (st->done) return;
-  const StopTest s = stop_test(rzb + ((j - 1) & 1) * kBufLen, nvp, j, maxit, tol_nb, sm);
-  if (s.stop) {
-    record_stop(st, j, s);
-    return;
-  }
-  double beta = 0.0;   // the reference's m_alpha = rho/rho0 (:590)
-  if (j >= 2) beta = s.rz / sum_parts(rzb + (j & 1) * kBufLen, nvp, sm);
-  const T bt = (T)beta;
+  const int done = st->done;
   double spq = 0.0;
-  tiles_spmv<T>(ntile, tile, ia, ja, a, zp, bt, prod, sm, [&](int r, T pr, T qr) {
-    pnew[r] = pr;
-    q[r] = qr;
-    spq += (double)pr * (double)qr;
-  });
-  put_part(pq, blockIdx.x, spq, sm);
+  const bool ran = tiles_spmv<T>(
+      ntile, tile, ia, ja, a, zp, prod, sm[0],
+      [&](T& bt) {
+        const double* cur = rzb + ((j - 1) & 1) * kBufLen;
+        const double* old = rzb + (j & 1) * kBufLen;
+        const bool finished = cur[2 * kVecParts] != 0.0;
+        double v[3] = {part_of(cur, nvp), part_of(cur + kVecParts, nvp),
+                       j >= 2 ? part_of(old, nvp) : 0.0};
+        if (done) return false;
+        block_sums_all<3>(v, sm);
+        const double normr = sqrt(v[1]);
+        if (j >= 2 && (finished || normr < tol_nb || (long long)(j - 1) >= maxit)) {
+          record_stop(st, pub, j, v[1], normr, tol_nb);
+          return false;
+        }
+        bt = j >= 2 ? (T)(v[0] / v[2]) : T(0);   // the reference's m_alpha = rho/rho0 (:590)
+        return true;
+      },
+      [&](int r, T pr, T qr) {
+        pnew[r] = pr;
+        q[r] = qr;
+        spq += (double)pr * (double)qr;
+      });
+  if (ran) put_part(pq, blockIdx.x, spq, sm[0]);
 }
+
+// V consecutive values of a vector, 16 bytes: one load or store
+template <class T>
+struct alignas(16) Vec {
+  static constexpr int V = 16 / sizeof(T);
+  T v[V];
+};
 
 // iteration j, second half (ConjugateGradients::pq/rz, :672-750): alpha,
 // r -= alpha q, z = r/d, x += alpha p_j; partials of (r,z), (r,r) and the
-// finished flag into buffer j & 1
+// finished flag into buffer j & 1.  z goes only into the (z, p) pairs that
+// the next SpMV gathers.  16-byte loads, those of a thread's first values
+// in flight while alpha is summed.
 template <class T>
 __global__ __launch_bounds__(kCgThreads) void k_cg_update(
     int j, int64_t n, const T* __restrict__ q, const T* __restrict__ d,
-    const T* __restrict__ p, T* __restrict__ r, T* __restrict__ z, T* __restrict__ x,
+    const T* __restrict__ p, T* __restrict__ r, T* __restrict__ x,
     T* __restrict__ zp, double* __restrict__ rzb, int nvp, const double* __restrict__ pq,
-    int nsp, const CgState* st, long long maxit, double tol_nb, double brk) {
-  __shared__ double sm[kCgThreads / 64];
-  if (st->done) return;
-  const StopTest s = stop_test(rzb + ((j - 1) & 1) * kBufLen, nvp, j, maxit, tol_nb, sm);
-  if (s.stop) return;
-  const double PQ = sum_parts(pq, nsp, sm);
-  const bool finished = fabs(PQ) < brk;        // ConjugateGradients.cpp:680-687
-  const double alpha = finished ? 0.0 : s.rz / PQ;
+    int nsp, const CgState* st, double brk) {
+  constexpr int V = Vec<T>::V;
+  __shared__ double sm[2][kCgThreads / 64];
+  const int done = st->done;  // the stop test of this iteration's SpMV
+  const int64_t nv = n / V, step = (int64_t)gridDim.x * kCgThreads;
+  int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
+  Vec<T> rv, qv, dv, pv, xv;
+  auto load = [&](int64_t k) {
+    rv = reinterpret_cast<const Vec<T>*>(r)[k];
+    qv = reinterpret_cast<const Vec<T>*>(q)[k];
+    dv = reinterpret_cast<const Vec<T>*>(d)[k];
+    pv = reinterpret_cast<const Vec<T>*>(p)[k];
+    xv = reinterpret_cast<const Vec<T>*>(x)[k];
+  };
+  if (i < nv) load(i);
+  double v[2] = {part_of(rzb + ((j - 1) & 1) * kBufLen, nvp), part_of(pq, nsp)};
+  if (done) return;
+  block_sums_all<2>(v, sm);
+  const bool finished = fabs(v[1]) < brk;      // ConjugateGradients.cpp:680-687
+  const double alpha = finished ? 0.0 : v[0] / v[1];
   const T al = (T)alpha;
   double rz = 0.0, rr = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kCgThreads) {
-    const T ri = r[i] - al * q[i];
-    const T zi = ri / d[i];
-    const T pi = p[i];
-    r[i] = ri;
-    z[i] = zi;
-    x[i] += al * pi;
-    reinterpret_cast<Pair<T>*>(zp)[i] = Pair<T>{zi, pi};   // the next SpMV's gathers
+  while (i < nv) {
+    Pair<T> o[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const T ri = rv.v[k] - al * qv.v[k];
+      const T zi = ri / dv.v[k];
+      rv.v[k] = ri;
+      xv.v[k] += al * pv.v[k];
+      o[k] = Pair<T>{zi, pv.v[k]};
+      rz += (double)ri * (double)zi;
+      rr += (double)ri * (double)ri;
+    }
+    reinterpret_cast<Vec<T>*>(r)[i] = rv;
+    reinterpret_cast<Vec<T>*>(x)[i] = xv;
+#pragma unroll
+    for (int k = 0; k < V; ++k) reinterpret_cast<Pair<T>*>(zp)[i * V + k] = o[k];
+    i += step;
+    if (i < nv) load(i);
+  }
+  // the last n mod V rows
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x < n - nv * V) {
+    const int64_t k = nv * V + threadIdx.x;
+    const T ri = r[k] - al * q[k];
+    const T zi = ri / d[k];
+    const T pi = p[k];
+    r[k] = ri;
+    x[k] += al * pi;
+    reinterpret_cast<Pair<T>*>(zp)[k] = Pair<T>{zi, pi};
     rz += (double)ri * (double)zi;
     rr += (double)ri * (double)ri;
   }
   double* out = rzb + (j & 1) * kBufLen;
-  put_part(out, blockIdx.x, rz, sm);
-  put_part(out + kVecParts, blockIdx.x, rr, sm);
+  put_part(out, blockIdx.x, rz, sm[0]);
+  put_part(out + kVecParts, blockIdx.x, rr, sm[1]);
   if (blockIdx.x == 0 && threadIdx.x == 0) out[2 * kVecParts] = finished ? 1.0 : 0.0;
 }
 
@@ -527,28 +644,33 @@ __global__ __launch_bounds__(kCgThreads) void k_fcg_pack_dot(
 // (z_k, q_{k-1}) partials, `prev` the (p,q) partials of iteration k-1 (the
 // buffers alternate by iteration parity, so nothing read is overwritten).
 __global__ __launch_bounds__(kCgThreads) void k_fcg_spmv(
-    int first, int ntile, const int* __restrict__ tile, const int* __restrict__ ia,
+    int first, int ntile, const int4* __restrict__ tile, const int* __restrict__ ia,
     const int* __restrict__ ja, const double* __restrict__ a, const double* __restrict__ zp,
     double* __restrict__ pnew, double* __restrict__ q, const double* __restrict__ r,
     const double* __restrict__ prev, double* __restrict__ cur, int nvp, int nsp) {
-  __shared__ double sm[kCgThreads / 64];
+  __shared__ double sm[2][kCgThreads / 64];
   __shared__ double prod[tile_nnz<double>()];
-  double beta = 0.0;
-  if (!first) {
-    const double zq = sum_parts(cur, nvp, sm);                 // (z, q_prev)
-    const double pq = sum_parts(prev + kMaxParts, nsp, sm);    // (p, q)_prev
-    beta = pq != 0.0 ? -zq / pq : 0.0;
-  }
   double spq = 0.0, spr = 0.0;
-  tiles_spmv<double>(ntile, tile, ia, ja, a, zp, beta, prod, sm,
-                     [&](int row, double pr, double qr) {
-                       pnew[row] = pr;
-                       q[row] = qr;
-                       spq += pr * qr;
-                       spr += pr * r[row];
-                     });
-  put_part(cur + kMaxParts, blockIdx.x, spq, sm);
-  put_part(cur + 2 * kMaxParts, blockIdx.x, spr, sm);
+  tiles_spmv<double>(
+      ntile, tile, ia, ja, a, zp, prod, sm[0],
+      [&](double& beta) {
+        double v[2] = {0.0, 0.0};                 // (z, q_prev), (p, q)_prev
+        if (!first) {
+          v[0] = part_of(cur, nvp);
+          v[1] = part_of(prev + kMaxParts, nsp);
+        }
+        block_sums_all<2>(v, sm);
+        beta = v[1] != 0.0 ? -v[0] / v[1] : 0.0;
+        return true;
+      },
+      [&](int row, double pr, double qr) {
+        pnew[row] = pr;
+        q[row] = qr;
+        spq += pr * qr;
+        spr += pr * r[row];
+      });
+  put_part(cur + kMaxParts, blockIdx.x, spq, sm[0]);
+  put_part(cur + 2 * kMaxParts, blockIdx.x, spr, sm[1]);
 }
 
 // alpha = (p,r)/(p,q); x += alpha p; r -= alpha q; partials of (r,r)
@@ -612,6 +734,9 @@ void free_solver(CgSolver* s) {
   if (!s) return;
   dev_free_all(s->allocs);
   if (s->hst) (void)hipHostFree(s->hst);
+  if (s->hpub) (void)hipHostFree(s->hpub);
+  for (hipEvent_t e : s->ev)
+    if (e) (void)hipEventDestroy(e);
   if (s->bcbuf.p) (void)hipFree(s->bcbuf.p);
   delete s;
 }
@@ -668,40 +793,61 @@ int read_state(xg_ctx* c) {
 }
 
 // Iterations j = 1, 2, ... of the recurrence set up in buffer 0 of rzb, until
-// the stop test holds (at the latest at j = maxit + 1); the host checks the
-// state every `batch` iterations.  T: FP64 solve or the FP32 inner solve.
+// the stop test holds (at the latest at j = maxit + 1).  The kernel that
+// finds the stop writes the final state to pinned memory; the host looks at
+// it once per batch of iterations, and from the second batch on it enqueues
+// the next one before it waits, so the device is not idle meanwhile (a batch
+// enqueued past the stop is all no-ops).  The stream is drained before
+// this returns.  T: FP64 solve or the FP32 inner solve.
 template <class T>
 int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T* x,
            int64_t maxit, double tol_nb, double brk, int64_t jstart = 1) {
   CgSolver* s = c->cg;
   const bool f32 = sizeof(T) == 4;
   const int ntile = f32 ? s->ntile32 : s->ntile;
-  const int* dtile = f32 ? s->dtile32 : s->dtile;
-  const int gr = std::max(1, std::min(ntile, kMaxParts)), gv = grid_vec(s->nrow);
+  const int4* dtile = f32 ? s->dtile32 : s->dtile;
+  const int gr = std::max(1, std::min(ntile, kSpmvGrid)), gv = grid_vec(s->nrow);
   const int batch = 8;
   // the (z, p) pairs of the first SpMV; each update writes the next ones
   T* zp = f32 ? reinterpret_cast<T*>(s->zp32) : reinterpret_cast<T*>(s->zp);
+  s->hpub->done = 0;
   hipLaunchKernelGGL(k_pack_zp<T>, dim3((unsigned)((s->nrow + kCgThreads - 1) / kCgThreads)),
                      dim3(kCgThreads), 0, c->stream, s->nrow, z,
                      (jstart - 1) & 1 ? p1 : p0, zp);
-  for (int64_t j0 = jstart;; j0 += batch) {
-    if (j0 > maxit + 1 + batch)
-      return fail(c, XG_EHIP, "CG: stop test not reached on the device");
+  auto enqueue = [&](int64_t j0, int slot) -> int {
     for (int i = 0; i < batch; ++i) {
       const int j = (int)(j0 + i);
       T* pnew = j & 1 ? p1 : p0;
       hipLaunchKernelGGL(k_cg_spmv<T>, dim3(gr), dim3(kCgThreads), 0, c->stream, j,
                          ntile, dtile, s->dia, s->dja, a, zp, pnew, q, s->rzb, gv, s->pq,
-                         s->st, (long long)maxit, tol_nb);
+                         s->st, s->hpub, (long long)maxit, tol_nb);
       hipLaunchKernelGGL(k_cg_update<T>, dim3(gv), dim3(kCgThreads), 0, c->stream, j,
-                         s->nrow, q, d, pnew, r, z, x, zp, s->rzb, gv, s->pq, gr, s->st,
-                         (long long)maxit, tol_nb, brk);
+                         s->nrow, q, d, pnew, r, x, zp, s->rzb, gv, s->pq, gr, s->st, brk);
     }
     XG_HIP(c, hipGetLastError());
-    int rc = read_state(c);
-    if (rc) return rc;
-    if (s->hst->done) return XG_OK;
+    XG_HIP(c, hipEventRecord(s->ev[slot], c->stream));
+    return XG_OK;
+  };
+  int rc = enqueue(jstart, 0);
+  if (rc) return rc;
+  int64_t enq = 1, waited = 0;   // batches enqueued, batches waited for
+  for (;;) {
+    XG_HIP(c, hipEventSynchronize(s->ev[waited & 1]));
+    ++waited;
+    if (static_cast<volatile CgState*>(s->hpub)->done) break;
+    // the stop test holds at the latest in the SpMV of iteration maxit + 1
+    while (enq < waited + 2 && jstart + enq * batch <= maxit + 1) {
+      if ((rc = enqueue(jstart + enq * batch, (int)(enq & 1)))) return rc;
+      ++enq;
+    }
+    if (enq == waited) return fail(c, XG_EHIP, "CG: stop test not reached on the device");
   }
+  XG_HIP(c, hipStreamSynchronize(c->stream));
+  s->hst->it = s->hpub->it;
+  s->hst->rr = s->hpub->rr;
+  s->hst->converged = s->hpub->converged;
+  s->hst->done = 1;
+  return XG_OK;
 }
 
 // ConjugateGradients::apply's Dirichlet rows (CSR::dirichlet in decreasing
@@ -846,7 +992,7 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
   // SpMV tiles: consecutive rows, at most kCgThreads rows and tnz nonzeros
   // each (a longer row alone)
   auto tiles = [&](int64_t tnz) {
-    std::vector<int32_t> tile(1, 0);
+    std::vector<int4> tile;
     for (int64_t r = 0; r < nrow;) {
       int64_t r1 = r, nz = 0;
       while (r1 < nrow && r1 - r < kCgThreads && nz + (s->ia[r1 + 1] - s->ia[r1]) <= tnz) {
@@ -854,14 +1000,14 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
         ++r1;
       }
       if (r1 == r) r1 = r + 1;
-      tile.push_back((int32_t)r1);
+      tile.push_back(make_int4((int)r, (int)r1, (int)s->ia[r], (int)(s->ia[r1] - s->ia[r])));
       r = r1;
     }
     return tile;
   };
-  const std::vector<int32_t> tile = tiles(tile_nnz<double>()), tile32 = tiles(tile_nnz<float>());
-  s->ntile = (int)(tile.size() - 1);
-  s->ntile32 = (int)(tile32.size() - 1);
+  const std::vector<int4> tile = tiles(tile_nnz<double>()), tile32 = tiles(tile_nnz<float>());
+  s->ntile = (int)tile.size();
+  s->ntile32 = (int)tile32.size();
   std::vector<float> a32(nnz);
   for (int64_t j = 0; j < nnz; ++j) a32[j] = (float)a[j];
   int rc;
@@ -902,6 +1048,17 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
     free_solver(s);
     return fail(c, XG_EHIP, "hipHostMalloc");
   }
+  if (hipHostMalloc((void**)&s->hpub, sizeof(CgState), hipHostMallocCoherent) != hipSuccess) {
+    s->hpub = nullptr;
+    free_solver(s);
+    return fail(c, XG_EHIP, "hipHostMalloc");
+  }
+  for (hipEvent_t& e : s->ev)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      e = nullptr;
+      free_solver(s);
+      return fail(c, XG_EHIP, "hipEventCreate");
+    }
   XG_HIP(c, hipMemset(s->x, 0, n * 8));
   XG_HIP(c, hipMemset(s->b, 0, n * 8));
   CgState z0;
@@ -1232,7 +1389,7 @@ int xg_cg_solve_flexible(xg_ctx* c, int pc_kind, int64_t inner, int64_t maxit,
   if (s->restore && (rc = restore_values(c))) return rc;
   const int64_t n = s->nrow;
   const int gr = grid_rows(n), gv = grid_vec(n);
-  const int gt = std::max(1, std::min(s->ntile, kMaxParts));   // FCG SpMV tiles
+  const int gt = std::max(1, std::min(s->ntile, kSpmvGrid));   // FCG SpMV tiles
   hipLaunchKernelGGL(k_cg_residual, dim3(gr), dim3(kCgThreads), 0, c->stream, n,
                      s->dia, s->dja, s->da, s->x, s->b, s->r, s->d, s->pc);
   hipLaunchKernelGGL(k_f32_from_f64, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, n,
