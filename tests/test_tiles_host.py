@@ -1,0 +1,26 @@
+"""CPU check of the SpMV row tiles (xyst_amd/csrc/xg_tiles.cpp)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("tiles") / "tiles_check")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-pthread", "-o", out,
+                    os.path.join(ROOT, "tests", "cpp", "tiles_check.cpp"),
+                    os.path.join(ROOT, "xyst_amd", "csrc", "xg_tiles.cpp")], check=True)
+    return out
+
+
+@pytest.mark.parametrize("nrow,ncol,mean,nlong", [
+    (1, 1, 1, 0), (128, 128, 0, 0), (129, 300, 1, 0), (1000, 1000, 15, 0),
+    (3001, 5000, 15, 3), (4000, 2048, 100, 4), (200000, 200000, 15, 2)])
+def test_tiles_cover_the_matrix(exe, nrow, ncol, mean, nlong):
+    for seed in (1, 2):
+        r = subprocess.run([exe] + [str(v) for v in (nrow, ncol, mean, nlong, seed)],
+                           capture_output=True, text=True)
+        assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout

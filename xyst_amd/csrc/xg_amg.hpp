@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "xg_internal.hpp"
+#include "xg_tiles.hpp"
 
 namespace xg {
 
@@ -51,9 +52,24 @@ int amg_setup(int64_t n, const int64_t* ia, const int32_t* ja, const double* a,
 
 // Device side (xg_amg.hip), as seen by the CG driver.
 // (Re)builds and uploads the hierarchy for the matrix (n, ia, ja, a) when
-// `version` differs from the one uploaded.
+// `version` differs from the one uploaded; fine: the matrix' row tiles on the
+// device, which have to live as long as that version is applied.
 int xg_amg_prepare_internal(xg_ctx* c, int64_t n, const int64_t* ia, const int32_t* ja,
-                            const double* a, int64_t version);
-// z = V-cycle(S r) (FP32 inside), r and z FP64 device vectors of n
-int xg_amg_apply_internal(xg_ctx* c, const double* r, double* z);
+                            const double* a, int64_t version, const xg::TileMat& fine);
+// What the finest level of a V-cycle for the residual r (FP64) starts from:
+// b = sign r and its first sweep x = w dinv b, n rows, written by the caller.
+struct AmgInput {
+  int n;
+  const float *sign, *dinv;
+  float w;
+  float *b, *x;
+};
+AmgInput xg_amg_input(xg_ctx* c);
+// The V-cycle z of an iteration of flexible CG, from the caller's b and x:
+// out the (z_i, p_i) pairs that its SpMV gathers, p (null in the first
+// iteration: zeros) the last search direction, and partials of (z, q),
+// *npart of them (at most 1024), in `part`.  Nothing runs when *done
+// (device) is set.
+int xg_amg_apply_fcg(xg_ctx* c, const double* p, const double* q, double* zp, double* part,
+                     const int* done, int* npart);
 void xg_amg_free(xg_ctx* c);

@@ -18,15 +18,15 @@
 // in pinned host memory, where the host looks once per batch of iterations.
 // Results are deterministic.
 //
-// SpMV of the recurrences (CG and flexible CG): tiles of consecutive rows (at
-// most 2048 nonzeros in FP64, 4096 in FP32); a workgroup forms a tile's
-// products with coalesced loads of the values and column indices into LDS,
-// (z, p) gathered as one pair, then one thread per row sums them in CSR
-// order.  The setup's residual keeps 8 lanes per CSR row (rows hold ~15
-// entries on tet meshes), lane partials combined by a fixed butterfly.
+// SpMV of the recurrences (CG and flexible CG): row tiles with a column list
+// each (xg_tiles.hpp), a row's products summed by one thread in CSR order
+// (the order of ConjugateGradients' CSR::mult).  The setup's residual keeps
+// 8 lanes per CSR row (rows hold ~15 entries on tet meshes), lane partials
+// combined by a fixed butterfly.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -36,6 +36,7 @@
 #include "xg_amg.hpp"
 #include "xg_cg.hpp"
 #include "xg_gnn.hpp"
+#include "xg_tiles_dev.hpp"
 
 using namespace xgd;
 
@@ -44,18 +45,7 @@ namespace {
 constexpr int kCgThreads = 256;
 constexpr int kLanesPerRow = 8;
 constexpr int kMaxParts = 2048;
-// row tiles of the CG SpMV: consecutive rows holding at most tile_nnz<T>
-// nonzeros (a longer row is a tile of its own) and at most kCgThreads rows;
-// 16 KiB of LDS products per tile in FP64 and in FP32
-template <class T>
-constexpr int tile_nnz() { return sizeof(T) == 4 ? 4096 : 2048; }
-
-// workgroups of a SpMV launch: four per CU, so that a launch of more than
-// 1024 tiles walks them evenly with the next tile's loads in flight (per
-// iteration of Jacobi-PCG with one workgroup per tile, at most 2048: 29.8 us
-// at 64^3 and 68 us at 100^3; 1280: 29.5 and 71; 1024: 27.8 and 65.3; 768:
-// 27.8 and 65.8; 512: 29.1 and 71.6)
-constexpr int kSpmvGrid = 1024;
+static_assert(kCgThreads == kTileThreads, "the recurrence kernels walk tiles");
 constexpr int kVecParts = 512;    // workgroups of the vector kernels (max)
 constexpr int kBufLen = 2 * kVecParts + 8;   // rz[.], rr[.], finished flag
 
@@ -75,16 +65,18 @@ struct CgSolver {
   std::vector<int32_t> ja;
   std::vector<double> a0;
   std::vector<double> abc;       // host copy of the values on the device
-  int64_t vals_version = 0;      // changes whenever the device values do
+  // changes whenever the device values do, and differs between solvers
+  int64_t vals_version = 0;
   bool dev_bc = false;           // device values carry Dirichlet rows
   bool restore = false;          // restore the original values before reuse
   std::vector<int64_t> bc_key;   // Dirichlet (node, mask...) set of the device values
   std::vector<DevArr> allocs;
   int *dia = nullptr, *dja = nullptr;
-  int ntile = 0, ntile32 = 0;
-  int4* dtile = nullptr;         // FP64 SpMV tiles: first row, row end, first
-                                 // nonzero, nonzeros
-  int4* dtile32 = nullptr;       // the same for the FP32 products
+  int ntile = 0;                 // SpMV tiles
+  xg::Tile* dtile = nullptr;
+  int* ducol = nullptr;
+  uint16_t* dlidx = nullptr;
+  xg::TileMat tiles() const { return xg::TileMat{ntile, dtile, dia, dja, ducol, dlidx}; }
   double* da = nullptr;          // values as used by the solve
   float* da32 = nullptr;         // FP32 copy for the mixed-precision inner solve
   double *x = nullptr, *b = nullptr, *r = nullptr, *z = nullptr, *d = nullptr;
@@ -277,104 +269,50 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_setup_final(
   }
 }
 
-// q = A p with p = z + bt p_old for the rows of this workgroup's tiles
-// (ti = blockIdx.x, + gridDim.x, ...): a tile's products a_k (z_c + bt p_c)
-// are formed with coalesced loads of a and ja into LDS, (z_c, p_c) read as
-// one pair, then each row is summed by one thread in CSR order (the order of
-// ConjugateGradients' CSR::mult); row(r, p_r, q_r) is called once per row,
-// by that thread (thread 0 for a row longer than a tile).  Every thread of
-// the workgroup calls this (it holds barriers).
-//
-// Up to some 600,000 rows a launch has one tile per workgroup and its time
-// is a chain of dependent loads, not bytes: so the tile's record comes in
-// one load, a thread's whole share of the tile is in flight before anything
-// is waited for, and coef() -- the scalars, themselves sums over the last
-// kernel's partials -- runs while it is; on larger systems the next tile's
-// share is loaded while the current one's rows are summed.
-template <class T, class Coef, class Row>
-__device__ inline bool tiles_spmv(int ntile, const int4* __restrict__ tile,
-                                  const int* __restrict__ ia, const int* __restrict__ ja,
-                                  const T* __restrict__ a, const T* __restrict__ zp,
-                                  T* prod, double* sm, Coef coef, Row row) {
-  constexpr int kTileNnz = tile_nnz<T>();
-  constexpr int kShare = kTileNnz / kCgThreads;   // products of a thread
-  constexpr int kGather = 4;                      // gathers in flight
-  const Pair<T>* zpp = reinterpret_cast<const Pair<T>*>(zp);
-  const int t = threadIdx.x;
-  unsigned cc[kShare];
-  T av[kShare];
-  int4 W = make_int4(0, 0, 0, 0);
-  int e0 = 0, e1 = 0;
-  // loads past the end of the tile are of its last entry: no branch between
-  // the loads
-  auto fetch = [&](int ti) {
-    if (ti >= ntile) return;
-    W = tile[ti];
-    if (W.w > kTileNnz) return;
-    const unsigned last = (unsigned)max(W.w, 1) - 1;
-    const int* jt = ja + W.z;
-    const T* at = a + W.z;
-#pragma unroll
-    for (int u = 0; u < kShare; ++u) {
-      const unsigned kk = min((unsigned)(t + u * kCgThreads), last);
-      cc[u] = (unsigned)jt[kk];
-      av[u] = at[kk];
-    }
-    const unsigned r = min((unsigned)t, (unsigned)(W.y - W.x - 1));
-    const int* it = ia + W.x;
-    e0 = it[r] - W.z;
-    e1 = it[r + 1] - W.z;
-  };
-  fetch(blockIdx.x);
+// source of the recurrences' SpMV: p_c = z_c + bt p_c from the (z, p) pairs,
+// one load each
+template <class T>
+struct PairSource {
+  using Raw = Pair<T>;
+  const Pair<T>* zp;
   T bt;
-  if (!coef(bt)) return false;
-  for (int ti = blockIdx.x; ti < ntile; ti += gridDim.x) {
-    const int r0 = W.x, r1 = W.y, k0 = W.z, nz = W.w;
-    if (nz <= kTileNnz) {
-#pragma unroll
-      for (int u0 = 0; u0 < kShare; u0 += kGather) {
-        Pair<T> v[kGather];
-#pragma unroll
-        for (int u = 0; u < kGather; ++u) v[u] = zpp[cc[u0 + u]];
-#pragma unroll
-        for (int u = 0; u < kGather; ++u)
-          prod[t + (u0 + u) * kCgThreads] = av[u0 + u] * (v[u].z + bt * v[u].p);
-      }
-      const int f0 = e0, f1 = e1, r = r0 + t;
-      Pair<T> own = {};
-      if (r < r1) own = zpp[r];
-      fetch(ti + gridDim.x);
-      __syncthreads();
-      if (r < r1) {
-        T acc = T(0);
-        for (int k = f0; k < f1; k += 8) {
-          T v[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) v[u] = prod[min(k + u, kTileNnz - 1)];
-#pragma unroll
-          for (int u = 0; u < 8; ++u)
-            if (k + u < f1) acc += v[u];
-        }
-        row(r, own.z + bt * own.p, acc);
-      }
-      __syncthreads();        // prod is the next tile's
-    } else {
-      // one row longer than a tile: strided partial sums, fixed-order tree
-      T acc = T(0);
-      for (int k = t; k < nz; k += kCgThreads) {
-        const Pair<T> v = zpp[ja[k0 + k]];
-        acc += a[k0 + k] * (v.z + bt * v.p);
-      }
-      const double sum = block_sum_all((double)acc, sm);
-      if (t == 0) {
-        const Pair<T> v = zpp[r0];
-        row(r0, v.z + bt * v.p, (T)sum);
-      }
-      fetch(ti + gridDim.x);
-    }
+  __device__ Raw load(unsigned c) const { return zp[c]; }
+  __device__ T value(const Raw& v) const { return v.z + bt * v.p; }
+};
+
+// row r of q = A p: stores p_r, q_r, adds to the thread's (p, q)
+template <class T>
+struct CgRow {
+  using Raw = Pair<T>;
+  const PairSource<T>& src;
+  T *pnew, *q;
+  double spq;
+  __device__ Raw load(int r) const { return src.load((unsigned)r); }
+  __device__ void apply(int r, const Raw& own, T qr) {
+    const T pr = src.value(own);
+    pnew[r] = pr;
+    q[r] = qr;
+    spq += (double)pr * (double)qr;
   }
-  return true;
-}
+};
+
+// the same for the flexible recurrence, which also takes (p, r) (r and a
+// third column are not loaded ahead: their registers would spill)
+struct FcgRow {
+  using Raw = Pair<double>;
+  const PairSource<double>& src;
+  const double* r;
+  double *pnew, *q;
+  double spq, spr;
+  __device__ Raw load(int i) const { return src.load((unsigned)i); }
+  __device__ void apply(int i, const Raw& own, double qr) {
+    const double pr = src.value(own), ri = r[i];
+    pnew[i] = pr;
+    q[i] = qr;
+    spq += pr * qr;
+    spr += pr * ri;
+  }
+};
 
 // iteration j, first half: p_j = z + beta p_{j-1} (both read from the (z, p)
 // pairs the previous update wrote), q = A p_j, partials of
@@ -387,41 +325,35 @@ __device__ inline bool tiles_spmv(int ntile, const int4* __restrict__ tile,
 // copy rate, 27.8 us measured (37 before the loads were put ahead of the
 // scalars); 65 us at 100^3, 81 before.
 template <class T>
-__global__ __launch_bounds__(kCgThreads) void k_cg_spmv(
-    int j, int ntile, const int4* __restrict__ tile, const int* __restrict__ ia,
-    const int* __restrict__ ja, const T* __restrict__ a, const T* __restrict__ zp,
+__global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_cg_spmv(
+    int j, xg::TileMat M, const T* __restrict__ a, const T* __restrict__ zp,
     T* __restrict__ pnew, T* __restrict__ q,
     const double* __restrict__ rzb, int nvp, double* __restrict__ pq, CgState* st,
     CgState* pub, long long maxit, double tol_nb) {
-  constexpr int kTileNnz = tile_nnz<T>();
-  __shared__ double sm[3][kCgThreads / 64];
-  __shared__ T prod[kTileNnz];
+  __shared__ TileLds<T> lds;
   const int done = st->done;
-  double spq = 0.0;
-  const bool ran = tiles_spmv<T>(
-      ntile, tile, ia, ja, a, zp, prod, sm[0],
-      [&](T& bt) {
+  PairSource<T> src{reinterpret_cast<const Pair<T>*>(zp), T(0)};
+  CgRow<T> row{src, pnew, q, 0.0};
+  const bool ran = tiles_spmv<T, false, 3>(
+      M, a, src, row,
+      [&]() {
         const double* cur = rzb + ((j - 1) & 1) * kBufLen;
         const double* old = rzb + (j & 1) * kBufLen;
         const bool finished = cur[2 * kVecParts] != 0.0;
         double v[3] = {part_of(cur, nvp), part_of(cur + kVecParts, nvp),
                        j >= 2 ? part_of(old, nvp) : 0.0};
         if (done) return false;
-        block_sums_all<3>(v, sm);
+        block_sums_all<3>(v, lds.sm);
         const double normr = sqrt(v[1]);
         if (j >= 2 && (finished || normr < tol_nb || (long long)(j - 1) >= maxit)) {
           record_stop(st, pub, j, v[1], normr, tol_nb);
           return false;
         }
-        bt = j >= 2 ? (T)(v[0] / v[2]) : T(0);   // the reference's m_alpha = rho/rho0 (:590)
+        src.bt = j >= 2 ? (T)(v[0] / v[2]) : T(0);   // the reference's m_alpha (:590)
         return true;
       },
-      [&](int r, T pr, T qr) {
-        pnew[r] = pr;
-        q[r] = qr;
-        spq += (double)pr * (double)qr;
-      });
-  if (ran) put_part(pq, blockIdx.x, spq, sm[0]);
+      lds);
+  if (ran) put_part(pq, blockIdx.x, row.spq, lds.sm[0]);
 }
 
 // V consecutive values of a vector, 16 bytes: one load or store
@@ -495,9 +427,15 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_update(
     rr += (double)ri * (double)ri;
   }
   double* out = rzb + (j & 1) * kBufLen;
-  put_part(out, blockIdx.x, rz, sm[0]);
-  put_part(out + kVecParts, blockIdx.x, rr, sm[1]);
-  if (blockIdx.x == 0 && threadIdx.x == 0) out[2 * kVecParts] = finished ? 1.0 : 0.0;
+  __syncthreads();            // sm free from its first use
+  v[0] = rz;
+  v[1] = rr;
+  block_sums_all<2>(v, sm);
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = v[0];
+    out[kVecParts + blockIdx.x] = v[1];
+    if (blockIdx.x == 0) out[2 * kVecParts] = finished ? 1.0 : 0.0;
+  }
 }
 
 // ---- mixed precision helpers ----
@@ -597,6 +535,35 @@ __global__ __launch_bounds__(kCgThreads) void k_sum_to_state(
   if (threadIdx.x == 0) st->rr = v;
 }
 
+// The start of iteration k of flexible CG with the multigrid preconditioner:
+// the stop test after iteration k - 1 (not for k = 0), from its (r,r)
+// partials, which every workgroup sums alike; then the V-cycle's right-hand
+// side b = S r and its first sweep x = w D^-1 b.
+__global__ __launch_bounds__(kCgThreads) void k_fcg_in(
+    int k, const double* __restrict__ part, int npart, long long maxit, double target,
+    CgState* st, CgState* pub, const double* __restrict__ r, AmgInput in) {
+  __shared__ double sm[1][kCgThreads / 64];
+  const int done = st->done;
+  const int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
+  const bool mine = i < in.n;
+  const float b = mine ? in.sign[i] * (float)r[i] : 0.f;
+  const float wd = mine ? in.w * in.dinv[i] : 0.f;
+  if (k > 0) {
+    double v[1] = {part_of(part, npart)};
+    if (done) return;
+    block_sums_all<1>(v, sm);
+    const double nr = sqrt(v[0]);
+    if (nr < target || k >= maxit) {
+      record_stop(st, pub, k + 1, v[0], nr, target);
+      return;
+    }
+  }
+  if (mine) {
+    in.b[i] = b;
+    in.x[i] = wd * b;
+  }
+}
+
 __global__ void k_f32_from_f64(int64_t n, const double* __restrict__ s,
                                float* __restrict__ d) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -643,53 +610,80 @@ __global__ __launch_bounds__(kCgThreads) void k_fcg_pack_dot(
 // the buffer of iteration k.  first != 0: beta = 0.  `cur` holds the
 // (z_k, q_{k-1}) partials, `prev` the (p,q) partials of iteration k-1 (the
 // buffers alternate by iteration parity, so nothing read is overwritten).
-__global__ __launch_bounds__(kCgThreads) void k_fcg_spmv(
-    int first, int ntile, const int4* __restrict__ tile, const int* __restrict__ ia,
-    const int* __restrict__ ja, const double* __restrict__ a, const double* __restrict__ zp,
+// Nothing runs once st (null: not asked) says that the solve is done.
+__global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_fcg_spmv(
+    int first, xg::TileMat M, const double* __restrict__ a, const double* __restrict__ zp,
     double* __restrict__ pnew, double* __restrict__ q, const double* __restrict__ r,
-    const double* __restrict__ prev, double* __restrict__ cur, int nvp, int nsp) {
-  __shared__ double sm[2][kCgThreads / 64];
-  __shared__ double prod[tile_nnz<double>()];
-  double spq = 0.0, spr = 0.0;
-  tiles_spmv<double>(
-      ntile, tile, ia, ja, a, zp, prod, sm[0],
-      [&](double& beta) {
+    const double* __restrict__ prev, double* __restrict__ cur, int nvp, int nsp,
+    const CgState* st) {
+  __shared__ TileLds<double> lds;
+  PairSource<double> src{reinterpret_cast<const Pair<double>*>(zp), 0.0};
+  FcgRow row{src, r, pnew, q, 0.0, 0.0};
+  const int done = st ? st->done : 0;
+  const bool ran = tiles_spmv<double, false, 2>(
+      M, a, src, row,
+      [&]() {
         double v[2] = {0.0, 0.0};                 // (z, q_prev), (p, q)_prev
         if (!first) {
           v[0] = part_of(cur, nvp);
           v[1] = part_of(prev + kMaxParts, nsp);
         }
-        block_sums_all<2>(v, sm);
-        beta = v[1] != 0.0 ? -v[0] / v[1] : 0.0;
+        if (done) return false;
+        block_sums_all<2>(v, lds.sm);
+        src.bt = v[1] != 0.0 ? -v[0] / v[1] : 0.0;
         return true;
       },
-      [&](int row, double pr, double qr) {
-        pnew[row] = pr;
-        q[row] = qr;
-        spq += pr * qr;
-        spr += pr * r[row];
-      });
-  put_part(cur + kMaxParts, blockIdx.x, spq, sm[0]);
-  put_part(cur + 2 * kMaxParts, blockIdx.x, spr, sm[1]);
+      lds);
+  if (!ran) return;
+  put_part(cur + kMaxParts, blockIdx.x, row.spq, lds.sm[0]);
+  put_part(cur + 2 * kMaxParts, blockIdx.x, row.spr, lds.sm[1]);
 }
 
-// alpha = (p,r)/(p,q); x += alpha p; r -= alpha q; partials of (r,r)
+// alpha = (p,r)/(p,q); x += alpha p; r -= alpha q; partials of (r,r).  Loads
+// as in k_cg_update.
 __global__ __launch_bounds__(kCgThreads) void k_fcg_update(
     int64_t n, const double* __restrict__ p, const double* __restrict__ q,
-    double* __restrict__ r, double* __restrict__ x, double* __restrict__ fb, int nsp) {
-  __shared__ double sm[kCgThreads / 64];
-  const double PQ = sum_parts(fb + kMaxParts, nsp, sm);
-  const double PR = sum_parts(fb + 2 * kMaxParts, nsp, sm);
-  const double alpha = PQ != 0.0 ? PR / PQ : 0.0;
+    double* __restrict__ r, double* __restrict__ x, double* __restrict__ fb, int nsp,
+    const CgState* st) {
+  constexpr int V = Vec<double>::V;
+  __shared__ double sm[2][kCgThreads / 64];
+  const int done = st ? st->done : 0;
+  const int64_t nv = n / V, step = (int64_t)gridDim.x * kCgThreads;
+  int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
+  Vec<double> rv, qv, pv, xv;
+  auto load = [&](int64_t k) {
+    rv = reinterpret_cast<const Vec<double>*>(r)[k];
+    qv = reinterpret_cast<const Vec<double>*>(q)[k];
+    pv = reinterpret_cast<const Vec<double>*>(p)[k];
+    xv = reinterpret_cast<const Vec<double>*>(x)[k];
+  };
+  if (i < nv) load(i);
+  double v[2] = {part_of(fb + kMaxParts, nsp), part_of(fb + 2 * kMaxParts, nsp)};
+  if (done) return;
+  block_sums_all<2>(v, sm);
+  const double alpha = v[0] != 0.0 ? v[1] / v[0] : 0.0;
   double rr = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kCgThreads) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
+  while (i < nv) {
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      xv.v[k] += alpha * pv.v[k];
+      rv.v[k] -= alpha * qv.v[k];
+      rr += rv.v[k] * rv.v[k];
+    }
+    reinterpret_cast<Vec<double>*>(r)[i] = rv;
+    reinterpret_cast<Vec<double>*>(x)[i] = xv;
+    i += step;
+    if (i < nv) load(i);
+  }
+  // the last n mod V rows
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x < n - nv * V) {
+    const int64_t k = nv * V + threadIdx.x;
+    x[k] += alpha * p[k];
+    const double ri = r[k] - alpha * q[k];
+    r[k] = ri;
     rr += ri * ri;
   }
-  put_part(fb + 3 * kMaxParts, blockIdx.x, rr, sm);
+  put_part(fb + 3 * kMaxParts, blockIdx.x, rr, sm[0]);
 }
 
 // z = r / d (Jacobi preconditioner of the flexible solve)
@@ -804,9 +798,7 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
            int64_t maxit, double tol_nb, double brk, int64_t jstart = 1) {
   CgSolver* s = c->cg;
   const bool f32 = sizeof(T) == 4;
-  const int ntile = f32 ? s->ntile32 : s->ntile;
-  const int4* dtile = f32 ? s->dtile32 : s->dtile;
-  const int gr = std::max(1, std::min(ntile, kSpmvGrid)), gv = grid_vec(s->nrow);
+  const int gr = std::max(1, std::min(s->ntile, kSpmvGrid)), gv = grid_vec(s->nrow);
   const int batch = 8;
   // the (z, p) pairs of the first SpMV; each update writes the next ones
   T* zp = f32 ? reinterpret_cast<T*>(s->zp32) : reinterpret_cast<T*>(s->zp);
@@ -819,8 +811,8 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
       const int j = (int)(j0 + i);
       T* pnew = j & 1 ? p1 : p0;
       hipLaunchKernelGGL(k_cg_spmv<T>, dim3(gr), dim3(kCgThreads), 0, c->stream, j,
-                         ntile, dtile, s->dia, s->dja, a, zp, pnew, q, s->rzb, gv, s->pq,
-                         s->st, s->hpub, (long long)maxit, tol_nb);
+                         s->tiles(), a, zp, pnew, q, s->rzb, gv, s->pq, s->st, s->hpub,
+                         (long long)maxit, tol_nb);
       hipLaunchKernelGGL(k_cg_update<T>, dim3(gv), dim3(kCgThreads), 0, c->stream, j,
                          s->nrow, q, d, pnew, r, x, zp, s->rzb, gv, s->pq, gr, s->st, brk);
     }
@@ -847,6 +839,54 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
   s->hst->rr = s->hpub->rr;
   s->hst->converged = s->hpub->converged;
   s->hst->done = 1;
+  return XG_OK;
+}
+
+// Flexible CG with the multigrid preconditioner from the state of xg_cg_setup
+// (not converged) until ||r|| < target or maxit iterations.  The stop test
+// of iteration k runs at the start of iteration k + 1, whose kernels are then
+// no-ops; as in run_cg the host enqueues that iteration before it waits for
+// the last one, and the stream is drained before this returns.
+int run_fcg_amg(xg_ctx* c, int64_t maxit, double target) {
+  CgSolver* s = c->cg;
+  const int64_t n = s->nrow;
+  const int gv = grid_vec(n), gt = std::max(1, std::min(s->ntile, kSpmvGrid));
+  double* P[2] = {s->p0, s->p1};
+  double* Q[2] = {s->q, s->q2};
+  const AmgInput in = xg_amg_input(c);
+  s->hpub->done = 0;
+  hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(64), 0, c->stream, s->st);
+  auto enqueue = [&](int64_t k) -> int {
+    double* Bk = s->fb + (k & 1) * 4 * kMaxParts;
+    double* Bp = s->fb + ((k + 1) & 1) * 4 * kMaxParts;
+    hipLaunchKernelGGL(k_fcg_in, dim3(nblocks(n)), dim3(kCgThreads), 0, c->stream, (int)k,
+                       Bp + 3 * kMaxParts, gv, (long long)maxit, target, s->st, s->hpub, s->r,
+                       in);
+    int nzq = 0, rc;
+    if ((rc = xg_amg_apply_fcg(c, k > 0 ? P[(k + 1) & 1] : nullptr, Q[(k + 1) & 1],
+                               s->zp, Bk, &s->st->done, &nzq)))
+      return rc;
+    hipLaunchKernelGGL(k_fcg_spmv, dim3(gt), dim3(kCgThreads), 0, c->stream, k == 0 ? 1 : 0,
+                       s->tiles(), s->da, s->zp, P[k & 1], Q[k & 1], s->r, Bp, Bk, nzq, gt,
+                       s->st);
+    hipLaunchKernelGGL(k_fcg_update, dim3(gv), dim3(kCgThreads), 0, c->stream, n, P[k & 1],
+                       Q[k & 1], s->r, s->x, Bk, gt, s->st);
+    XG_HIP(c, hipGetLastError());
+    XG_HIP(c, hipEventRecord(s->ev[k & 1], c->stream));
+    return XG_OK;
+  };
+  int rc = enqueue(0);
+  if (rc) return rc;
+  for (int64_t k = 0;; ++k) {
+    // iteration maxit only holds the stop test
+    if (k < maxit && (rc = enqueue(k + 1))) return rc;
+    XG_HIP(c, hipEventSynchronize(s->ev[k & 1]));
+    if (static_cast<volatile CgState*>(s->hpub)->done) break;
+    if (k > maxit) return fail(c, XG_EHIP, "flexible CG: stop test not reached on the device");
+  }
+  XG_HIP(c, hipStreamSynchronize(c->stream));
+  s->hst->it = s->hpub->it;
+  s->hst->rr = s->hpub->rr;
   return XG_OK;
 }
 
@@ -971,7 +1011,9 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
   const int64_t nnz = (int64_t)ia[nrow] - base;
   if (nnz <= 0 || nnz >= (1ll << 31)) return fail(c, XG_EINVAL, "xg_cg_matrix: bad nnz");
   XG_HIP(c, hipSetDevice(c->device));
+  static std::atomic<int64_t> serial{0};
   auto* s = new CgSolver;
+  s->vals_version = ++serial << 32;
   s->ncomp = ncomp;
   s->nrow = nrow;
   s->nnz = nnz;
@@ -989,32 +1031,17 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
   s->a0.assign(a, a + nnz);
   s->abc = s->a0;
   std::vector<int32_t> ia32(s->ia.begin(), s->ia.end());
-  // SpMV tiles: consecutive rows, at most kCgThreads rows and tnz nonzeros
-  // each (a longer row alone)
-  auto tiles = [&](int64_t tnz) {
-    std::vector<int4> tile;
-    for (int64_t r = 0; r < nrow;) {
-      int64_t r1 = r, nz = 0;
-      while (r1 < nrow && r1 - r < kCgThreads && nz + (s->ia[r1 + 1] - s->ia[r1]) <= tnz) {
-        nz += s->ia[r1 + 1] - s->ia[r1];
-        ++r1;
-      }
-      if (r1 == r) r1 = r + 1;
-      tile.push_back(make_int4((int)r, (int)r1, (int)s->ia[r], (int)(s->ia[r1] - s->ia[r])));
-      r = r1;
-    }
-    return tile;
-  };
-  const std::vector<int4> tile = tiles(tile_nnz<double>()), tile32 = tiles(tile_nnz<float>());
-  s->ntile = (int)tile.size();
-  s->ntile32 = (int)tile32.size();
+  xg::TileSet ts;
+  xg::build_tiles(nrow, nrow, s->ia.data(), s->ja.data(), ts);
+  s->ntile = (int)ts.tile.size();
   std::vector<float> a32(nnz);
   for (int64_t j = 0; j < nnz; ++j) a32[j] = (float)a[j];
   int rc;
   auto& L = s->allocs;
   const size_t n = (size_t)nrow;
   if ((rc = upload(c, L, &s->dia, ia32)) || (rc = upload(c, L, &s->dja, s->ja)) ||
-      (rc = upload(c, L, &s->dtile, tile)) || (rc = upload(c, L, &s->dtile32, tile32)) ||
+      (rc = upload(c, L, &s->dtile, ts.tile)) || (rc = upload(c, L, &s->ducol, ts.ucol)) ||
+      (rc = upload(c, L, &s->dlidx, ts.lidx)) ||
       (rc = upload(c, L, &s->da, s->a0)) || (rc = upload(c, L, &s->da32, a32)) ||
       (rc = dev_alloc(c, L, (void**)&s->x, n * 8)) ||
       (rc = dev_alloc(c, L, (void**)&s->b, n * 8)) ||
@@ -1405,7 +1432,7 @@ int xg_cg_solve_flexible(xg_ctx* c, int pc_kind, int64_t inner, int64_t maxit,
     if (s->ncomp != 1)
       return fail(c, XG_EUNSUPPORTED, "AMG preconditioner: one component per node only");
     if ((rc = xg_amg_prepare_internal(c, n, s->ia.data(), s->ja.data(), s->abc.data(),
-                                      s->vals_version)))
+                                      s->vals_version, s->tiles())))
       return rc;
   }
   if ((rc = read_state(c))) return rc;
@@ -1422,16 +1449,18 @@ int xg_cg_solve_flexible(xg_ctx* c, int pc_kind, int64_t inner, int64_t maxit,
   double best = nr;
   int64_t kbest = 0;
   bool learned = pc_kind == 2;
-  for (; k < maxit && !(nr < target); ++k) {
+  if (pc_kind == 3 && !(nr < target)) {
+    if ((rc = run_fcg_amg(c, maxit, target))) return rc;
+    nr = sqrt(s->hst->rr);
+    k = tin = s->hst->it;
+  }
+  for (; pc_kind != 3 && k < maxit && !(nr < target); ++k) {
     double* Bk = s->fb + (k & 1) * 4 * kMaxParts;
     double* Bp = s->fb + ((k + 1) & 1) * 4 * kMaxParts;
     if (pc_kind == 0 || (pc_kind == 2 && !learned)) {
       if (pc_kind == 2) ++tin;
       hipLaunchKernelGGL(k_jacobi_apply, dim3(gv), dim3(kCgThreads), 0, c->stream, n,
                          s->r, s->d, s->z);
-    } else if (pc_kind == 3) {
-      if ((rc = xg_amg_apply_internal(c, s->r, s->z))) return rc;
-      ++tin;
     } else if (pc_kind == 2) {
       if ((rc = xg_gnn_apply_internal(c, s->dia, s->dja, s->r, s->d, s->z))) return rc;
       int used = 0;
@@ -1452,10 +1481,10 @@ int xg_cg_solve_flexible(xg_ctx* c, int pc_kind, int64_t inner, int64_t maxit,
                        k > 0 ? 1 : 0,
                        s->z, Q[(k + 1) & 1], P[(k + 1) & 1], s->zp, Bk);
     hipLaunchKernelGGL(k_fcg_spmv, dim3(gt), dim3(kCgThreads), 0, c->stream, k == 0 ? 1 : 0,
-                       s->ntile, s->dtile, s->dia, s->dja, s->da, s->zp, P[k & 1], Q[k & 1],
-                       s->r, Bp, Bk, gv, gt);
+                       s->tiles(), s->da, s->zp, P[k & 1], Q[k & 1], s->r, Bp, Bk, gv, gt,
+                       nullptr);
     hipLaunchKernelGGL(k_fcg_update, dim3(gv), dim3(kCgThreads), 0, c->stream, n,
-                       P[k & 1], Q[k & 1], s->r, s->x, Bk, gt);
+                       P[k & 1], Q[k & 1], s->r, s->x, Bk, gt, nullptr);
     hipLaunchKernelGGL(k_sum_to_state, dim3(1), dim3(kCgThreads), 0, c->stream,
                        Bk + 3 * kMaxParts, gv, s->st);
     XG_HIP(c, hipGetLastError());

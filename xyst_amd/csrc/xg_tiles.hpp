@@ -1,0 +1,49 @@
+// Row tiles of a CSR matrix for SpMV on the device (xg_cg.hip, xg_amg.hip).
+//
+// A tile is a run of consecutive rows with at most kTileNnz nonzeros and
+// kTileRows rows (a longer row is a tile of its own, without a column list).
+// Neighbouring rows share most of their columns: the matrix of a tet mesh
+// has some 560 different ones among a tile's 2048 nonzeros.  So a tile lists
+// its columns once, ascending, and its nonzeros hold 16-bit positions in
+// that list: a workgroup reads every source value once, with neighbouring
+// lanes on neighbouring addresses, into LDS, where the nonzeros find it, and
+// a nonzero costs 2 bytes of index instead of 4 (with the lists, 3.1).
+#pragma once
+#include <cstdint>
+#include <vector>
+
+namespace xg {
+
+constexpr int kTileNnz = 2048;
+constexpr int kTileRows = 128;   // two threads of a workgroup per row
+
+struct alignas(32) Tile {
+  int row0, row1;   // rows
+  int k0, nz;       // first nonzero, nonzeros
+  int u0, nu;       // column list
+  int pad0, pad1;
+};
+
+// on the device, with the matrix' row offsets
+struct TileMat {
+  int ntile = 0;
+  const Tile* tile = nullptr;
+  const int* ia = nullptr;
+  const int* ja = nullptr;   // columns (only of rows longer than a tile)
+  const int* ucol = nullptr;
+  const uint16_t* lidx = nullptr;
+};
+
+struct TileSet {
+  bool has_long = false;        // a row is longer than a tile
+  std::vector<Tile> tile;
+  std::vector<int32_t> ucol;    // the tiles' columns
+  std::vector<uint16_t> lidx;   // per nonzero: position in its tile's list
+};
+
+// Tiles of the matrix with row offsets ia (nrow + 1, from 0) and columns ja
+// below ncol.  Threads work on runs of tiles; the result does not depend on
+// their number.
+void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t);
+
+}  // namespace xg
