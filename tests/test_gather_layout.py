@@ -1,0 +1,49 @@
+"""CPU check of the small meshes' block layouts
+(tests/cpp/gather_layout_check.cpp)."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from xyst_amd import riemann as X
+from xyst_amd.meshgen import box_mesh, renumber_mesh
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("gather") / "gather_layout_check")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", out,
+                    os.path.join(ROOT, "tests", "cpp", "gather_layout_check.cpp"),
+                    os.path.join(ROOT, "xyst_amd", "csrc", "xg_layout.cpp")], check=True)
+    return out
+
+
+@pytest.mark.parametrize("n,order", [(1, "lex"), (2, "lex"), (9, "lex"), (9, "random"),
+                                     (14, "rcm+block")])
+def test_small_blocks_reach_every_node_once(exe, tmp_path, n, order):
+    m = box_mesh(n, seed=n)
+    N = m["coord"].shape[1]
+    if order == "random":
+        m = renumber_mesh(m, np.random.default_rng(3).permutation(N))
+    elif order == "rcm+block":
+        m = renumber_mesh(m, X.mesh_rcm(N, m["inpoel"]))
+        m = renumber_mesh(m, X.mesh_block_order(m["coord"], 1024))
+    e, _ = X.mesh_domint(m["coord"], m["inpoel"])
+    e = e.astype(np.int32)
+    flip = np.random.default_rng(n).random(len(e)) < 0.5     # both orientations
+    e[flip] = e[flip][:, ::-1]
+    f = tmp_path / "mesh.bin"
+    with open(f, "wb") as fh:
+        np.array([N, len(e), len(m["triinpoel"]), len(m["inpoel"])], np.int64).tofile(fh)
+        for a in (e[:, 0], e[:, 1], m["triinpoel"], m["inpoel"]):
+            np.ascontiguousarray(a, np.int32).tofile(fh)
+    for kind in ("rhs", "grad", "cho", "tet"):
+        for nodes in (1, 16, 31, 77):
+            for gather in ((1,) if kind == "grad" else (0, 1)):
+                r = subprocess.run([exe, str(f), kind, str(nodes), str(gather)],
+                                   capture_output=True, text=True)
+                assert r.returncode == 0 and r.stdout.startswith("ok"), \
+                    (kind, nodes, gather, r.stderr)

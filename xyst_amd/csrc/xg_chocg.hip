@@ -9,7 +9,8 @@
 // the block's nodes are staged in LDS with the NV values the operator reads;
 // per chunk each thread computes one edge's (or one face corner's) NF values
 // into LDS; the thread owning local node t sums the chunk's slots touching it
-// in slot order; halo partials go to slots that k_fixup adds in block order.
+// in slot order; halo partials go to slots that k_fixup adds in block order
+// (none on small meshes, whose blocks are gather blocks: xg::cho_blocks).
 // No atomics: every result is bitwise reproducible.
 //
 // div/grad/vgrad/flux add to their output, as the reference's do (the caller
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(kT) void k_cho_blocks(ChoArgs a) {
     double* o = a.out + (size_t)(own0 + t) * NF;
 #pragma unroll
     for (int k = 0; k < NF; ++k) o[k] = a.accum ? o[k] + acc[k] : acc[k];
-  } else if (t < nloc) {
+  } else if (t < nloc && B1.x >= 0) {
     double* o = a.S + (size_t)(B1.x + t - nown) * NF;
 #pragma unroll
     for (int k = 0; k < NF; ++k) o[k] = acc[k];
@@ -846,8 +847,9 @@ int xg_chocg_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
   for (int64_t f = 0; f < ntri * 3; ++f) tri32[f] = (int)tri[f];
   std::vector<uint8_t> nosym(ntri * 3 + 1, 0);
   xg::Layout L;
-  int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), nosym.data(),
-                            xg::kBlockNodes, xg::kBlockCap, xg::kChunkSlots, L, c->err);
+  const xg::BlockPlan plan = xg::cho_blocks(npoin);
+  int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), nosym.data(), plan.nodes,
+                            xg::kBlockCap, xg::kChunkSlots, L, c->err, plan.gather, true);
   if (rc) return rc;
   std::vector<double> dwl(L.eidx.size());
   for (size_t e = 0; e < L.eidx.size(); ++e) dwl[e] = w[L.eidx[e]];

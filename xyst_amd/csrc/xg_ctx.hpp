@@ -44,24 +44,20 @@ struct xg_ctx {
   int64_t nedge = 0;
   uint32_t* elpq = nullptr;
   double *dx = nullptr, *dy = nullptr, *dz = nullptr;
-  // grad blocks (a gather layout: no halo partials, no boundary faces)
+  // grad blocks (a gather layout: no halo partials)
   int nblk = 0, nchunk = 0;
   int4 *blk0 = nullptr, *blk1 = nullptr;     // (own0,nown,nloc,halo_off), (slot0,chunk0,chunk1,-)
   int *halo = nullptr;
   int4 *chk = nullptr;                       // (kind,first,count,tend_off)
   int *chk_ent = nullptr;                    // ent_off
   uint16_t *tend = nullptr, *entries = nullptr;
-  // grad boundary faces
-  int nbnode = 0;
-  int *bnode = nullptr, *boff = nullptr, *bface = nullptr;
-  int* tri = nullptr;
+  // grad boundary faces: local ids, normals (3 per face)
+  uint32_t *gfab = nullptr, *gfcs = nullptr;
+  double* gfn = nullptr;
   // RieCG stepping
   bool have_riecg = false;
   int ncomp = 5;                         // components per node (xg_riecg_set_ncomp)
   double* vol = nullptr;
-  // per node: 1 = boundary node, whose gradient k_grad_bnd completes and
-  // divides by vol; the others are divided by k_grad_blocks (RK stages)
-  uint8_t* gflag = nullptr;
   int nsymnode = 0;
   int *symnode = nullptr, *symoff = nullptr;
   double* symnorm = nullptr;

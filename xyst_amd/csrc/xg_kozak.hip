@@ -18,7 +18,9 @@
 //    chunks.
 // Then the thread owning local node t adds (or, for the bounds, takes the
 // max/min of) the chunk's corner values that touch it, in slot order; halo
-// partials go to slots that k_fixup adds to their owners in block order.
+// partials go to slots that k_fixup adds to their owners in block order (on
+// small meshes blocks are small and hold every tet that touches their nodes:
+// no halo partials, xg::tet_blocks).
 // No atomics: every sum has a fixed order and the result is bitwise
 // reproducible.
 #include <hip/hip_runtime.h>
@@ -384,7 +386,7 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
     double* o = R + (size_t)(own0 + t) * NO;
 #pragma unroll
     for (int c = 0; c < NO; ++c) o[c] = acc[c];
-  } else if (t < nloc) {
+  } else if (t < nloc && B1.x >= 0) {
     double* o = S + (size_t)(B1.x + t - nown) * NO;
 #pragma unroll
     for (int c = 0; c < NO; ++c) o[c] = acc[c];
@@ -511,7 +513,7 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
       }
     }
   }
-  if (t < nloc) {
+  if (t < nown || (t < nloc && B1.x >= 0)) {
     double* o = t < nown ? Q + (size_t)(own0 + t) * NB
                          : S + (size_t)(B1.x + t - nown) * NB;
 #pragma unroll
@@ -687,7 +689,7 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
     double* o = A + (size_t)(own0 + t) * NC;
 #pragma unroll
     for (int c = 0; c < NC; ++c) o[c] = acc[c];
-  } else if (t < nloc) {
+  } else if (t < nloc && B1.x >= 0) {
     double* o = S + (size_t)(B1.x + t - nown) * NC;
 #pragma unroll
     for (int c = 0; c < NC; ++c) o[c] = acc[c];
@@ -895,8 +897,9 @@ int xg_kozak_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
     return fail(c, XG_EINVAL, "xg_kozak_upload: bad arguments");
   XG_HIP(c, hipSetDevice(c->device));
   xg::TetLayout L;
-  int rc = xg::build_tet_layout((int)npoin, ntet, inpoel, xg::kKozNodes, xg::kKozCap,
-                                L, c->err, xg::kTetsPerPairChunk);
+  const xg::BlockPlan plan = xg::tet_blocks(npoin);
+  int rc = xg::build_tet_layout((int)npoin, ntet, inpoel, plan.nodes, xg::kKozCap, L, c->err,
+                                xg::kTetsPerPairChunk, plan.gather);
   if (rc) return rc;
   auto* k = new KozakMesh;
   k->npoin = (int)npoin;

@@ -105,7 +105,8 @@ static void full_lists(int npoin, const std::vector<int>& p, const std::vector<i
 int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                  const std::vector<double>& d, int64_t ntri, const int* tri,
                  const uint8_t* besym, int block_nodes, int block_cap,
-                 int chunk_slots, Layout& L, std::string& err, bool gather) {
+                 int chunk_slots, Layout& L, std::string& err, bool gather,
+                 bool gather_faces) {
   const int64_t ne = (int64_t)p.size();
   L = Layout();
   if (chunk_slots < 3 || chunk_slots > kChunkSlots) {
@@ -117,12 +118,22 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
   // lies beyond it), or both ways for a gather layout
   std::vector<int64_t> uoff;
   std::vector<int> up;
-  if (gather)
+  if (gather && gather_faces && ntri) {
+    // the faces' edges too: a block holds the nodes of every face it takes
+    std::vector<int> pf(p), qf(q);
+    for (int64_t f = 0; f < ntri; ++f)
+      for (int a = 0; a < 3; ++a) {
+        pf.push_back(tri[f * 3 + a]);
+        qf.push_back(tri[f * 3 + (a + 1) % 3]);
+      }
+    full_lists(npoin, pf, qf, uoff, up);
+  } else if (gather) {
     full_lists(npoin, p, q, uoff, up);
-  else
+  } else {
     upper_lists(npoin, p, q, uoff, up);
+  }
   // (boundary faces are tet faces: their nodes are edge neighbours of the
-  // face's smallest node, so the edge lists already cover them)
+  // face's smallest node, so the upper lists already cover them)
   std::vector<int> bstart;
   int prc = partition_blocks(npoin, uoff, up, block_nodes, block_cap, bstart, err);
   if (prc) return prc;
@@ -130,17 +141,23 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
   std::vector<int> blk_of(npoin);
   for (int b = 0; b < nblk; ++b)
     for (int i = bstart[b]; i < bstart[b + 1]; ++i) blk_of[i] = b;
-  // work items per block (gather: an edge belongs to the blocks of both its
-  // ends, and there are no boundary faces)
+  // work items per block (gather: an edge or face belongs to the blocks of
+  // all its nodes)
   std::vector<std::vector<int64_t>> bedges(nblk), bfaces(nblk);
   for (int64_t e = 0; e < ne; ++e) {
     const int b0 = blk_of[std::min(p[e], q[e])], b1 = blk_of[std::max(p[e], q[e])];
     bedges[b0].push_back(e);
     if (gather && b1 != b0) bedges[b1].push_back(e);
   }
-  for (int64_t f = 0; f < (gather ? 0 : ntri); ++f) {
-    int m = std::min(tri[f * 3], std::min(tri[f * 3 + 1], tri[f * 3 + 2]));
-    bfaces[blk_of[m]].push_back(f);
+  for (int64_t f = 0; f < (gather && !gather_faces ? 0 : ntri); ++f) {
+    const int* N = tri + f * 3;
+    if (!gather) {
+      bfaces[blk_of[std::min(N[0], std::min(N[1], N[2]))]].push_back(f);
+      continue;
+    }
+    const int b[3] = {blk_of[N[0]], blk_of[N[1]], blk_of[N[2]]};
+    for (int a = 0; a < 3; ++a)
+      if ((a < 1 || b[a] != b[0]) && (a < 2 || b[a] != b[1])) bfaces[b[a]].push_back(f);
   }
   L.blk.resize(nblk);
   std::vector<std::vector<std::pair<int,int>>> fix(npoin);   // node -> (block, slot)
@@ -158,7 +175,8 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     }
     for (int64_t f : bfaces[b])
       for (int a = 0; a < 3; ++a)
-        if (tri[f * 3 + a] >= bstart[b + 1]) halo.push_back(tri[f * 3 + a]);
+        if (tri[f * 3 + a] >= bstart[b + 1] || tri[f * 3 + a] < bstart[b])
+          halo.push_back(tri[f * 3 + a]);
     std::sort(halo.begin(), halo.end());
     halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
     B.nloc = B.nown + (int)halo.size();
@@ -167,7 +185,7 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
       return XG_EUNSUPPORTED;
     }
     B.halo_off = (int)L.halo.size();
-    B.slot0 = nslot;
+    B.slot0 = gather ? -1 : nslot;
     for (size_t h = 0; h < halo.size(); ++h) {
       L.halo.push_back(halo[h]);
       if (!gather) fix[halo[h]].emplace_back(b, nslot + (int)h);
@@ -234,7 +252,8 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
       for (size_t i = i0; i < i1; ++i) {
         int64_t f = F[i];
         for (int a = 0; a < 3; ++a)
-          ent.emplace_back(local[tri[f * 3 + a]], (uint16_t)(3 * (i - i0) + a));
+          if (!gather || local[tri[f * 3 + a]] < B.nown)
+            ent.emplace_back(local[tri[f * 3 + a]], (uint16_t)(3 * (i - i0) + a));
       }
       emit(1, (int64_t)L.fab.size(), (int)(i1 - i0), ent);
       for (size_t i = i0; i < i1; ++i) {
@@ -274,7 +293,7 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
 // chunk tet i, and every local node sums its slots in slot order.
 int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
                      int block_nodes, int block_cap, TetLayout& L,
-                     std::string& err, int tets_per_chunk) {
+                     std::string& err, int tets_per_chunk, bool gather) {
   if (tets_per_chunk < 1 || 4 * tets_per_chunk > 32768) {
     err = "kozak layout: bad chunk size";
     return XG_EINVAL;
@@ -298,7 +317,10 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
   // unique edges suffice for the partition (duplicates only repeat marks)
   std::vector<int64_t> uoff;
   std::vector<int> up;
-  upper_lists(npoin, p, q, uoff, up);
+  if (gather)
+    full_lists(npoin, p, q, uoff, up);
+  else
+    upper_lists(npoin, p, q, uoff, up);
   for (int i = 0; i < npoin; ++i) {
     auto b = up.begin() + uoff[i], e = up.begin() + uoff[i + 1];
     std::sort(b, e);
@@ -327,8 +349,15 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
   std::vector<std::vector<int64_t>> btets(nblk);
   for (int64_t e = 0; e < ntet; ++e) {
     const size_t* N = inpoel + e * 4;
-    size_t m = std::min(std::min(N[0], N[1]), std::min(N[2], N[3]));
-    btets[blk_of[m]].push_back(e);
+    if (!gather) {
+      btets[blk_of[std::min(std::min(N[0], N[1]), std::min(N[2], N[3]))]].push_back(e);
+      continue;
+    }
+    for (int a = 0; a < 4; ++a) {
+      bool first = true;
+      for (int c = 0; c < a; ++c) first = first && blk_of[N[c]] != blk_of[N[a]];
+      if (first) btets[blk_of[N[a]]].push_back(e);
+    }
   }
   L.blk.resize(nblk);
   std::vector<std::vector<std::pair<int,int>>> fix(npoin);
@@ -341,7 +370,8 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
     std::vector<int> halo;
     for (int64_t e : btets[b])
       for (int a = 0; a < 4; ++a)
-        if ((int)inpoel[e * 4 + a] >= bstart[b + 1]) halo.push_back((int)inpoel[e * 4 + a]);
+        if ((int)inpoel[e * 4 + a] >= bstart[b + 1] || (int)inpoel[e * 4 + a] < bstart[b])
+          halo.push_back((int)inpoel[e * 4 + a]);
     std::sort(halo.begin(), halo.end());
     halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
     B.nloc = B.nown + (int)halo.size();
@@ -350,12 +380,12 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
       return XG_EUNSUPPORTED;
     }
     B.halo_off = (int)L.halo.size();
-    B.slot0 = nslot;
+    B.slot0 = gather ? -1 : nslot;
     for (size_t h = 0; h < halo.size(); ++h) {
       L.halo.push_back(halo[h]);
-      fix[halo[h]].emplace_back(b, nslot + (int)h);
+      if (!gather) fix[halo[h]].emplace_back(b, nslot + (int)h);
     }
-    nslot += (int)halo.size();
+    if (!gather) nslot += (int)halo.size();
     for (int i = 0; i < B.nown; ++i) local[B.own0 + i] = i;
     for (size_t h = 0; h < halo.size(); ++h) local[halo[h]] = B.nown + (int)h;
     auto& T = btets[b];
@@ -374,7 +404,8 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
       std::vector<std::pair<int, uint16_t>> ent;
       for (size_t i = i0; i < i1; ++i)
         for (int a = 0; a < 4; ++a)
-          ent.emplace_back(local[inpoel[T[i] * 4 + a]], (uint16_t)(4 * (i - i0) + a));
+          if (!gather || local[inpoel[T[i] * 4 + a]] < B.nown)
+            ent.emplace_back(local[inpoel[T[i] * 4 + a]], (uint16_t)(4 * (i - i0) + a));
       std::stable_sort(ent.begin(), ent.end(),
                        [](const auto& x, const auto& y) { return x.first < y.first; });
       Chunk C;
@@ -400,6 +431,9 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
     for (int i = 0; i < B.nown; ++i) local[B.own0 + i] = -1;
     for (size_t h = 0; h < halo.size(); ++h) local[halo[h]] = -1;
   }
+  // the kernels prefetch 4 entries per tet; a gather chunk holds fewer (see
+  // build_layout)
+  if (gather) L.entries.resize(L.entries.size() + 4 * (size_t)tets_per_chunk, 0);
   L.nslot = nslot;
   L.fx_off.push_back(0);
   for (int n = 0; n < npoin; ++n) {

@@ -32,7 +32,7 @@ constexpr int kRhsNodes = 312;
 struct Block {
   int own0 = 0, nown = 0, nloc = 0;  // owned ids [own0, own0+nown); local ids
   int halo_off = 0;                  // halo node ids at halo[halo_off ...]
-  int slot0 = 0;                     // first halo output slot
+  int slot0 = 0;                     // first halo output slot (-1: none)
   int chunk0 = 0, chunk1 = 0;        // chunks [chunk0, chunk1)
 };
 
@@ -86,22 +86,72 @@ struct TetLayout {
   std::vector<int> fx_node, fx_off, fx_slot;
 };
 
+// gather: a block takes every tet that touches one of its nodes and its
+// entries reach its owned corners only (as for the edge layouts below)
 int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
                      int block_nodes, int block_cap, TetLayout& L,
                      std::string& err,
-                     int tets_per_chunk = kTetsPerPairChunk);
+                     int tets_per_chunk = kTetsPerPairChunk, bool gather = false);
 
 // chunk_slots: flux slots per edge chunk (<= kChunkSlots; boundary-face
 // chunks hold chunk_slots / 3 faces).
 // gather: a block takes every edge that touches one of its nodes (edges
 // between two blocks are in both), its halo is every outside end of those,
 // and its entries add each edge to its owned ends only, so every owned sum
-// is complete in its block: no halo slots, no fix-up lists, and no boundary
-// faces (an operator on such a layout adds boundary terms by itself)
+// is complete in its block: no halo slots (Block::slot0 is -1) and no
+// fix-up lists.  gather_faces: likewise every boundary face that touches one
+// of its nodes; without it a gather layout carries no boundary faces.
 int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                  const std::vector<double>& d, int64_t ntri, const int* tri,
                  const uint8_t* besym, int block_nodes, int block_cap,
-                 int chunk_slots, Layout& L, std::string& err, bool gather = false);
+                 int chunk_slots, Layout& L, std::string& err, bool gather = false,
+                 bool gather_faces = false);
+
+// Blocks of small meshes.  At the full block sizes a mesh of a few thousand
+// nodes fills a few of the 256 CUs, and each block walks its chunks alone: so
+// they are cut into about as many blocks as run at once, and where that is
+// the faster, into gather blocks, which need no halo fix-up.  Times of the
+// full blocks and of these, in us:
+//  riemann::grad (two workgroups per CU: at most 512 blocks): RieCG step of
+//    three gradients on 33^3 (39,304 nodes) 241 -> 183, on 40^3 equal;
+//  riemann::rhs (likewise): 12^3 20.6 -> 6.9, 24^3 21.1 -> 9.9, 29^3 (27,000
+//    nodes) 23.7 -> 14.5, with 6 components (one workgroup per CU) 23.9 ->
+//    20.5; on 31^3 (32,768) 22.4 -> 20.4, but 22.7 -> 27.9 with 6;
+//  the tet operators, KozCG step: 12^3 201 -> 84, 20^3 (9,261) 201 -> 104, as
+//    scatter blocks 117; 24^3 (15,625) 203 -> 140 and 125 as scatter blocks,
+//    36^3 216 -> 178, 39^3 (64,000) 216 -> 197, 42^3 equal;
+//  the chorin operators (one workgroup per CU: at most 256 blocks),
+//    chorin::rhs: 12^3 20.0 -> 6.2, 20^3 20.6 -> 8.3, 28^3 (24,389) 20.7 ->
+//    11.6, as scatter blocks 14.5; 33^3 22.2 -> 23.3.
+constexpr int64_t kSmallGrad = 49152;
+constexpr int64_t kSmallRhs = 28672;
+constexpr int64_t kSmallTetGather = 10240;
+constexpr int64_t kSmallTet = 65536;
+constexpr int64_t kSmallCho = 28672;
+
+struct BlockPlan {
+  int nodes;     // owned nodes per block, at most
+  bool gather;   // a gather layout
+};
+
+inline int small_nodes(int64_t npoin, int64_t nblk) {
+  return (int)(npoin < 16 * nblk ? 16 : (npoin + nblk - 1) / nblk);
+}
+inline BlockPlan grad_blocks(int64_t npoin) {
+  return {npoin <= kSmallGrad ? small_nodes(npoin, 512) : kGradNodes, true};
+}
+inline BlockPlan rhs_blocks(int64_t npoin) {
+  if (npoin <= kSmallRhs) return {small_nodes(npoin, 512), true};
+  return {kRhsNodes, false};
+}
+inline BlockPlan tet_blocks(int64_t npoin) {
+  if (npoin <= kSmallTetGather) return {small_nodes(npoin, 320), true};
+  return {npoin <= kSmallTet ? small_nodes(npoin, 768) : kKozNodes, false};
+}
+inline BlockPlan cho_blocks(int64_t npoin) {
+  if (npoin <= kSmallCho) return {small_nodes(npoin, 224), true};
+  return {kBlockNodes, false};
+}
 
 int block_order(int64_t npoin, const double* x, const double* y,
                 const double* z, int leaf, size_t* perm);

@@ -6,11 +6,12 @@
 //   rhs:  k_rhs_blocks -- one 512-thread workgroup per node block (two per
 //         CU); the block's node data staged in LDS, one node sum per thread;
 //         k_fixup<5> adds halo partials.
-//   grad: k_grad_blocks -- a gather layout of its own (edges between two
-//         blocks evaluated in both, so no halo partials and no fix-up), also
-//         512 threads and two workgroups per CU, each node thread gathering
-//         its edges' terms from LDS-staged primitive states; k_grad_bnd adds
-//         boundary-face terms.
+//   grad: k_grad_blocks -- a gather layout of its own (edges and boundary
+//         faces between two blocks evaluated in both, so no halo partials
+//         and no fix-up), also 512 threads and two workgroups per CU, each
+//         node thread gathering its edges' terms from LDS-staged primitive
+//         states, then its boundary faces'.
+// Small meshes use gather layouts of small blocks for both (xg::rhs_blocks).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -63,15 +64,19 @@ struct ChunkPrefetch {
   }
 };
 
-// riemann::grad domain term (Riemann.cpp:263-328) on the grad (gather)
-// layout: a block holds every edge touching one of its nodes, so each owned
+// riemann::grad (Riemann.cpp:229-367) on the grad (gather) layout: a block
+// holds every edge and boundary face touching one of its nodes, so each owned
 // node's sum is complete here.  The block's primitive states are staged in
-// LDS.  Per chunk: each thread writes one edge's (u_p + u_q, D) to LDS; then
-// the thread owning local node t adds -/+ D (u_p + u_q) for the chunk's edges
-// touching it, in slot order.
-// DIV: owned nodes without boundary terms (gflag 0) are final here and are
-// divided by their volume (RieCG.cpp:935-939).  NC components per node
-// (5 + transported scalars).
+// LDS.  Per chunk of edges (:263-328): each thread writes one edge's (u_p +
+// u_q, D) to LDS; then the thread owning local node t adds -/+ D (u_p + u_q)
+// for the chunk's edges touching it, in slot order.  Per chunk of boundary
+// faces (:332-359): a thread writes one face's 3 NC values, which as in the
+// reference go to every node of the face alike: g[j] n[j] for direction j,
+// with g[j] the 4:1:1-weighted value belonging to the face's j-th node.  (As a
+// kernel of its own, one thread per boundary node, the faces took 12 us on
+// 2,197 nodes and 23 us on 912,673, of 17 and 199 us for the edges.)
+// DIV: divided by the nodal volume (RieCG.cpp:935-939).  NC components per
+// node (5 + transported scalars).
 template <bool DIV, int NC>
 __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_grad_blocks(
     int nblk, const int4* __restrict__ blk0, const int4* __restrict__ blk1,
@@ -79,12 +84,13 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4)
     const int* __restrict__ chk_ent, const uint16_t* __restrict__ tend,
     const uint16_t* __restrict__ entries, const uint32_t* __restrict__ elpq,
     const double* __restrict__ dx, const double* __restrict__ dy,
-    const double* __restrict__ dz, const double* __restrict__ U,
-    double* __restrict__ G, const uint8_t* __restrict__ gflag,
-    const double* __restrict__ vol) {
+    const double* __restrict__ dz, const uint32_t* __restrict__ fab,
+    const uint32_t* __restrict__ fcs, const double* __restrict__ fn,
+    const double* __restrict__ U, double* __restrict__ G, const double* __restrict__ vol) {
   constexpr int CAP = xg::kGradCap;
   constexpr int FW = NC + 3;   // an edge's record: u_p + u_q, then D
   static_assert(CAP <= kGradThreads, "one local node per thread");
+  static_assert(kGradThreads / 3 * 3 * NC <= kGradThreads * FW, "a chunk's faces fit F");
   __shared__ double sP[NC * CAP];
   __shared__ double F[kGradThreads * FW];
   __shared__ uint16_t sE[2 * kGradThreads];
@@ -92,7 +98,7 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4)
   const int t = threadIdx.x;
   const int b = xcd_block(blockIdx.x, nblk);
   const int4 B0 = blk0[b];   // own0, nown, nloc, halo_off
-  const int4 B1 = blk1[b];   // slot0, chunk0, chunk1
+  const int4 B1 = blk1[b];   // -, chunk0, chunk1
   const int own0 = B0.x, nown = B0.y, nloc = B0.z;
   if (t < nloc) {
     int g = t < nown ? own0 + t : halo[B0.w + t - nown];
@@ -105,10 +111,6 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4)
 #pragma unroll
     for (int c = 0; c < NC; ++c) sP[c * CAP + t] = u[c];
   }
-  // prefetch of the next edge chunk (a gather layout has no boundary-face
-  // chunks, and any would be skipped: k_grad_bnd adds those terms)
-  int ch = B1.y;
-  while (ch < B1.z && chk[ch].x != 0) ++ch;
   ChunkPrefetch<kGradThreads> pf;
   uint32_t pq_n = 0;
   double dx_n = 0.0, dy_n = 0.0, dz_n = 0.0;
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4)
     if (c < B1.z) {
       const int4 C = chk[c];
       pf.load(C, chk_ent[c], nloc, t, tend, entries);
-      if (t < C.z) {
+      if (C.x == 0 && t < C.z) {
         int e = C.y + t;
         pq_n = elpq[e];
         dx_n = dx[e];
@@ -125,49 +127,70 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4)
       }
     }
   };
-  fetch(ch);
+  fetch(B1.y);
   double acc[3 * NC];
 #pragma unroll
   for (int k = 0; k < 3 * NC; ++k) acc[k] = 0.0;
-  while (ch < B1.z) {
+  for (int ch = B1.y; ch < B1.z; ++ch) {
     const int4 C = chk[ch];
-    int nx = ch + 1;
-    while (nx < B1.z && chk[nx].x != 0) ++nx;
     const uint32_t pq = pq_n;
     const double d0 = dx_n, d1 = dy_n, d2 = dz_n;
     __syncthreads();          // staging done / previous chunk consumed
     pf.store(C, nloc, t, sE, sT);
     if (t < C.z) {
-      int lp = pq & 0xffff, lq = pq >> 16;
-      double* f = F + t * FW;
+      if (C.x == 0) {
+        int lp = pq & 0xffff, lq = pq >> 16;
+        double* f = F + t * FW;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) f[c] = sP[c * CAP + lq] + sP[c * CAP + lp];
-      f[NC] = d0;
-      f[NC + 1] = d1;
-      f[NC + 2] = d2;
-    }
-    fetch(nx);                // in flight during the accumulation below
-    __syncthreads();          // F, sE, sT complete
-    if (t < nown) {           // halo nodes have no entries here
-      int e0 = t ? sT[t - 1] : 0, e1 = sT[t];
-      for (int j = e0; j < e1; ++j) {
-        int v = sE[j];
-        const double* f = F + (v & 0x3ff) * FW;
-        double sg = (v & 0x8000) ? -1.0 : 1.0;
-        double D0 = sg * f[NC], D1 = sg * f[NC + 1], D2 = sg * f[NC + 2];
+        for (int c = 0; c < NC; ++c) f[c] = sP[c * CAP + lq] + sP[c * CAP + lp];
+        f[NC] = d0;
+        f[NC + 1] = d1;
+        f[NC + 2] = d2;
+      } else {
+        const size_t fi = (size_t)(C.y + t);
+        const uint32_t ab = fab[fi], cs = fcs[fi];
+        const int A = ab & 0xffff, B = ab >> 16, D = cs & 0xffff;
+        const double n0 = fn[fi * 3], n1 = fn[fi * 3 + 1], n2 = fn[fi * 3 + 2];
+        double* f = F + t * (3 * NC);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-          acc[c * 3 + 0] += D0 * f[c];
-          acc[c * 3 + 1] += D1 * f[c];
-          acc[c * 3 + 2] += D2 * f[c];
+          const double ua = sP[c * CAP + A], ub = sP[c * CAP + B], uc = sP[c * CAP + D];
+          const double uab = (ua + ub) * 0.25, ubc = (ub + uc) * 0.25, uca = (uc + ua) * 0.25;
+          f[c * 3 + 0] = (uab + uca + ua) * n0;
+          f[c * 3 + 1] = (uab + ubc + ub) * n1;
+          f[c * 3 + 2] = (ubc + uca + uc) * n2;
         }
       }
     }
-    ch = nx;
+    fetch(ch + 1);            // in flight during the accumulation below
+    __syncthreads();          // F, sE, sT complete
+    if (t < nown) {           // halo nodes have no entries here
+      int e0 = t ? sT[t - 1] : 0, e1 = sT[t];
+      if (C.x == 0) {
+        for (int j = e0; j < e1; ++j) {
+          int v = sE[j];
+          const double* f = F + (v & 0x3ff) * FW;
+          double sg = (v & 0x8000) ? -1.0 : 1.0;
+          double D0 = sg * f[NC], D1 = sg * f[NC + 1], D2 = sg * f[NC + 2];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            acc[c * 3 + 0] += D0 * f[c];
+            acc[c * 3 + 1] += D1 * f[c];
+            acc[c * 3 + 2] += D2 * f[c];
+          }
+        }
+      } else {
+        for (int j = e0; j < e1; ++j) {
+          const double* f = F + (sE[j] / 3) * (3 * NC);   // slot 3 face + corner
+#pragma unroll
+          for (int k = 0; k < 3 * NC; ++k) acc[k] += f[k];
+        }
+      }
+    }
   }
   if (t < nown) {
     double* o = G + (size_t)(own0 + t) * (3 * NC);
-    if (DIV && gflag[own0 + t] == 0) {
+    if (DIV) {
       const double v = vol[own0 + t];
 #pragma unroll
       for (int k = 0; k < 3 * NC; ++k) o[k] = acc[k] / v;
@@ -176,66 +199,6 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4)
       for (int k = 0; k < 3 * NC; ++k) o[k] = acc[k];
     }
   }
-}
-
-// gflag: the nodes with boundary-face gradient terms
-__global__ void k_gflag(int n, const int* __restrict__ node, uint8_t bit,
-                        uint8_t* __restrict__ gflag) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) gflag[node[i]] |= bit;
-}
-
-__global__ void k_fill_u8(int64_t n, uint8_t* __restrict__ a) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = 0;
-}
-
-// riemann::grad boundary integral (Riemann.cpp:332-359) gathered per node.
-// As in the reference, every node of a face receives g[j]*n[j] for direction
-// j, with g[j] the 4:1:1-weighted value belonging to the face's j-th node.
-// DIV: boundary nodes are final here and are divided by their volume
-template <bool DIV, int NC>
-__global__ __launch_bounds__(kBlock) void k_grad_bnd(
-    int nb, const int* __restrict__ bnode, const int* __restrict__ boff,
-    const int* __restrict__ bface, const int* __restrict__ tri,
-    const double* __restrict__ x, const double* __restrict__ y,
-    const double* __restrict__ z, const double* __restrict__ U,
-    double* __restrict__ G, const double* __restrict__ vol) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb) return;
-  int n = bnode[i];
-  double acc[3 * NC];
-#pragma unroll
-  for (int k = 0; k < 3 * NC; ++k) acc[k] = G[(size_t)n * (3 * NC) + k];
-  for (int k = boff[i]; k < boff[i + 1]; ++k) {
-    int f = bface[k] >> 2;
-    int A = tri[f * 3 + 0], B = tri[f * 3 + 1], C = tri[f * 3 + 2];
-    double u[3][NC];
-    xg::primitive<NC>(U, A, u[0]);
-    xg::primitive<NC>(U, B, u[1]);
-    xg::primitive<NC>(U, C, u[2]);
-    double ba[3] = {x[B] - x[A], y[B] - y[A], z[B] - z[A]};
-    double ca[3] = {x[C] - x[A], y[C] - y[A], z[C] - z[A]};
-    double nr[3] = {(ba[1] * ca[2] - ca[1] * ba[2]) / 12.0,
-                    (ba[2] * ca[0] - ca[2] * ba[0]) / 12.0,
-                    (ba[0] * ca[1] - ca[0] * ba[1]) / 12.0};
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      double uab = (u[0][c] + u[1][c]) / 4.0;
-      double ubc = (u[1][c] + u[2][c]) / 4.0;
-      double uca = (u[2][c] + u[0][c]) / 4.0;
-      double g[3] = {uab + uca + u[0][c], uab + ubc + u[1][c], ubc + uca + u[2][c]};
-#pragma unroll
-      for (int j = 0; j < 3; ++j) acc[c * 3 + j] += g[j] * nr[j];
-    }
-  }
-  if (DIV) {
-    const double v = vol[n];
-#pragma unroll
-    for (int k = 0; k < 3 * NC; ++k) acc[k] /= v;
-  }
-#pragma unroll
-  for (int k = 0; k < 3 * NC; ++k) G[(size_t)n * (3 * NC) + k] = acc[k];
 }
 
 // advbnd (Riemann.cpp:768-878) for one boundary face from the staged
@@ -431,7 +394,7 @@ void k_rhs_blocks(
     double* o = R + (size_t)(own0 + t) * NC;
 #pragma unroll
     for (int c = 0; c < NC; ++c) o[c] = acc[c];
-  } else if (t < nloc) {
+  } else if (t < nloc && B1.x >= 0) {
     double* o = S + (size_t)(B1.x + t - nown) * NC;
 #pragma unroll
     for (int c = 0; c < NC; ++c) o[c] = acc[c];
@@ -570,30 +533,13 @@ int check_mesh(xg_ctx* c, int ncomp) {
 
 template <int NC>
 void launch_grad_nc(xg_ctx* c, const double* U, double* G, bool div) {
-  if (div)
-    hipLaunchKernelGGL((k_grad_blocks<true, NC>), dim3(c->nblk), dim3(kGradThreads), 0,
-                       c->stream, c->nblk, c->blk0, c->blk1, c->halo, c->chk,
-                       c->chk_ent, c->tend, c->entries, c->elpq, c->dx, c->dy,
-                       c->dz, U, G, c->gflag, c->vol);
-  else
-    hipLaunchKernelGGL((k_grad_blocks<false, NC>), dim3(c->nblk), dim3(kGradThreads), 0,
-                       c->stream, c->nblk, c->blk0, c->blk1, c->halo, c->chk,
-                       c->chk_ent, c->tend, c->entries, c->elpq, c->dx, c->dy,
-                       c->dz, U, G, nullptr, nullptr);
-  if (c->nbnode) {
-    if (div)
-      hipLaunchKernelGGL((k_grad_bnd<true, NC>), dim3(nblocks(c->nbnode)), dim3(kBlock), 0,
-                         c->stream, c->nbnode, c->bnode, c->boff, c->bface,
-                         c->tri, c->x, c->y, c->z, U, G, c->vol);
-    else
-      hipLaunchKernelGGL((k_grad_bnd<false, NC>), dim3(nblocks(c->nbnode)), dim3(kBlock), 0,
-                         c->stream, c->nbnode, c->bnode, c->boff, c->bface,
-                         c->tri, c->x, c->y, c->z, U, G, nullptr);
-  }
+  auto kern = div ? k_grad_blocks<true, NC> : k_grad_blocks<false, NC>;
+  hipLaunchKernelGGL(kern, dim3(c->nblk), dim3(kGradThreads), 0, c->stream, c->nblk, c->blk0,
+                     c->blk1, c->halo, c->chk, c->chk_ent, c->tend, c->entries, c->elpq, c->dx,
+                     c->dy, c->dz, c->gfab, c->gfcs, c->gfn, U, G, c->vol);
 }
 
-// div: G = grad(U)/vol (the RK stage; needs xg_riecg_setup), each node
-// divided by the last kernel that adds to it; otherwise grad(U) undivided.
+// div: G = grad(U)/vol (the RK stage; needs xg_riecg_setup).
 // nc components per node (checked by the caller).
 int launch_grad(xg_ctx* c, int nc, const double* U, double* G, bool div = false) {
   static_assert(XG_MAX_NCOMP == 7, "one instantiation per component count");
@@ -880,12 +826,12 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
   std::vector<int> tri32(ntri * 3);
   for (int64_t f = 0; f < ntri * 3; ++f) tri32[f] = (int)tri[f];
   xg::Layout L, LR;
-  int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym,
-                            xg::kGradNodes, xg::kGradCap, xg::kGradSlots, L, c->err,
-                            true);
+  const xg::BlockPlan bg = xg::grad_blocks(npoin), br = xg::rhs_blocks(npoin);
+  int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, bg.nodes,
+                            xg::kGradCap, xg::kGradSlots, L, c->err, bg.gather, true);
   if (rc) return rc;
-  rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, xg::kRhsNodes,
-                        xg::kRhsCap, xg::kRhsSlots, LR, c->err);
+  rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, br.nodes, xg::kRhsCap,
+                        xg::kRhsSlots, LR, c->err, br.gather, true);
   if (rc) return rc;
   std::vector<int4> b0(L.blk.size()), b1(L.blk.size());
   for (size_t b = 0; b < L.blk.size(); ++b) {
@@ -900,23 +846,15 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
     c0[i] = make_int4(C.kind, C.first, C.count, C.tend_off);
     c1[i] = C.ent_off;
   }
-  // boundary gather lists for the gradient: node -> (face*4 + position)
-  std::vector<int> bcnt((size_t)npoin + 1, 0);
-  for (int64_t f = 0; f < ntri * 3; ++f) ++bcnt[tri[f] + 1];
-  std::vector<int> bnode, boff(1, 0), bface;
-  {
-    std::vector<int> start((size_t)npoin + 1, 0);
-    for (int64_t i = 0; i < npoin; ++i) start[i + 1] = start[i] + bcnt[i + 1];
-    std::vector<int> fill(ntri * 3);
-    std::vector<int> pos(start.begin(), start.end() - 1);
-    for (int64_t f = 0; f < ntri; ++f)
-      for (int a = 0; a < 3; ++a) fill[pos[tri[f * 3 + a]]++] = (int)(f * 4 + a);
-    for (int64_t i = 0; i < npoin; ++i) {
-      if (start[i + 1] == start[i]) continue;
-      bnode.push_back((int)i);
-      bface.insert(bface.end(), fill.begin() + start[i], fill.begin() + start[i + 1]);
-      boff.push_back((int)bface.size());
-    }
+  // normals of the grad layout's boundary faces, (b - a) x (c - a) / 12
+  std::vector<double> fn(L.fidx.size() * 3);
+  for (size_t i = 0; i < L.fidx.size(); ++i) {
+    const size_t* N = tri + L.fidx[i] * 3;
+    const double ax = x[N[1]] - x[N[0]], ay = y[N[1]] - y[N[0]], az = z[N[1]] - z[N[0]];
+    const double bx = x[N[2]] - x[N[0]], by = y[N[2]] - y[N[0]], bz = z[N[2]] - z[N[0]];
+    fn[i * 3 + 0] = (ay * bz - by * az) / 12.0;
+    fn[i * 3 + 1] = (az * bx - bz * ax) / 12.0;
+    fn[i * 3 + 2] = (ax * by - bx * ay) / 12.0;
   }
   // device arrays
   (void)hipStreamSynchronize(c->stream);
@@ -932,15 +870,14 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
       (rc = upload(c, M, &c->chk, c0)) || (rc = upload(c, M, &c->chk_ent, c1)) ||
       (rc = upload(c, M, &c->tend, L.tend)) ||
       (rc = upload(c, M, &c->entries, L.entries)) ||
-      (rc = upload(c, M, &c->tri, tri32)) || (rc = upload(c, M, &c->bnode, bnode)) ||
-      (rc = upload(c, M, &c->boff, boff)) || (rc = upload(c, M, &c->bface, bface)))
+      (rc = upload(c, M, &c->gfab, L.fab)) || (rc = upload(c, M, &c->gfcs, L.fcs)) ||
+      (rc = upload(c, M, &c->gfn, fn)))
     return rc;
   if ((rc = upload_blocks(c, M, LR, c->rb))) return rc;
   c->npoin = (int)npoin;
   c->nedge = ne;
   c->nblk = (int)L.blk.size();
   c->nchunk = (int)L.chunks.size();
-  c->nbnode = (int)bnode.size();
   c->have_mesh = true;
   c->have_riecg = false;
   return XG_OK;
@@ -1060,15 +997,8 @@ int xg_riecg_setup(xg_ctx* c, const double* vol, int64_t nsym,
   if ((rc = upload(c, L, &c->vol, vol, (size_t)c->npoin)) ||
       (rc = upload(c, L, &c->symnode, node)) || (rc = upload(c, L, &c->symoff, off)) ||
       (rc = upload(c, L, &c->symnorm, nrm)) ||
-      (rc = dev_alloc(c, L, (void**)&c->red, sizeof(double) * (kRedBlocks + 1))) ||
-      (rc = dev_alloc(c, L, (void**)&c->gflag, (size_t)c->npoin)))
+      (rc = dev_alloc(c, L, (void**)&c->red, sizeof(double) * (kRedBlocks + 1))))
     return rc;
-  hipLaunchKernelGGL(k_fill_u8, dim3(nblocks(c->npoin)), dim3(kBlock), 0, c->stream,
-                     (int64_t)c->npoin, c->gflag);
-  if (c->nbnode)
-    hipLaunchKernelGGL(k_gflag, dim3(nblocks(c->nbnode)), dim3(kBlock), 0, c->stream,
-                       c->nbnode, c->bnode, (uint8_t)1, c->gflag);
-  XG_HIP(c, hipGetLastError());
   c->nsymnode = (int)node.size();
   c->have_riecg = true;
   return XG_OK;
