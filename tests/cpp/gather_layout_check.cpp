@@ -5,17 +5,85 @@
 // index and prefetch bound of the kernels must stay inside its list.
 // Input file: int64 npoin, ne, ntri, ntet; int32 p[ne], q[ne], tri[3 ntri],
 // tet[4 ntet].
-// Arguments: FILE KIND(rhs|grad|cho|tet) NODES GATHER.
+// Arguments: FILE KIND(rhs|grad|cho|tet|rows) NODES GATHER, for rows (node rows,
+// xg_rows.hpp) the lanes per node instead of GATHER.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
 
 #include "../../xyst_amd/csrc/xg_layout.hpp"
+#include "../../xyst_amd/csrc/xg_rows.hpp"
 
 #define CHECK(c) do { if (!(c)) { std::fprintf(stderr, "FAIL %s:%d %s\n", __FILE__, __LINE__, #c); std::exit(1); } } while (0)
 
 static int64_t val(int64_t item, int corner) { return (item * 7 + corner * 3) % 1009 - 500; }
+
+// every edge at both ends with that end's sign, every face at its three nodes,
+// in input order
+static void check_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                       const std::vector<int>& tri, int nodes, int lanes) {
+  std::vector<double> d(3 * p.size());
+  for (size_t i = 0; i < d.size(); ++i) d[i] = 1.0 + (double)i;
+  xg::RowLayout L;
+  std::string err;
+  const int cap = 700, per = 64 / lanes;
+  CHECK(xg::build_rows(npoin, p, q, d, (int64_t)tri.size() / 3, tri.data(), nodes, cap, lanes, L,
+                       err) == 0);
+  std::vector<std::vector<int64_t>> edges(npoin), faces(npoin), ge(npoin), gf(npoin);
+  for (size_t e = 0; e < p.size(); ++e) {
+    edges[p[e]].push_back(-(int64_t)e - 1);
+    edges[q[e]].push_back((int64_t)e + 1);
+  }
+  for (size_t k = 0; k < tri.size(); ++k) faces[tri[k]].push_back(k);
+  int next = 0;
+  for (const auto& B : L.blk) {
+    CHECK(B.own0 == next && B.nown > 0 && B.nown <= nodes && B.nloc <= cap);
+    next += B.nown;
+    CHECK(B.halo_off + B.nloc - B.nown <= (int)L.halo.size());
+    auto glob = [&](int l) {
+      CHECK(l >= 0 && l < B.nloc);
+      return l < B.nown ? B.own0 + l : L.halo[B.halo_off + l - B.nown];
+    };
+    for (int w = 0; w * per < B.nown; ++w) {
+      CHECK(B.wave0 + w < (int)L.wave.size());
+      const auto& W = L.wave[B.wave0 + w];
+      CHECK(W.e0 + 64 * W.erows <= (int)L.nb.size() && L.dx.size() == L.nb.size());
+      CHECK(W.f0 + 64 * W.frows <= (int)L.fab.size());
+      for (int k = w * per; k < std::min(B.nown, (w + 1) * per); ++k)
+        for (int j = 0;; ++j) {
+          const int lane = (k - w * per) * lanes + j % lanes, row = j / lanes;
+          const int g = (B.wave0 + w) * 64 + lane;
+          const bool has = row < L.deg[g], face = row < L.fdeg[g];
+          if (!has && !face) break;
+          CHECK((!has || row < W.erows) && (!face || row < W.frows));
+          if (has) {
+            const size_t at = W.e0 + 64 * (size_t)row + lane;
+            const int64_t e = L.eidx[at];
+            const bool first = L.dx[at] < 0.0;
+            CHECK(L.dx[at] == (first ? -1 : 1) * d[3 * e] &&
+                  L.dy[at] == (first ? -1 : 1) * d[3 * e + 1] &&
+                  L.dz[at] == (first ? -1 : 1) * d[3 * e + 2]);
+            CHECK((first ? p[e] : q[e]) == B.own0 + k);
+            CHECK(glob(L.nb[at]) == (first ? q[e] : p[e]));
+            ge[B.own0 + k].push_back(first ? -e - 1 : e + 1);
+          }
+          if (face) {
+            const size_t at = W.f0 + 64 * (size_t)row + lane;
+            const int64_t f = L.fidx[at];
+            const int a = L.fcs[at] >> 16;
+            CHECK(glob(L.fab[at] & 0xffff) == tri[3 * f] && glob(L.fab[at] >> 16) == tri[3 * f + 1] &&
+                  glob(L.fcs[at] & 0xffff) == tri[3 * f + 2]);
+            CHECK(a < 3 && tri[3 * f + a] == B.own0 + k);
+            gf[B.own0 + k].push_back(3 * f + a);
+          }
+        }
+    }
+  }
+  CHECK(next == npoin);
+  CHECK(ge == edges && gf == faces);
+  std::printf("ok blocks=%zu\n", L.blk.size());
+}
 
 int main(int argc, char** argv) {
   CHECK(argc == 5);
@@ -33,6 +101,10 @@ int main(int argc, char** argv) {
   CHECK(std::fread(tri.data(), 4, tri.size(), f) == tri.size());
   CHECK(std::fread(t32.data(), 4, t32.size(), f) == t32.size());
   std::fclose(f);
+  if (!std::strcmp(kind, "rows")) {
+    check_rows(npoin, p, q, tri, nodes, std::atoi(argv[4]));
+    return 0;
+  }
   std::string err;
   std::vector<int64_t> want(npoin, 0), got(npoin, -1);
   const bool tets = !std::strcmp(kind, "tet");

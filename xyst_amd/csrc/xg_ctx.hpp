@@ -18,6 +18,7 @@ struct KozakMesh;  // xg_kozak.hip
 struct ChoMesh;    // xg_chocg.hip
 struct GnnNet;     // xg_gnn.hip
 struct AmgDev;     // xg_amg.hip
+struct RowsDev;    // xg_rows_dev.hpp
 
 struct xg_ctx {
   int device = 0;
@@ -42,18 +43,7 @@ struct xg_ctx {
   } rb;
   double *x = nullptr, *y = nullptr, *z = nullptr;
   int64_t nedge = 0;
-  uint32_t* elpq = nullptr;
-  double *dx = nullptr, *dy = nullptr, *dz = nullptr;
-  // grad blocks (a gather layout: no halo partials)
-  int nblk = 0, nchunk = 0;
-  int4 *blk0 = nullptr, *blk1 = nullptr;     // (own0,nown,nloc,halo_off), (slot0,chunk0,chunk1,-)
-  int *halo = nullptr;
-  int4 *chk = nullptr;                       // (kind,first,count,tend_off)
-  int *chk_ent = nullptr;                    // ent_off
-  uint16_t *tend = nullptr, *entries = nullptr;
-  // grad boundary faces: local ids, normals (3 per face)
-  uint32_t *gfab = nullptr, *gfcs = nullptr;
-  double* gfn = nullptr;
+  RowsDev* grows = nullptr;    // riemann::grad's node rows (xg_rows_dev.hpp)
   // RieCG stepping
   bool have_riecg = false;
   int ncomp = 5;                         // components per node (xg_riecg_set_ncomp)

@@ -25,6 +25,7 @@
 // The layout is fastest when node ids are block-contiguous and spatially
 // compact (xg_mesh_block_order), but is correct for any numbering.
 #include "xg_layout.hpp"
+#include "xg_rows.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -283,6 +284,142 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     L.fx_node.push_back(n);
     for (auto& bs : fix[n]) L.fx_slot.push_back(bs.second);
     L.fx_off.push_back((int)L.fx_slot.size());
+  }
+  return XG_OK;
+}
+
+int build_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+               const std::vector<double>& d, int64_t ntri, const int* tri, int block_nodes,
+               int cap, int lanes, RowLayout& L, std::string& err) {
+  L = RowLayout();
+  const int64_t ne = (int64_t)p.size();
+  if (lanes < 1 || 64 % lanes || cap > 65535) {
+    err = "rows: bad lanes or capacity";
+    return XG_EINVAL;
+  }
+  // the edges of every node, in input order; its faces
+  std::vector<int64_t> off(npoin + 1, 0), foff(npoin + 1, 0);
+  for (int64_t e = 0; e < ne; ++e) {
+    ++off[p[e] + 1];
+    ++off[q[e] + 1];
+  }
+  for (int64_t k = 0; k < 3 * ntri; ++k) ++foff[tri[k] + 1];
+  for (int i = 0; i < npoin; ++i) {
+    off[i + 1] += off[i];
+    foff[i + 1] += foff[i];
+  }
+  std::vector<int64_t> inc(off[npoin]), finc(foff[npoin]);
+  {
+    std::vector<int64_t> pos(off.begin(), off.end() - 1);
+    for (int64_t e = 0; e < ne; ++e) {
+      inc[pos[p[e]]++] = e;
+      inc[pos[q[e]]++] = e;
+    }
+    pos.assign(foff.begin(), foff.end() - 1);
+    for (int64_t k = 0; k < 3 * ntri; ++k) finc[pos[tri[k]]++] = k;
+  }
+  // neighbours of every node (of its faces too) for the partition
+  std::vector<int64_t> uoff(npoin + 1, 0);
+  std::vector<int> up;
+  up.reserve(inc.size() + 2 * finc.size());
+  for (int i = 0; i < npoin; ++i) {
+    for (int64_t k = off[i]; k < off[i + 1]; ++k)
+      up.push_back(p[inc[k]] == i ? q[inc[k]] : p[inc[k]]);
+    for (int64_t k = foff[i]; k < foff[i + 1]; ++k) {
+      const int* N = tri + finc[k] / 3 * 3;
+      for (int a = 0; a < 3; ++a)
+        if (N[a] != i) up.push_back(N[a]);
+    }
+    uoff[i + 1] = (int64_t)up.size();
+  }
+  std::vector<int> bstart;
+  int rc = partition_blocks(npoin, uoff, up, block_nodes, cap, bstart, err);
+  if (rc) return rc;
+  const int nblk = (int)bstart.size() - 1;
+  std::vector<int> local(npoin, -1);
+  L.blk.resize(nblk);
+  for (int b = 0; b < nblk; ++b) {
+    RowBlock& B = L.blk[b];
+    const int s = bstart[b], e = bstart[b + 1];
+    B.own0 = s;
+    B.nown = e - s;
+    B.halo_off = (int)L.halo.size();
+    std::vector<int> halo;
+    for (int i = s; i < e; ++i)
+      for (int64_t k = uoff[i]; k < uoff[i + 1]; ++k)
+        if (up[k] < s || up[k] >= e) halo.push_back(up[k]);
+    std::sort(halo.begin(), halo.end());
+    halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
+    L.halo.insert(L.halo.end(), halo.begin(), halo.end());
+    B.nloc = B.nown + (int)halo.size();
+    if (B.nloc > cap) {
+      err = "rows: block exceeds its capacity";
+      return XG_EUNSUPPORTED;
+    }
+    for (int i = s; i < e; ++i) local[i] = i - s;
+    for (size_t h = 0; h < halo.size(); ++h) local[halo[h]] = B.nown + (int)h;
+    B.wave0 = (int)L.wave.size();
+    const int per = 64 / lanes;   // nodes of a wave
+    for (int w0 = 0; w0 < B.nown; w0 += per) {
+      RowWave W;
+      int64_t most = 0, fmost = 0;
+      for (int k = w0; k < std::min(B.nown, w0 + per); ++k) {
+        most = std::max(most, off[s + k + 1] - off[s + k]);
+        fmost = std::max(fmost, foff[s + k + 1] - foff[s + k]);
+      }
+      W.erows = (int)((most + lanes - 1) / lanes);
+      W.frows = (int)((fmost + lanes - 1) / lanes);
+      if (W.erows > 255 || W.frows > 255) {
+        err = "rows: too many edges at a node";
+        return XG_EUNSUPPORTED;
+      }
+      W.e0 = (int)L.nb.size();
+      W.f0 = (int)L.fab.size();
+      if (L.nb.size() + 64 * (size_t)W.erows >= (1u << 31)) {
+        err = "rows: too many edges";
+        return XG_EUNSUPPORTED;
+      }
+      L.wave.push_back(W);
+      L.nb.resize(W.e0 + 64 * (size_t)W.erows, 0);
+      L.dx.resize(L.nb.size(), 0.0);
+      L.dy.resize(L.nb.size(), 0.0);
+      L.dz.resize(L.nb.size(), 0.0);
+      L.eidx.resize(L.nb.size(), -1);
+      L.fab.resize(W.f0 + 64 * (size_t)W.frows, 0);
+      L.fcs.resize(L.fab.size(), 0);
+      L.fidx.resize(L.fab.size(), -1);
+      const size_t g0 = L.deg.size();
+      L.deg.resize(g0 + 64, 0);
+      L.fdeg.resize(g0 + 64, 0);
+      for (int k = w0; k < std::min(B.nown, w0 + per); ++k) {
+        const int i = s + k, l0 = (k - w0) * lanes;
+        for (int64_t j = 0; j < off[i + 1] - off[i]; ++j) {
+          const int64_t ed = inc[off[i] + j];
+          const int lane = l0 + (int)(j % lanes);
+          const size_t at = W.e0 + 64 * (size_t)(j / lanes) + lane;
+          const bool first = p[ed] == i;
+          const double sg = first ? -1.0 : 1.0;
+          L.nb[at] = (uint16_t)local[first ? q[ed] : p[ed]];
+          L.dx[at] = sg * d[ed * 3];
+          L.dy[at] = sg * d[ed * 3 + 1];
+          L.dz[at] = sg * d[ed * 3 + 2];
+          L.eidx[at] = ed;
+          ++L.deg[g0 + lane];
+        }
+        for (int64_t j = 0; j < foff[i + 1] - foff[i]; ++j) {
+          const int64_t f = finc[foff[i] + j] / 3, a = finc[foff[i] + j] % 3;
+          const int lane = l0 + (int)(j % lanes);
+          const size_t at = W.f0 + 64 * (size_t)(j / lanes) + lane;
+          const int* N = tri + f * 3;
+          L.fab[at] = (uint32_t)local[N[0]] | ((uint32_t)local[N[1]] << 16);
+          L.fcs[at] = (uint32_t)local[N[2]] | ((uint32_t)a << 16);
+          L.fidx[at] = f;
+          ++L.fdeg[g0 + lane];
+        }
+      }
+    }
+    for (int i = s; i < e; ++i) local[i] = -1;
+    for (int h : halo) local[h] = -1;
   }
   return XG_OK;
 }

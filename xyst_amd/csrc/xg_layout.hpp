@@ -16,12 +16,14 @@ constexpr int kChunkSlots = 1024;
 constexpr int kBlockCap = 616;
 // owned nodes per block (a block also stops growing at kBlockCap)
 constexpr int kBlockNodes = 432;
-// riemann::grad blocks (a gather layout): 5 primitive doubles per local
-// node beside 512 slots of 8 doubles and the entry lists, 56,320 bytes of
-// LDS, so two 512-thread workgroups share a CU
-constexpr int kGradSlots = 512;
-constexpr int kGradCap = 512;
+// riemann::grad blocks (node rows, xg_rows.hpp): one thread per owned node,
+// the primitive state of the local ones in LDS (30,720 bytes: five
+// workgroups share a CU); small meshes: 16 nodes, four lanes each.
+// kGradSlots: chunk slots where a gather layout is built at these sizes.
 constexpr int kGradNodes = 384;
+constexpr int kGradCap = 768;
+constexpr int kGradSlots = 1024;
+constexpr int kGradSmallCap = 256;
 // riemann::rhs has blocks of its own, small enough that two 512-thread
 // workgroups share a CU: 23 doubles per local node, 512 flux slots of 5
 // doubles and the entry lists take 80,560 of the 81,920 bytes of LDS each
@@ -112,9 +114,8 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
 // they are cut into about as many blocks as run at once, and where that is
 // the faster, into gather blocks, which need no halo fix-up.  Times of the
 // full blocks and of these, in us:
-//  riemann::grad (two workgroups per CU: at most 512 blocks): RieCG step of
-//    three gradients on 33^3 (39,304 nodes) 241 -> 183, on 40^3 equal;
-//  riemann::rhs (likewise): 12^3 20.6 -> 6.9, 24^3 21.1 -> 9.9, 29^3 (27,000
+//  riemann::grad: sixteen nodes, four lanes each (its waves are independent);
+//  riemann::rhs (two workgroups per CU: at most 512 blocks): 12^3 20.6 -> 6.9, 24^3 21.1 -> 9.9, 29^3 (27,000
 //    nodes) 23.7 -> 14.5, with 6 components (one workgroup per CU) 23.9 ->
 //    20.5; on 31^3 (32,768) 22.4 -> 20.4, but 22.7 -> 27.9 with 6;
 //  the tet operators, KozCG step: 12^3 201 -> 84, 20^3 (9,261) 201 -> 104, as
@@ -136,9 +137,6 @@ struct BlockPlan {
 
 inline int small_nodes(int64_t npoin, int64_t nblk) {
   return (int)(npoin < 16 * nblk ? 16 : (npoin + nblk - 1) / nblk);
-}
-inline BlockPlan grad_blocks(int64_t npoin) {
-  return {npoin <= kSmallGrad ? small_nodes(npoin, 512) : kGradNodes, true};
 }
 inline BlockPlan rhs_blocks(int64_t npoin) {
   if (npoin <= kSmallRhs) return {small_nodes(npoin, 512), true};

@@ -6,12 +6,10 @@
 //   rhs:  k_rhs_blocks -- one 512-thread workgroup per node block (two per
 //         CU); the block's node data staged in LDS, one node sum per thread;
 //         k_fixup<5> adds halo partials.
-//   grad: k_grad_blocks -- a gather layout of its own (edges and boundary
-//         faces between two blocks evaluated in both, so no halo partials
-//         and no fix-up), also 512 threads and two workgroups per CU, each
-//         node thread gathering its edges' terms from LDS-staged primitive
-//         states, then its boundary faces'.
-// Small meshes use gather layouts of small blocks for both (xg::rhs_blocks).
+//   grad: k_grad_rows -- node rows (xg_rows.hpp): each edge evaluated at both
+//         ends, a lane per node.
+// Small meshes use gather blocks for the rhs (xg::rhs_blocks) and four lanes
+// per node for the gradient.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,6 +25,7 @@
 using xg::Cfg;
 
 #include "xg_blocks.hpp"
+#include "xg_rows_dev.hpp"
 #include "xg_amg.hpp"
 #include "xg_ctx.hpp"
 #include "xg_gnn.hpp"
@@ -34,10 +33,138 @@ using xg::Cfg;
 namespace {
 
 using namespace xgd;
-constexpr int kGradThreads = xg::kGradSlots;
 constexpr int kRhsThreads = xg::kRhsSlots;
 
 // ----------------------------------------------------------------- kernels --
+
+// riemann::grad (Riemann.cpp:229-367) on node rows (xg_rows.hpp): the block's
+// primitive states are staged in LDS, then each node's lane (or LPN lanes)
+// adds D (u + u_neighbour) over its edges (:263-328), reading neighbour ids
+// and integrals with consecutive addresses across the wave, and over its
+// boundary faces (:332-359) the faces' values, which as in the reference go
+// to every node of a face alike: g[j] n[j] for direction j, with g[j] the
+// 4:1:1-weighted value belonging to the face's j-th node.
+// What bounds it: the bytes, 26 per entry (two entries an edge), 40 of U (about
+// twice, with the halo) and 120 of G per node: 0.51 GB on 96^3 (912,673
+// nodes), 128 us, 4.0 TB/s.  A block kernel that evaluated an edge once or
+// twice into LDS and summed it per node between barriers took 207 us.  Two rows
+// in flight instead of four: 131 us; six waves per SIMD (spills): 135 us.
+// DIV: divided by the nodal volume (RieCG.cpp:935-939).  NC components per
+// node (5 + transported scalars).
+template <bool DIV, int NC, int LPN, int NT, int CAP>
+__global__ __launch_bounds__(NT) void k_grad_rows(RowsDev L, const double* __restrict__ U,
+                                                 double* __restrict__ G,
+                                                 const double* __restrict__ vol) {
+  constexpr int K = 3 * NC;
+  constexpr int AHEAD = 4;     // rows in flight
+  __shared__ double sP[NC * CAP];
+  static_assert(NT / 64 * 32 * K <= NC * CAP || LPN > 1, "the stores' buffers reuse sP");
+  const int t = threadIdx.x, lane = t & 63;
+  const int b = xcd_block(blockIdx.x, L.nblk);
+  const int4 B = L.blk[b];     // own0, nown, nloc, halo_off
+  const int w0 = L.wave0[b];
+  const int own0 = B.x, nown = B.y, nloc = B.z;
+  for (int i = t; i < nloc; i += NT) {
+    const int g = i < nown ? own0 + i : L.halo[B.w + i - nown];
+    double s[NC], u[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) s[c] = U[(size_t)g * NC + c];
+    xg::primitive_fast(s, u);
+#pragma unroll
+    for (int c = 5; c < NC; ++c) u[c] = s[c];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) sP[c * CAP + i] = u[c];
+  }
+  const int n = t / LPN;       // local node
+  const bool any = (t & ~63) / LPN < nown;   // the wave has nodes
+  int4 W = make_int4(0, 0, 0, 0);
+  int deg = 0, fdeg = 0;
+  if (any) {
+    W = L.wave[w0 + (t >> 6)];
+    deg = L.deg[(w0 + (t >> 6)) * 64 + lane];
+    fdeg = L.fdeg[(w0 + (t >> 6)) * 64 + lane];
+  }
+  int nb[AHEAD];
+  double D[AHEAD][3];
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (j0 + u < W.y) {      // the same for the wave
+        const int e = W.x + (j0 + u) * 64 + lane;
+        nb[u] = L.nb[e];
+        D[u][0] = L.dx[e];
+        D[u][1] = L.dy[e];
+        D[u][2] = L.dz[e];
+      }
+  };
+  fetch(0);
+  __syncthreads();             // the block's nodes are staged
+  double own[NC], acc[K];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) own[c] = sP[c * CAP + min(n, nloc - 1)];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc[k] = 0.0;
+  for (int j0 = 0; j0 < W.y; j0 += AHEAD) {
+    int m[AHEAD];
+    double d[AHEAD][3];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      m[u] = nb[u];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) d[u][k] = D[u][k];
+    }
+    fetch(j0 + AHEAD);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (j0 + u < deg) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const double f = own[c] + sP[c * CAP + m[u]];
+          acc[c * 3 + 0] += d[u][0] * f;
+          acc[c * 3 + 1] += d[u][1] * f;
+          acc[c * 3 + 2] += d[u][2] * f;
+        }
+      }
+  }
+  for (int j = 0; j < W.w; ++j) {
+    if (j >= fdeg) continue;
+    const size_t e = (size_t)W.z + j * 64 + lane;
+    const uint32_t ab = L.fab[e], cs = L.fcs[e];
+    const int a = ab & 0xffff, bb = ab >> 16, cc = cs & 0xffff;
+    const double n0 = L.fn[e * 3], n1 = L.fn[e * 3 + 1], n2 = L.fn[e * 3 + 2];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const double ua = sP[c * CAP + a], ub = sP[c * CAP + bb], uc = sP[c * CAP + cc];
+      const double uab = (ua + ub) * 0.25, ubc = (ub + uc) * 0.25, uca = (uc + ua) * 0.25;
+      acc[c * 3 + 0] += (uab + uca + ua) * n0;
+      acc[c * 3 + 1] += (uab + ubc + ub) * n1;
+      acc[c * 3 + 2] += (ubc + uca + uc) * n2;
+    }
+  }
+  if (LPN > 1) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] = node_sum<LPN>(acc[k]);
+  }
+  if (DIV && n < nown) {
+    const double v = vol[own0 + n];
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] /= v;
+  }
+  if constexpr (LPN > 1) {
+    if (n < nown) {
+      double* o = G + (size_t)(own0 + n) * K;
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if ((k & (LPN - 1)) == (t & (LPN - 1))) o[k] = acc[k];
+    }
+  } else {
+    __syncthreads();           // sP is read no more
+    const int left = nown - (t & ~63);
+    if (left > 0)
+      store_nodes<K>(acc, sP + (t >> 6) * 32 * K, G + (size_t)(own0 + (t & ~63)) * K,
+                     min(left, 64), lane);
+  }
+}
 
 // Per-chunk bookkeeping shared by the block kernels: the chunk's entry list
 // (slot | sign bit, grouped by local node) and each local node's entry end
@@ -63,143 +190,6 @@ struct ChunkPrefetch {
     if (t < nloc) sT[t] = te;
   }
 };
-
-// riemann::grad (Riemann.cpp:229-367) on the grad (gather) layout: a block
-// holds every edge and boundary face touching one of its nodes, so each owned
-// node's sum is complete here.  The block's primitive states are staged in
-// LDS.  Per chunk of edges (:263-328): each thread writes one edge's (u_p +
-// u_q, D) to LDS; then the thread owning local node t adds -/+ D (u_p + u_q)
-// for the chunk's edges touching it, in slot order.  Per chunk of boundary
-// faces (:332-359): a thread writes one face's 3 NC values, which as in the
-// reference go to every node of the face alike: g[j] n[j] for direction j,
-// with g[j] the 4:1:1-weighted value belonging to the face's j-th node.  (As a
-// kernel of its own, one thread per boundary node, the faces took 12 us on
-// 2,197 nodes and 23 us on 912,673, of 17 and 199 us for the edges.)
-// DIV: divided by the nodal volume (RieCG.cpp:935-939).  NC components per
-// node (5 + transported scalars).
-template <bool DIV, int NC>
-__global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_grad_blocks(
-    int nblk, const int4* __restrict__ blk0, const int4* __restrict__ blk1,
-    const int* __restrict__ halo, const int4* __restrict__ chk,
-    const int* __restrict__ chk_ent, const uint16_t* __restrict__ tend,
-    const uint16_t* __restrict__ entries, const uint32_t* __restrict__ elpq,
-    const double* __restrict__ dx, const double* __restrict__ dy,
-    const double* __restrict__ dz, const uint32_t* __restrict__ fab,
-    const uint32_t* __restrict__ fcs, const double* __restrict__ fn,
-    const double* __restrict__ U, double* __restrict__ G, const double* __restrict__ vol) {
-  constexpr int CAP = xg::kGradCap;
-  constexpr int FW = NC + 3;   // an edge's record: u_p + u_q, then D
-  static_assert(CAP <= kGradThreads, "one local node per thread");
-  static_assert(kGradThreads / 3 * 3 * NC <= kGradThreads * FW, "a chunk's faces fit F");
-  __shared__ double sP[NC * CAP];
-  __shared__ double F[kGradThreads * FW];
-  __shared__ uint16_t sE[2 * kGradThreads];
-  __shared__ uint16_t sT[CAP];
-  const int t = threadIdx.x;
-  const int b = xcd_block(blockIdx.x, nblk);
-  const int4 B0 = blk0[b];   // own0, nown, nloc, halo_off
-  const int4 B1 = blk1[b];   // -, chunk0, chunk1
-  const int own0 = B0.x, nown = B0.y, nloc = B0.z;
-  if (t < nloc) {
-    int g = t < nown ? own0 + t : halo[B0.w + t - nown];
-    double s[NC], u[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) s[c] = U[(size_t)g * NC + c];
-    xg::primitive_fast(s, u);
-#pragma unroll
-    for (int c = 5; c < NC; ++c) u[c] = s[c];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) sP[c * CAP + t] = u[c];
-  }
-  ChunkPrefetch<kGradThreads> pf;
-  uint32_t pq_n = 0;
-  double dx_n = 0.0, dy_n = 0.0, dz_n = 0.0;
-  auto fetch = [&](int c) {
-    if (c < B1.z) {
-      const int4 C = chk[c];
-      pf.load(C, chk_ent[c], nloc, t, tend, entries);
-      if (C.x == 0 && t < C.z) {
-        int e = C.y + t;
-        pq_n = elpq[e];
-        dx_n = dx[e];
-        dy_n = dy[e];
-        dz_n = dz[e];
-      }
-    }
-  };
-  fetch(B1.y);
-  double acc[3 * NC];
-#pragma unroll
-  for (int k = 0; k < 3 * NC; ++k) acc[k] = 0.0;
-  for (int ch = B1.y; ch < B1.z; ++ch) {
-    const int4 C = chk[ch];
-    const uint32_t pq = pq_n;
-    const double d0 = dx_n, d1 = dy_n, d2 = dz_n;
-    __syncthreads();          // staging done / previous chunk consumed
-    pf.store(C, nloc, t, sE, sT);
-    if (t < C.z) {
-      if (C.x == 0) {
-        int lp = pq & 0xffff, lq = pq >> 16;
-        double* f = F + t * FW;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) f[c] = sP[c * CAP + lq] + sP[c * CAP + lp];
-        f[NC] = d0;
-        f[NC + 1] = d1;
-        f[NC + 2] = d2;
-      } else {
-        const size_t fi = (size_t)(C.y + t);
-        const uint32_t ab = fab[fi], cs = fcs[fi];
-        const int A = ab & 0xffff, B = ab >> 16, D = cs & 0xffff;
-        const double n0 = fn[fi * 3], n1 = fn[fi * 3 + 1], n2 = fn[fi * 3 + 2];
-        double* f = F + t * (3 * NC);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const double ua = sP[c * CAP + A], ub = sP[c * CAP + B], uc = sP[c * CAP + D];
-          const double uab = (ua + ub) * 0.25, ubc = (ub + uc) * 0.25, uca = (uc + ua) * 0.25;
-          f[c * 3 + 0] = (uab + uca + ua) * n0;
-          f[c * 3 + 1] = (uab + ubc + ub) * n1;
-          f[c * 3 + 2] = (ubc + uca + uc) * n2;
-        }
-      }
-    }
-    fetch(ch + 1);            // in flight during the accumulation below
-    __syncthreads();          // F, sE, sT complete
-    if (t < nown) {           // halo nodes have no entries here
-      int e0 = t ? sT[t - 1] : 0, e1 = sT[t];
-      if (C.x == 0) {
-        for (int j = e0; j < e1; ++j) {
-          int v = sE[j];
-          const double* f = F + (v & 0x3ff) * FW;
-          double sg = (v & 0x8000) ? -1.0 : 1.0;
-          double D0 = sg * f[NC], D1 = sg * f[NC + 1], D2 = sg * f[NC + 2];
-#pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            acc[c * 3 + 0] += D0 * f[c];
-            acc[c * 3 + 1] += D1 * f[c];
-            acc[c * 3 + 2] += D2 * f[c];
-          }
-        }
-      } else {
-        for (int j = e0; j < e1; ++j) {
-          const double* f = F + (sE[j] / 3) * (3 * NC);   // slot 3 face + corner
-#pragma unroll
-          for (int k = 0; k < 3 * NC; ++k) acc[k] += f[k];
-        }
-      }
-    }
-  }
-  if (t < nown) {
-    double* o = G + (size_t)(own0 + t) * (3 * NC);
-    if (DIV) {
-      const double v = vol[own0 + t];
-#pragma unroll
-      for (int k = 0; k < 3 * NC; ++k) o[k] = acc[k] / v;
-    } else {
-#pragma unroll
-      for (int k = 0; k < 3 * NC; ++k) o[k] = acc[k];
-    }
-  }
-}
 
 // advbnd (Riemann.cpp:768-878) for one boundary face from the staged
 // primitive states: the three corner contributions (fab + fca + f_a style
@@ -533,10 +523,16 @@ int check_mesh(xg_ctx* c, int ncomp) {
 
 template <int NC>
 void launch_grad_nc(xg_ctx* c, const double* U, double* G, bool div) {
-  auto kern = div ? k_grad_blocks<true, NC> : k_grad_blocks<false, NC>;
-  hipLaunchKernelGGL(kern, dim3(c->nblk), dim3(kGradThreads), 0, c->stream, c->nblk, c->blk0,
-                     c->blk1, c->halo, c->chk, c->chk_ent, c->tend, c->entries, c->elpq, c->dx,
-                     c->dy, c->dz, c->gfab, c->gfcs, c->gfn, U, G, c->vol);
+  const RowsDev& L = *c->grows;
+  if (L.lanes == 1) {
+    auto kern = div ? k_grad_rows<true, NC, 1, xg::kGradNodes, xg::kGradCap>
+                    : k_grad_rows<false, NC, 1, xg::kGradNodes, xg::kGradCap>;
+    hipLaunchKernelGGL(kern, dim3(L.nblk), dim3(xg::kGradNodes), 0, c->stream, L, U, G, c->vol);
+  } else {
+    auto kern = div ? k_grad_rows<true, NC, 4, 64, xg::kGradSmallCap>
+                    : k_grad_rows<false, NC, 4, 64, xg::kGradSmallCap>;
+    hipLaunchKernelGGL(kern, dim3(L.nblk), dim3(64), 0, c->stream, L, U, G, c->vol);
+  }
 }
 
 // div: G = grad(U)/vol (the RK stage; needs xg_riecg_setup).
@@ -759,6 +755,7 @@ int xg_ctx_destroy(xg_ctx* c) {
   if (c->gnn) xg_gnn_free(c);
   if (c->diagbuf.p) (void)hipFree(c->diagbuf.p);
   if (c->amg) xg_amg_free(c);
+  delete c->grows;
   delete c;
   return XG_OK;
 }
@@ -825,30 +822,27 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
       return fail(c, XG_EINVAL, "xg_mesh_upload: boundary face node out of range");
   std::vector<int> tri32(ntri * 3);
   for (int64_t f = 0; f < ntri * 3; ++f) tri32[f] = (int)tri[f];
-  xg::Layout L, LR;
-  const xg::BlockPlan bg = xg::grad_blocks(npoin), br = xg::rhs_blocks(npoin);
-  int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, bg.nodes,
-                            xg::kGradCap, xg::kGradSlots, L, c->err, bg.gather, true);
+  const xg::BlockPlan br = xg::rhs_blocks(npoin);
+  xg::RowLayout L;
+  xg::Layout LR;
+  int lanes = npoin <= xg::kSmallGrad ? 4 : 1;
+  int rc = XG_EUNSUPPORTED;
+  if (lanes == 4)   // a node with too many neighbours for it: the other
+    rc = xg::build_rows((int)npoin, p, q, d, ntri, tri32.data(), 16, xg::kGradSmallCap, 4, L,
+                        c->err);
+  if (rc == XG_EUNSUPPORTED) {
+    lanes = 1;
+    rc = xg::build_rows((int)npoin, p, q, d, ntri, tri32.data(), xg::kGradNodes, xg::kGradCap,
+                        1, L, c->err);
+  }
   if (rc) return rc;
   rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, br.nodes, xg::kRhsCap,
                         xg::kRhsSlots, LR, c->err, br.gather, true);
   if (rc) return rc;
-  std::vector<int4> b0(L.blk.size()), b1(L.blk.size());
-  for (size_t b = 0; b < L.blk.size(); ++b) {
-    const auto& B = L.blk[b];
-    b0[b] = make_int4(B.own0, B.nown, B.nloc, B.halo_off);
-    b1[b] = make_int4(B.slot0, B.chunk0, B.chunk1, 0);
-  }
-  std::vector<int4> c0(L.chunks.size());
-  std::vector<int> c1(L.chunks.size());
-  for (size_t i = 0; i < L.chunks.size(); ++i) {
-    const auto& C = L.chunks[i];
-    c0[i] = make_int4(C.kind, C.first, C.count, C.tend_off);
-    c1[i] = C.ent_off;
-  }
-  // normals of the grad layout's boundary faces, (b - a) x (c - a) / 12
-  std::vector<double> fn(L.fidx.size() * 3);
+  // normals of the rows' boundary faces, (b - a) x (c - a) / 12
+  std::vector<double> fn(L.fidx.size() * 3, 0.0);
   for (size_t i = 0; i < L.fidx.size(); ++i) {
+    if (L.fidx[i] < 0) continue;
     const size_t* N = tri + L.fidx[i] * 3;
     const double ax = x[N[1]] - x[N[0]], ay = y[N[1]] - y[N[0]], az = z[N[1]] - z[N[0]];
     const double bx = x[N[2]] - x[N[0]], by = y[N[2]] - y[N[0]], bz = z[N[2]] - z[N[0]];
@@ -862,22 +856,13 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
   c->have_mesh = false;
   auto& M = c->mesh_allocs;
   if ((rc = upload(c, M, &c->x, x, npoin)) || (rc = upload(c, M, &c->y, y, npoin)) ||
-      (rc = upload(c, M, &c->z, z, npoin)) || (rc = upload(c, M, &c->elpq, L.elpq)) ||
-      (rc = upload(c, M, &c->dx, L.dx)) ||
-      (rc = upload(c, M, &c->dy, L.dy)) || (rc = upload(c, M, &c->dz, L.dz)) ||
-      (rc = upload(c, M, &c->blk0, b0)) || (rc = upload(c, M, &c->blk1, b1)) ||
-      (rc = upload(c, M, &c->halo, L.halo)) ||
-      (rc = upload(c, M, &c->chk, c0)) || (rc = upload(c, M, &c->chk_ent, c1)) ||
-      (rc = upload(c, M, &c->tend, L.tend)) ||
-      (rc = upload(c, M, &c->entries, L.entries)) ||
-      (rc = upload(c, M, &c->gfab, L.fab)) || (rc = upload(c, M, &c->gfcs, L.fcs)) ||
-      (rc = upload(c, M, &c->gfn, fn)))
+      (rc = upload(c, M, &c->z, z, npoin)))
     return rc;
+  if (!c->grows) c->grows = new RowsDev;
+  if ((rc = upload_rows(c, M, L, fn, lanes, *c->grows))) return rc;
   if ((rc = upload_blocks(c, M, LR, c->rb))) return rc;
   c->npoin = (int)npoin;
   c->nedge = ne;
-  c->nblk = (int)L.blk.size();
-  c->nchunk = (int)L.chunks.size();
   c->have_mesh = true;
   c->have_riecg = false;
   return XG_OK;
