@@ -103,6 +103,20 @@ static void full_lists(int npoin, const std::vector<int>& p, const std::vector<i
   }
 }
 
+// Appends a chunk's entries (local node, slot | sign) grouped by node, each
+// node's in the order given, and every local node's entry end.
+static void group_entries(const std::vector<std::pair<int, uint16_t>>& ent, int nloc,
+                          std::vector<uint16_t>& entries, std::vector<uint16_t>& tend) {
+  const size_t e0 = entries.size(), t0 = tend.size();
+  std::vector<int> pos(nloc + 1, 0);
+  for (const auto& e : ent) ++pos[e.first + 1];
+  for (int n = 0; n < nloc; ++n) pos[n + 1] += pos[n];
+  tend.resize(t0 + nloc);
+  for (int n = 0; n < nloc; ++n) tend[t0 + n] = (uint16_t)pos[n + 1];
+  entries.resize(e0 + ent.size());
+  for (const auto& e : ent) entries[e0 + pos[e.first]++] = e.second;
+}
+
 // Cuts a block's items (edges or tets, in local order) into chunks of at most
 // `slots`, spreading the items of a node over the chunks: a chunk's node sums
 // take as long as the node with the most entries in it.  In local order alone
@@ -254,20 +268,13 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     // a dense table of per-node entry ends over all nloc local nodes
     auto emit = [&](int kind, int64_t first, int count,
                     const std::vector<std::pair<int, uint16_t>>& ent) {
-      std::vector<std::pair<int, uint16_t>> s(ent);
-      std::stable_sort(s.begin(), s.end(),
-                       [](const auto& x, const auto& y) { return x.first < y.first; });
       Chunk C;
       C.kind = kind;
       C.first = (int)first;
       C.count = count;
       C.tend_off = (int)L.tend.size();
       C.ent_off = (int)L.entries.size();
-      size_t k = 0;
-      for (int n = 0; n < B.nloc; ++n) {
-        while (k < s.size() && s[k].first == n) L.entries.push_back(s[k++].second);
-        L.tend.push_back((uint16_t)(L.entries.size() - C.ent_off));
-      }
+      group_entries(ent, B.nloc, L.entries, L.tend);
       L.chunks.push_back(C);
     };
     const auto parts = spread_chunks(E, chunk_slots, B.nloc, [&](int64_t e, int* node) {
@@ -602,19 +609,13 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
         for (int a = 0; a < 4; ++a)
           if (!gather || local[inpoel[P[i] * 4 + a]] < B.nown)
             ent.emplace_back(local[inpoel[P[i] * 4 + a]], (uint16_t)(4 * i + a));
-      std::stable_sort(ent.begin(), ent.end(),
-                       [](const auto& x, const auto& y) { return x.first < y.first; });
       Chunk C;
       C.kind = 2;
       C.first = (int)L.tab.size();
       C.count = (int)P.size();
       C.tend_off = (int)L.tend.size();
       C.ent_off = (int)L.entries.size();
-      size_t k = 0;
-      for (int n = 0; n < B.nloc; ++n) {
-        while (k < ent.size() && ent[k].first == n) L.entries.push_back(ent[k++].second);
-        L.tend.push_back((uint16_t)(L.entries.size() - C.ent_off));
-      }
+      group_entries(ent, B.nloc, L.entries, L.tend);
       L.chunks.push_back(C);
       for (int64_t e : P) {
         const size_t* N = inpoel + e * 4;
