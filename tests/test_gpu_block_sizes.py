@@ -75,6 +75,35 @@ def test_kozak(n):
     ctx.close()
 
 
+# the node kernels of the step add the halo slots themselves: full blocks
+# (halo slots) at 40, gather blocks (none) at 12; 5 and 6 components.  The
+# kernels repeat the oracle's operations per tet; the order of a node's sums
+# and the half step's rounding differ.
+@pytest.mark.parametrize("n,ns,fct", [(12, 1, True), (40, 0, False), (40, 1, False),
+                                      (40, 1, True)])
+def test_kozcg_halo_sums(n, ns, fct):
+    import torch
+    from xyst_amd import kozak as K
+    from xyst_amd import riemann as X
+    c = _case(n)
+    U0 = smooth_state(c.coord)
+    U0[c.coord[0] < 0.4, 4] *= 3.0
+    U0 = np.column_stack([U0] + [1.0 + 0.3 * np.sin(3.0 * c.coord[1] + i) for i in range(ns)])
+    ctx = X.Context(0)
+    K.upload(ctx, c.coord, c.inpoel)
+    K.setup(ctx, c.vol, c.symnodes, c.symnorms, fct=fct, fctsys=(0, 4), ncomp=5 + ns)
+    U = torch.tensor(U0, device="cuda")
+    Un = torch.empty_like(U)
+    dt = K.dt_dev(ctx, U, 0.5)
+    K.step_dev(ctx, dt, U, Un)
+    Uo, _ = O.kozcg_step(O.cfg(), O.fctcfg(fct, 1.0, False, [0, 4]), c.coord, c.inpoel, c.vol,
+                         dt, c.symnodes, c.symnorms, np.zeros(0, np.int64),
+                         np.zeros((0, 5 + ns)), U0)
+    assert np.all(np.abs(U.cpu().numpy() - Uo) <= 1e-11 * np.abs(Uo).max(0))
+    assert np.array_equal(Un.cpu().numpy(), U0)
+    ctx.close()
+
+
 # gather to full blocks between 29 and 30
 @pytest.mark.parametrize("n", [17, 29, 30])
 def test_chorin(n):

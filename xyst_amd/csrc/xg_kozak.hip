@@ -54,6 +54,8 @@ struct KozakMesh {
   double* slots = nullptr;
   int nfx = 0;
   int *fx_node = nullptr, *fx_off = nullptr, *fx_slot = nullptr;
+  int* fx_all = nullptr;                 // per node: its first fx_slot (npoin + 1)
+  double* tj = nullptr;                  // per layout tet: J / 120
   double *sU = nullptr, *sR = nullptr;   // staging of the host-pointer entry
   double* sD = nullptr;                  // (XG_MAX_NCOMP and dtp per node)
   int nslot = 0;
@@ -96,18 +98,21 @@ struct PairPrefetch {
   int4 C = make_int4(0, 0, 0, 0);   // kind, first, count, tend_off
   uint32_t ab = 0, cd = 0;
   uint16_t e0 = 0, e1 = 0, te = 0;
+  double j120 = 0.0;                // J / 120 where tj is given
   __device__ inline void load(int ch, int chunk1, const int4* __restrict__ chk,
                               const int* __restrict__ chk_ent,
                               const uint16_t* __restrict__ tend,
                               const uint16_t* __restrict__ entries,
                               const uint32_t* __restrict__ tab,
-                              const uint32_t* __restrict__ tcd, int t, int nloc) {
+                              const uint32_t* __restrict__ tcd, int t, int nloc,
+                              const double* __restrict__ tj = nullptr) {
     if (ch >= chunk1) return;
     C = chk[ch];
     const int i = t >> 1;
     const int e = C.y + (i < C.z ? i : 0);
     ab = tab[e];
     cd = tcd[e];
+    if (tj) j120 = tj[e];
     const int off = chk_ent[ch], ne = 4 * C.z;
     e0 = t < ne ? entries[off + t] : 0;
     e1 = kKozThreads + t < ne ? entries[off + kKozThreads + t] : 0;
@@ -127,25 +132,38 @@ __device__ inline void cross(const double a[3], const double b[3], double c[3]) 
   c[2] = a[0] * b[1] - b[0] * a[1];
 }
 
-// The tet's Jacobian and the antidiffusive contributions of its corners
-// 2h and 2h + 1 (KozCG::aec, KozCG.cpp:794-812) for NC components, in the
-// reference's operation order and without fused multiply-adds: the limiter
-// branches on their signs, so they are bit-identical.
-template <int NC>
-__device__ inline void pair_aec(const double X[4][3], const double* sU, int cap,
-                                const int N[4], int h, double ctau, double out[2][NC]) {
+// J / 120 of every layout tet, in the reference's operation order and without
+// fused multiply-adds (KozCG.cpp:794-800): mesh data, formed once at upload
+__global__ __launch_bounds__(kBlock) void k_tet_j120(
+    int64_t ntet, const int* __restrict__ tet, const double* __restrict__ x,
+    const double* __restrict__ y, const double* __restrict__ z, double* __restrict__ tj) {
 #pragma clang fp contract(off)
+  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (e >= ntet) return;
+  const int* N = tet + 4 * e;
+  const double* P[3] = {x, y, z};
   double ba[3], ca[3], da[3], t[3];
   for (int j = 0; j < 3; ++j) {
-    ba[j] = X[1][j] - X[0][j];
-    ca[j] = X[2][j] - X[0][j];
-    da[j] = X[3][j] - X[0][j];
+    const double o = P[j][N[0]];
+    ba[j] = P[j][N[1]] - o;
+    ca[j] = P[j][N[2]] - o;
+    da[j] = P[j][N[3]] - o;
   }
   t[0] = ca[1] * da[2] - da[1] * ca[2];
   t[1] = ca[2] * da[0] - da[2] * ca[0];
   t[2] = ca[0] * da[1] - da[0] * ca[1];
   const double J = ba[0] * t[0] + ba[1] * t[1] + ba[2] * t[2];
-  const double j120 = J / 120.0;
+  tj[e] = J / 120.0;
+}
+
+// The antidiffusive contributions of a tet's corners 2h and 2h + 1
+// (KozCG::aec, KozCG.cpp:794-812) for NC components, j120 = J / 120, in the
+// reference's operation order and without fused multiply-adds: the limiter
+// branches on their signs, so they are bit-identical.
+template <int NC>
+__device__ inline void pair_aec(double j120, const double* sU, int cap, const int N[4], int h,
+                                double ctau, double out[2][NC]) {
+#pragma clang fp contract(off)
   const double mo = j120 * -1.0, md = j120 * 3.0;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
@@ -189,7 +207,7 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
     const double* __restrict__ y, const double* __restrict__ z,
     const double* __restrict__ U, double* __restrict__ R,
     double* __restrict__ S, double gm1, double dt, const double* __restrict__ dtp,
-    double ctau, xg::Prob P) {
+    double ctau, const double* __restrict__ tj, xg::Prob P) {
   constexpr int CAP = xg::kKozCap;
   constexpr int NS = xg::kKozPairSlots;
   constexpr int NO = AEC ? 3 * NC : NC;
@@ -220,16 +238,17 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
   }
   const int i = t >> 1, h = t & 1;
   PairPrefetch pf;
-  pf.load(B1.y, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc);
+  pf.load(B1.y, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc, AEC ? tj : nullptr);
   double acc[NO];
 #pragma unroll
   for (int c = 0; c < NO; ++c) acc[c] = 0.0;
   for (int ch = B1.y; ch < B1.z; ++ch) {
     const int4 C = pf.C;
     const uint32_t ab = pf.ab, cd = pf.cd;
+    const double j120 = pf.j120;
     __syncthreads();          // staging done / previous chunk's F consumed
     pf.store(t, nloc, sE, sT);
-    pf.load(ch + 1, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc);
+    pf.load(ch + 1, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc, AEC ? tj : nullptr);
     double aec[2][NC];
     {
       const int N[4] = {(int)(ab & 0xffff), (int)(ab >> 16), (int)(cd & 0xffff),
@@ -346,7 +365,7 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
           }
         }
       }
-      if constexpr (AEC) pair_aec<NC>(X, sU, CAP, N, h, ctau, aec);
+      if constexpr (AEC) pair_aec<NC>(j120, sU, CAP, N, h, ctau, aec);
     }
     __syncthreads();          // F, sE, sT complete
     if (t < nloc) {
@@ -433,7 +452,7 @@ __device__ inline int local_to_global(int t, int own0, int nown,
 // thread owning local node t merges the bounds of the chunk's tets that
 // touch it (its entry list) into its running max/min in registers -- max
 // and min are exact and independent of order, so the result is
-// deterministic.  Halo partials go to slots that k_fixup_minmax merges.
+// deterministic.  Halo partials go to slots that k_kozcg_coef merges.
 // Owners also store the low-order solution UL.  NC components; dtp
 // (nullable) the nodes' local time steps of a steady run.
 template <bool CLIP, int NC>
@@ -524,38 +543,17 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
   }
 }
 
-// merges halo bounds into their owners (max for Q+, min for Q-), NC
-// components
-template <int NC>
-__global__ __launch_bounds__(kBlock) void k_fixup_minmax(
-    int nfx, const int* __restrict__ fx_node, const int* __restrict__ fx_off,
-    const int* __restrict__ fx_slot, const double* __restrict__ S,
-    double* __restrict__ Q) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nfx) return;
-  double* q = Q + (size_t)fx_node[i] * (2 * NC);
-  double v[2 * NC];
-#pragma unroll
-  for (int c = 0; c < 2 * NC; ++c) v[c] = q[c];
-  for (int k = fx_off[i]; k < fx_off[i + 1]; ++k) {
-    const double* s = S + (size_t)fx_slot[k] * (2 * NC);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      v[c] = smax(v[c], s[c]);
-      v[NC + c] = smin(v[NC + c], s[NC + c]);
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < 2 * NC; ++c) q[c] = v[c];
-}
-
-// limit coefficients C+/- (KozCG.cpp:1005-1024), one thread per node and
-// component (neighbouring threads read neighbouring words)
+// Limit coefficients C+/- (KozCG.cpp:1005-1024) from the owners' bounds Q and
+// the halo bounds S of the node's slots (max for Q+, min for Q-), one thread
+// per node and component (neighbouring threads read neighbouring words).
+// Bound by memory: 320 bytes a node, 64 us on 96^3 (4.6 TB/s); 35 + 48 us
+// while a pass of its own merged the bounds first.
 template <int NC>
 __global__ __launch_bounds__(kBlock) void k_kozcg_coef(
     int npoin, const double* __restrict__ W, const double* __restrict__ vol,
     const double* __restrict__ UL, const double* __restrict__ Q,
-    double* __restrict__ Cf) {
+    const int* __restrict__ fx_all, const int* __restrict__ fx_slot,
+    const double* __restrict__ S, double* __restrict__ Cf) {
 #pragma clang fp contract(off)
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= (int64_t)npoin * NC) return;
@@ -565,7 +563,13 @@ __global__ __launch_bounds__(kBlock) void k_kozcg_coef(
   const double v = vol[g];
   const double pp = W[g * (3 * NC) + NC + c] / v, pn = W[g * (3 * NC) + 2 * NC + c] / v;
   const double ul = UL[k];
-  const double qp = Q[g * (2 * NC) + c] - ul, qn = Q[g * (2 * NC) + NC + c] - ul;
+  double hi = Q[g * (2 * NC) + c], lo = Q[g * (2 * NC) + NC + c];
+  for (int f = fx_all[g]; f < fx_all[g + 1]; ++f) {
+    const double* s = S + (size_t)fx_slot[f] * (2 * NC);
+    hi = smax(hi, s[c]);
+    lo = smin(lo, s[NC + c]);
+  }
+  const double qp = hi - ul, qn = lo - ul;
   Cf[g * (2 * NC) + c] = pp < eps ? 0.0 : smin(1.0, qp / pp);
   Cf[g * (2 * NC) + NC + c] = pn > -eps ? 0.0 : smin(1.0, qn / pn);
 }
@@ -576,22 +580,22 @@ __global__ __launch_bounds__(kBlock) void k_kozcg_coef(
 // their min; the corner adds coef * aec.  Pair layout as kozak::rhs: thread
 // t recomputes the antidiffusive contributions of its two corners, takes
 // the min over them and, with one lane exchange, over its partner's; the
-// corner slots are summed per node as in the rhs.  NC components.
+// corner slots are summed per node as in the rhs.  NC components.  J / 120
+// comes per tet (its coordinates in LDS and the products again took the
+// kernel from 231 to 249 us on 96^3, with the coefficients in 8-byte loads).
 template <int NC>
 __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_kozcg_lim(
     int nblk, const int4* __restrict__ blk0, const int4* __restrict__ blk1,
     const int* __restrict__ halo, const int4* __restrict__ chk,
     const int* __restrict__ chk_ent, const uint16_t* __restrict__ tend,
     const uint16_t* __restrict__ entries, const uint32_t* __restrict__ tab,
-    const uint32_t* __restrict__ tcd, const double* __restrict__ x,
-    const double* __restrict__ y, const double* __restrict__ z,
+    const uint32_t* __restrict__ tcd, const double* __restrict__ tj,
     const double* __restrict__ U, const double* __restrict__ Cf,
     double* __restrict__ A, double* __restrict__ S, double ctau, int sysmask) {
   constexpr int CAP = xg::kKozCap;
   constexpr int NS = xg::kKozPairSlots;
   constexpr int NB = 2 * NC;
   __shared__ double sU[NC * CAP];
-  __shared__ double sX[3 * CAP];
   __shared__ double F[NS * NC];
   __shared__ int sG[CAP];
   __shared__ uint16_t sE[NS];
@@ -606,16 +610,13 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
     sG[t] = g;
 #pragma unroll
     for (int c = 0; c < NC; ++c) sU[c * CAP + t] = U[(size_t)g * NC + c];
-    sX[0 * CAP + t] = x[g];
-    sX[1 * CAP + t] = y[g];
-    sX[2 * CAP + t] = z[g];
   }
   const int i = t >> 1, h = t & 1;
   double acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0.0;
   PairPrefetch pf;
-  pf.load(B1.y, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc);
+  pf.load(B1.y, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc, tj);
   __syncthreads();            // staging done
   // the two corner nodes' limit coefficients C+ (NC) and C- (NC): the next
   // chunk's are loaded as soon as the current chunk's coefficients are
@@ -626,28 +627,29 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int na = k ? (int)(w >> 16) : (int)(w & 0xffff);
-      const double* cf = Cf + (size_t)sG[na] * NB;
+      // 16-byte loads: a node's record is 16 NC bytes of a 256-byte aligned array
+      const double2* cf = reinterpret_cast<const double2*>(Cf) + (size_t)sG[na] * NC;
 #pragma unroll
-      for (int c = 0; c < NB; ++c) cfn[k][c] = cf[c];
+      for (int c = 0; c < NC; ++c) {
+        const double2 v = cf[c];
+        cfn[k][2 * c] = v.x;
+        cfn[k][2 * c + 1] = v.y;
+      }
     }
   };
   if (B1.y < B1.z) fetch_cf(pf);
   for (int ch = B1.y; ch < B1.z; ++ch) {
     const int4 C = pf.C;
     const uint32_t ab = pf.ab, cd = pf.cd;
+    const double j120 = pf.j120;
     __syncthreads();          // previous chunk's F consumed
     pf.store(t, nloc, sE, sT);
-    pf.load(ch + 1, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc);
+    pf.load(ch + 1, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc, tj);
     {
       const int N[4] = {(int)(ab & 0xffff), (int)(ab >> 16), (int)(cd & 0xffff),
                         (int)(cd >> 16)};
-      double X[4][3];
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) X[k][j] = sX[j * CAP + N[k]];
       double aec[2][NC], coef[NC];
-      pair_aec<NC>(X, sU, CAP, N, h, ctau, aec);
+      pair_aec<NC>(j120, sU, CAP, N, h, ctau, aec);
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         const double qa = aec[0][c] > 0.0 ? cfn[0][c] : cfn[0][NC + c];
@@ -696,24 +698,52 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
   }
 }
 
-// new solution (KozCG.cpp:1144-1160), nc components per node; Un receives
-// the old one.  dtp (nullable): the nodes' local time steps without FCT.
-template <bool FCT>
+// new solution (KozCG.cpp:1144-1160), NC components per node; Un receives
+// the old one.  A: the owners' limited contributions (without FCT the rhs),
+// S the halo partials of the node's slots, added in block order.  Bound by
+// memory: 200 bytes a node, 51 us on 96^3 (19 + 30 us and a launch with a
+// fix-up pass of its own).  dtp (nullable): the nodes' local time steps
+// without FCT.
+template <bool FCT, int NC>
 __global__ __launch_bounds__(kBlock) void k_kozcg_solve(
-    int npoin, int nc, double dt, const double* __restrict__ dtp,
-    const double* __restrict__ UL, const double* __restrict__ A,
-    const double* __restrict__ R, const double* __restrict__ vol,
-    double* __restrict__ U, double* __restrict__ Un) {
+    int npoin, double dt, const double* __restrict__ dtp, const double* __restrict__ UL,
+    const double* __restrict__ A, const int* __restrict__ fx_all,
+    const int* __restrict__ fx_slot, const double* __restrict__ S,
+    const double* __restrict__ vol, double* __restrict__ U, double* __restrict__ Un) {
 #pragma clang fp contract(off)
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (int64_t)npoin * nc) return;
-  const int64_t g = k / nc;
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= (int64_t)npoin * NC) return;
+  const int64_t g = k / NC;
+  const int c = (int)(k - g * NC);
+  double a = A[k];
+  for (int f = fx_all[g]; f < fx_all[g + 1]; ++f) a += S[(size_t)fx_slot[f] * NC + c];
   const double u = U[k];
   Un[k] = u;
   if (FCT)
-    U[k] = UL[k] + A[k] / vol[g];
+    U[k] = UL[k] + a / vol[g];
   else
-    U[k] = u + (dtp ? dtp[g] : dt) * R[k] / vol[g];
+    U[k] = u + (dtp ? dtp[g] : dt) * a / vol[g];
+}
+
+// symmetry BCs on P+ and P- (KozCG.cpp:816-830; k_symbc on the 3-vectors at
+// component 1 of either): two threads per node
+template <int NC>
+__global__ __launch_bounds__(kBlock) void k_symbc_p(int ns, const int* __restrict__ node,
+                                                   const int* __restrict__ off,
+                                                   const double* __restrict__ nrm,
+                                                   double* __restrict__ W) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, i = k >> 1;
+  if (i >= ns) return;
+  double* u = W + (size_t)node[i] * (3 * NC) + (k & 1 ? 2 * NC + 1 : NC + 1);
+  double a = u[0], b = u[1], c = u[2];
+  for (int f = off[i]; f < off[i + 1]; ++f) {
+    const double* n = nrm + (size_t)f * 3;
+    const double vn = a * n[0] + b * n[1] + c * n[2];
+    a -= vn * n[0];
+    b -= vn * n[1];
+    c -= vn * n[2];
+  }
+  u[0] = a; u[1] = b; u[2] = c;
 }
 
 // Dirichlet BCs (physics::dirbc, BC.cpp:30-69): masked components of the
@@ -764,7 +794,7 @@ void launch_kozak_pairs(xg_ctx* c, const double* U, double* out, double* slots,
   hipLaunchKernelGGL(kern, dim3(k->nblk), dim3(kKozThreads), 0, c->stream, k->nblk,
                      k->blk0, k->blk1, k->halo, k->chk, k->chk_ent, k->tend, k->entries,
                      k->tab, k->tcd, k->x, k->y, k->z, U, out, slots,
-                     c->cfg.gamma - 1.0, dt, dtp, ctau, P);
+                     c->cfg.gamma - 1.0, dt, dtp, ctau, k->tj, P);
 }
 
 template <int NC>
@@ -810,12 +840,9 @@ void kozcg_step_nc(xg_ctx* c, double dt, const double* dtp, double* tp, int free
   const auto& f = k->fct;
   if (!f.fct) {
     if (k->nblk) launch_kozak_pairs<false, NC>(c, U, k->W, k->S15, dt, dtp, 0.0);
-    if (k->nfx)
-      hipLaunchKernelGGL(k_fixup<NC>, dim3(nblocks(k->nfx)), dim3(kBlock), 0,
-                         c->stream, k->nfx, k->fx_node, k->fx_off, k->fx_slot,
-                         k->S15, k->W);
-    hipLaunchKernelGGL(k_kozcg_solve<false>, dim3(nblocks(nn)), dim3(kBlock), 0,
-                       c->stream, n, NC, dt, dtp, nullptr, nullptr, k->W, k->vol, U, Un);
+    hipLaunchKernelGGL((k_kozcg_solve<false, NC>), dim3(nblocks(nn)), dim3(kBlock), 0,
+                       c->stream, n, dt, dtp, nullptr, k->W, k->fx_all, k->fx_slot, k->S15,
+                       k->vol, U, Un);
   } else {
     int sysmask = 0;
     for (int s = 0; s < f.nsys; ++s) sysmask |= 1 << f.sys[s];
@@ -826,14 +853,9 @@ void kozcg_step_nc(xg_ctx* c, double dt, const double* dtp, double* tp, int free
                          c->stream, k->nfx, k->fx_node, k->fx_off, k->fx_slot,
                          k->S15, k->W);
     // symmetry BCs on the antidiffusive contributions (KozCG.cpp:816-830)
-    if (k->nsymnode) {
-      hipLaunchKernelGGL(k_symbc, dim3(nblocks(k->nsymnode)), dim3(kBlock), 0,
-                         c->stream, k->nsymnode, k->symnode, k->symoff,
-                         k->symnorm, k->W, 3 * NC, NC + 1);
-      hipLaunchKernelGGL(k_symbc, dim3(nblocks(k->nsymnode)), dim3(kBlock), 0,
-                         c->stream, k->nsymnode, k->symnode, k->symoff,
-                         k->symnorm, k->W, 3 * NC, 2 * NC + 1);
-    }
+    if (k->nsymnode)
+      hipLaunchKernelGGL(k_symbc_p<NC>, dim3(nblocks(2 * (int64_t)k->nsymnode)), dim3(kBlock),
+                         0, c->stream, k->nsymnode, k->symnode, k->symoff, k->symnorm, k->W);
     // low-order solution and allowed bounds (KozCG::alw)
     if (k->nblk) {
       auto alw = f.fctclip ? k_kozcg_alw<true, NC> : k_kozcg_alw<false, NC>;
@@ -842,26 +864,19 @@ void kozcg_step_nc(xg_ctx* c, double dt, const double* dtp, double* tp, int free
                          k->entries, k->tab, k->tcd, k->W, U, k->vol, dt, dtp, k->UL,
                          k->Q, k->S15);
     }
-    if (k->nfx)
-      hipLaunchKernelGGL(k_fixup_minmax<NC>, dim3(nblocks(k->nfx)), dim3(kBlock), 0,
-                         c->stream, k->nfx, k->fx_node, k->fx_off, k->fx_slot,
-                         k->S15, k->Q);
     // limit coefficients and limited contributions (KozCG::lim)
     hipLaunchKernelGGL(k_kozcg_coef<NC>, dim3(nblocks(nn)), dim3(kBlock), 0,
-                       c->stream, n, k->W, k->vol, k->UL, k->Q, k->C);
+                       c->stream, n, k->W, k->vol, k->UL, k->Q, k->fx_all, k->fx_slot, k->S15,
+                       k->C);
     if (k->nblk)
       hipLaunchKernelGGL(k_kozcg_lim<NC>, dim3(k->nblk), dim3(kKozThreads), 0,
                          c->stream, k->nblk, k->blk0, k->blk1, k->halo, k->chk,
-                         k->chk_ent, k->tend, k->entries, k->tab, k->tcd, k->x,
-                         k->y, k->z, U, k->C, k->A, k->S15, f.fctdif, sysmask);
-    if (k->nfx)
-      hipLaunchKernelGGL(k_fixup<NC>, dim3(nblocks(k->nfx)), dim3(kBlock), 0,
-                         c->stream, k->nfx, k->fx_node, k->fx_off, k->fx_slot,
-                         k->S15, k->A);
+                         k->chk_ent, k->tend, k->entries, k->tab, k->tcd, k->tj, U, k->C, k->A,
+                         k->S15, f.fctdif, sysmask);
     // new solution (KozCG::solve)
-    hipLaunchKernelGGL(k_kozcg_solve<true>, dim3(nblocks(nn)), dim3(kBlock), 0,
-                       c->stream, n, NC, dt, nullptr, k->UL, k->A, nullptr, k->vol, U,
-                       Un);
+    hipLaunchKernelGGL((k_kozcg_solve<true, NC>), dim3(nblocks(nn)), dim3(kBlock), 0,
+                       c->stream, n, dt, nullptr, k->UL, k->A, k->fx_all, k->fx_slot, k->S15,
+                       k->vol, U, Un);
   }
   // KozCG::BC: Dirichlet, then symmetry
   if (k->ndir)
@@ -918,6 +933,10 @@ int xg_kozak_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
     ch[i] = make_int4(C.kind, C.first, C.count, C.tend_off);
     ce[i] = C.ent_off;
   }
+  std::vector<int> fxa((size_t)npoin + 1, 0);
+  for (size_t i = 0; i < L.fx_node.size(); ++i)
+    fxa[L.fx_node[i] + 1] = L.fx_off[i + 1] - L.fx_off[i];
+  for (int64_t i = 0; i < npoin; ++i) fxa[i + 1] += fxa[i];
   auto& A = k->allocs;
   const size_t n = (size_t)npoin;
   if ((rc = upload(c, A, &k->x, x, n)) || (rc = upload(c, A, &k->y, y, n)) ||
@@ -931,9 +950,27 @@ int xg_kozak_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
                       (size_t)L.nslot * XG_MAX_NCOMP * sizeof(double))) ||
       (rc = upload(c, A, &k->fx_node, L.fx_node)) ||
       (rc = upload(c, A, &k->fx_off, L.fx_off)) ||
-      (rc = upload(c, A, &k->fx_slot, L.fx_slot))) {
+      (rc = upload(c, A, &k->fx_slot, L.fx_slot)) || (rc = upload(c, A, &k->fx_all, fxa)) ||
+      (rc = dev_alloc(c, A, (void**)&k->tj, L.tab.size() * sizeof(double)))) {
     free_kozak(k);
     return rc;
+  }
+  if (!L.tglob.empty()) {
+    std::vector<DevArr> tmp;
+    int* tg = nullptr;
+    rc = upload(c, tmp, &tg, L.tglob);
+    const int64_t nt = (int64_t)L.tab.size();
+    if (!rc) {
+      hipLaunchKernelGGL(k_tet_j120, dim3(nblocks(nt)), dim3(kBlock), 0, c->stream, nt, tg, k->x,
+                         k->y, k->z, k->tj);
+      if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
+        rc = fail(c, XG_EHIP, "xg_kozak_upload: tet Jacobians");
+    }
+    dev_free_all(tmp);
+    if (rc) {
+      free_kozak(k);
+      return rc;
+    }
   }
   k->nfx = (int)L.fx_node.size();
   k->nslot = L.nslot;

@@ -79,7 +79,7 @@ constexpr int kTetsPerPairChunk = kKozPairSlots / 4;
 struct TetLayout {
   int npoin = 0;
   std::vector<uint32_t> tab, tcd;  // tets in block/chunk order: local a|b<<16, c|d<<16
-  std::vector<int> tglob;          // their global nodes (4 per tet, checks)
+  std::vector<int> tglob;          // their global nodes (4 per tet)
   std::vector<Block> blk;
   std::vector<Chunk> chunks;       // kind 2
   std::vector<int> halo;
