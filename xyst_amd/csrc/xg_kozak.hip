@@ -9,7 +9,8 @@
 // lists loaded while the current one computes.  Thread t handles corners 2h
 // and 2h + 1 (h = t % 2) of chunk tet t / 2; the two threads of a tet are
 // neighbouring lanes and combine their partial values with one DPP lane
-// exchange.
+// exchange; what a thread needs of the tet's other two corners it takes from
+// its partner, too, rather than from LDS again.
 //  * kozak::rhs (k_kozak_pairs): each thread evaluates the tet geometry and
 //    two corners' shares of the half-step state, the exchange completes the
 //    state, and the thread writes its two corners' second-step fluxes; in
@@ -132,6 +133,16 @@ __device__ inline void cross(const double a[3], const double b[3], double c[3]) 
   c[2] = a[0] * b[1] - b[0] * a[1];
 }
 
+// the value that the pair's lane H (0 or 1) holds: lanes 2 i and 2 i + 1 are a
+// tet's two halves
+template <int H>
+__device__ inline double quad_of(double v) {
+  constexpr int ctrl = H ? 0xf5 : 0xa0;   // quad_perm [1,1,3,3] : [0,0,2,2]
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
 // J / 120 of every layout tet, in the reference's operation order and without
 // fused multiply-adds (KozCG.cpp:794-800): mesh data, formed once at upload
 __global__ __launch_bounds__(kBlock) void k_tet_j120(
@@ -161,15 +172,14 @@ __global__ __launch_bounds__(kBlock) void k_tet_j120(
 // reference's operation order and without fused multiply-adds: the limiter
 // branches on their signs, so they are bit-identical.
 template <int NC>
-__device__ inline void pair_aec(double j120, const double* sU, int cap, const int N[4], int h,
+__device__ inline void pair_aec(double j120, const double* sU, int cap, int nA, int nB, int h,
                                 double ctau, double out[2][NC]) {
 #pragma clang fp contract(off)
   const double mo = j120 * -1.0, md = j120 * 3.0;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    double u[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) u[b] = sU[c * cap + N[b]];
+    const double o0 = sU[c * cap + nA], o1 = sU[c * cap + nB];
+    const double u[4] = {quad_of<0>(o0), quad_of<0>(o1), quad_of<1>(o0), quad_of<1>(o1)};
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int a = 2 * h + k;
@@ -189,7 +199,10 @@ __device__ inline void pair_aec(double j120, const double* sU, int cap, const in
 // writes its two corners' second-step fluxes into the chunk's corner slots
 // (4 i + a).  The thread owning local node t then adds the chunk's slots of
 // its node, in slot order; halo partials go to slots that k_fixup adds to
-// their owners.
+// their owners.  Bound by FP64 issue and LDS together (both two thirds busy,
+// four waves a SIMD): a corner's three flux directions are contracted with
+// its gradient before they multiply the components, and the corners' data is
+// read once per pair: 96^3 184 -> 167 us (5.3 M tets), with AEC 336 -> 303.
 // SRC: the problem's source term (Kozak.cpp:124-136, 163-173).
 // AEC: also the antidiffusive contributions of KozCG::aec, written into the
 // same corner slots after the fluxes are summed and summed per node by sign
@@ -251,13 +264,18 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
     pf.load(ch + 1, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc, AEC ? tj : nullptr);
     double aec[2][NC];
     {
-      const int N[4] = {(int)(ab & 0xffff), (int)(ab >> 16), (int)(cd & 0xffff),
-                        (int)(cd >> 16)};
+      // this thread's corners: (0, 1) or (2, 3); the others' from its partner
+      const uint32_t w = h ? cd : ab;
+      const int nA = (int)(w & 0xffff), nB = (int)(w >> 16);
       double X[4][3];
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) X[k][j] = sX[j * CAP + N[k]];
+      for (int j = 0; j < 3; ++j) {
+        const double xa = sX[j * CAP + nA], xb = sX[j * CAP + nB];
+        X[0][j] = quad_of<0>(xa);
+        X[1][j] = quad_of<0>(xb);
+        X[2][j] = quad_of<1>(xa);
+        X[3][j] = quad_of<1>(xb);
+      }
       double ba[3], ca[3], da[3];
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
@@ -270,17 +288,18 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
       cross(da, ba, g2);
       cross(ba, ca, g3);
       const double J = ba[0] * g1[0] + ba[1] * g1[1] + ba[2] * g1[2];
-      // this thread's corners: (0, 1) or (2, 3)
       double gA[3], gB[3];
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         gA[j] = h ? g2[j] : -g1[j] - g2[j] - g3[j];
         gB[j] = h ? g3[j] : g1[j];
       }
-      const int nA = h ? N[2] : N[0], nB = h ? N[3] : N[1];
       // steady: the mean of the corners' local time steps
-      const double dte =
-          dtp ? (((sD[N[0]] + sD[N[1]]) + sD[N[2]]) + sD[N[3]]) / 4.0 : dt;
+      double dte = dt;
+      if (dtp) {
+        const double da_ = sD[nA], db_ = sD[nB];
+        dte = (((quad_of<0>(da_) + quad_of<0>(db_)) + quad_of<1>(da_)) + quad_of<1>(db_)) / 4.0;
+      }
       const double coef = dte * xg::rcp(J) * 0.5;
       // the two corners' shares of the half-step state (Kozak.cpp:92-124)
       double hs[NC];
@@ -295,22 +314,20 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
         for (int c = 0; c < NC; ++c) u[c] = sU[c * CAP + na];
         const double ir = xg::rcp(u[0]);
         const double p = (u[4] - 0.5 * (u[1] * u[1] + u[2] * u[2] + u[3] * u[3]) * ir) * gm1;
+        // sum over j of g_j times the flux in direction j: the mass flux m
+        // carries every component, p adds to the momentum and the energy
+        double cg[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) cg[j] = coef * ga[j];
+        const double m = cg[0] * u[1] + cg[1] * u[2] + cg[2] * u[3];
+        const double v = m * ir;
         double hh[NC];
+        hh[0] = 0.25 * u[0] - m;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) hh[c] = 0.25 * u[c];
+        for (int j = 0; j < 3; ++j) hh[j + 1] = 0.25 * u[j + 1] - u[j + 1] * v - cg[j] * p;
+        hh[4] = 0.25 * u[4] - (u[4] + p) * v;
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const double cg = coef * ga[j];
-          const double uj = u[j + 1] * ir;
-          hh[0] -= cg * u[j + 1];
-          hh[1] -= cg * u[1] * uj;
-          hh[2] -= cg * u[2] * uj;
-          hh[3] -= cg * u[3] * uj;
-          hh[j + 1] -= cg * p;
-          hh[4] -= cg * (u[4] + p) * uj;
-#pragma unroll
-          for (int c = 5; c < NC; ++c) hh[c] -= cg * u[c] * uj;
-        }
+        for (int c = 5; c < NC; ++c) hh[c] = 0.25 * u[c] - u[c] * v;
         if constexpr (SRC) {
           double sa[5];
           xg::source(P, sX[0 * CAP + na], sX[1 * CAP + na], sX[2 * CAP + na], sa);
@@ -328,19 +345,6 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
       // second half step (Kozak.cpp:138-161): the two corners' fluxes
       const double ie = xg::rcp(ue[0]);
       const double pr = (ue[4] - 0.5 * (ue[1] * ue[1] + ue[2] * ue[2] + ue[3] * ue[3]) * ie) * gm1;
-      double fl[3][NC];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double uj = ue[j + 1] * ie;
-        fl[j][0] = ue[j + 1];
-        fl[j][1] = ue[1] * uj;
-        fl[j][2] = ue[2] * uj;
-        fl[j][3] = ue[3] * uj;
-        fl[j][j + 1] += pr;
-        fl[j][4] = (ue[4] + pr) * uj;
-#pragma unroll
-        for (int c = 5; c < NC; ++c) fl[j][c] = ue[c] * uj;
-      }
       double se[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
       double cj = 0.0;
       if constexpr (SRC) {
@@ -354,18 +358,26 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
         for (int k = 0; k < 2; ++k) {
           const double* ga = k ? gB : gA;
           const int slot = 4 * i + 2 * h + k;
+          const double g[3] = {ga[0] * (1.0 / 6.0), ga[1] * (1.0 / 6.0), ga[2] * (1.0 / 6.0)};
+          const double m = g[0] * ue[1] + g[1] * ue[2] + g[2] * ue[3];
+          const double v = m * ie;
+          double f[NC];
+          f[0] = m;
+#pragma unroll
+          for (int j = 0; j < 3; ++j) f[j + 1] = ue[j + 1] * v + g[j] * pr;
+          f[4] = (ue[4] + pr) * v;
+#pragma unroll
+          for (int c = 5; c < NC; ++c) f[c] = ue[c] * v;
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
-            double f = (ga[0] * (1.0 / 6.0)) * fl[0][c] + (ga[1] * (1.0 / 6.0)) * fl[1][c] +
-                       (ga[2] * (1.0 / 6.0)) * fl[2][c];
             if constexpr (SRC) {
-              if (c < 5) f += cj * se[c];
+              if (c < 5) f[c] += cj * se[c];
             }
-            F[slot * NC + c] = f;
+            F[slot * NC + c] = f[c];
           }
         }
       }
-      if constexpr (AEC) pair_aec<NC>(j120, sU, CAP, N, h, ctau, aec);
+      if constexpr (AEC) pair_aec<NC>(j120, sU, CAP, nA, nB, h, ctau, aec);
     }
     __syncthreads();          // F, sE, sT complete
     if (t < nloc) {
@@ -640,16 +652,14 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
   if (B1.y < B1.z) fetch_cf(pf);
   for (int ch = B1.y; ch < B1.z; ++ch) {
     const int4 C = pf.C;
-    const uint32_t ab = pf.ab, cd = pf.cd;
+    const uint32_t w = h ? pf.cd : pf.ab;
     const double j120 = pf.j120;
     __syncthreads();          // previous chunk's F consumed
     pf.store(t, nloc, sE, sT);
     pf.load(ch + 1, B1.z, chk, chk_ent, tend, entries, tab, tcd, t, nloc, tj);
     {
-      const int N[4] = {(int)(ab & 0xffff), (int)(ab >> 16), (int)(cd & 0xffff),
-                        (int)(cd >> 16)};
       double aec[2][NC], coef[NC];
-      pair_aec<NC>(j120, sU, CAP, N, h, ctau, aec);
+      pair_aec<NC>(j120, sU, CAP, (int)(w & 0xffff), (int)(w >> 16), h, ctau, aec);
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         const double qa = aec[0][c] > 0.0 ? cfn[0][c] : cfn[0][NC + c];
