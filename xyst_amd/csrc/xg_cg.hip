@@ -322,8 +322,8 @@ struct FcgRow {
 // kernel of this iteration and all later launches of the batch read.
 // An iteration (this and k_cg_update) moves 12 nnz + 44 n bytes of matrix
 // and pairs and 76 n of vectors in FP64: 15 us at 64^3 (274,625 rows) at the
-// copy rate, 27.8 us measured (37 before the loads were put ahead of the
-// scalars); 65 us at 100^3, 81 before.
+// copy rate, 26 us measured (37 before the loads were put ahead of the
+// scalars, 28 before the column lists); 62 us at 100^3, 81 before.
 template <class T>
 __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_cg_spmv(
     int j, xg::TileMat M, const T* __restrict__ a, const T* __restrict__ zp,

@@ -113,11 +113,13 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
 // nodes fills a few of the 256 CUs, and each block walks its chunks alone: so
 // they are cut into about as many blocks as run at once, and where that is
 // the faster, into gather blocks, which need no halo fix-up.  Times of the
-// full blocks and of these, in us:
+// full blocks and of these when the lines were drawn (chunks not yet spread,
+// the tet kernels' arithmetic heavier), in us:
 //  riemann::grad: sixteen nodes, four lanes each (its waves are independent);
-//  riemann::rhs (two workgroups per CU: at most 512 blocks): 12^3 20.6 -> 6.9, 24^3 21.1 -> 9.9, 29^3 (27,000
-//    nodes) 23.7 -> 14.5, with 6 components (one workgroup per CU) 23.9 ->
-//    20.5; on 31^3 (32,768) 22.4 -> 20.4, but 22.7 -> 27.9 with 6;
+//  riemann::rhs (two workgroups per CU: at most 512 blocks): 12^3 20.6 ->
+//    6.9, 24^3 21.1 -> 9.9, 29^3 (27,000 nodes) 23.7 -> 14.5, with 6
+//    components (one workgroup per CU) 23.9 -> 20.5; on 31^3 (32,768) 22.4 ->
+//    20.4, but 22.7 -> 27.9 with 6;
 //  the tet operators, KozCG step: 12^3 201 -> 84, 20^3 (9,261) 201 -> 104, as
 //    scatter blocks 117; 24^3 (15,625) 203 -> 140 and 125 as scatter blocks,
 //    36^3 216 -> 178, 39^3 (64,000) 216 -> 197, 42^3 equal;
