@@ -117,11 +117,15 @@ static void group_entries(const std::vector<std::pair<int, uint16_t>>& ent, int 
   for (const auto& e : ent) entries[e0 + pos[e.first]++] = e.second;
 }
 
-// Cuts a block's items (edges or tets, in local order) into chunks of at most
-// `slots`, spreading the items of a node over the chunks: a chunk's node sums
-// take as long as the node with the most entries in it.  In local order alone
-// a node's items fall into one or two chunks (kozak::rhs on 96^3 240 us, 183
-// spread; the KozCG step 1253 -> 1013; riemann::rhs on 128^3 470 -> 445).
+// Cuts a block's tets (in local order) into chunks of at most `slots`,
+// spreading the tets of a node over the chunks: a chunk's node sums take as
+// long as the node with the most entries in it.  In local order alone a
+// node's tets fall into one or two chunks (kozak::rhs on 96^3 240 us, 183
+// spread; the KozCG step 1253 -> 1013; its rounding error 7.3e-16 -> 6.9e-16).
+// Edges stay in local order: spread, riemann::rhs on 128^3 took 444 us
+// instead of 470 and chorin::rhs on 64^3 59.7 instead of 62.5, but neighbours
+// that nearly cancel were added apart, and the error against the exact sums
+// grew from 6.9e-16 to 7.5e-16 and from 4.2e-15 to 5.7e-15.
 // Greedy, in item order: the chunk where the item's nodes have the fewest
 // entries so far, then the emptiest.  ends(i, out): the local nodes that item
 // i adds to; returns how many.  The items of a chunk keep their order.
@@ -255,8 +259,7 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     if (!gather) nslot += (int)halo.size();
     for (int i = 0; i < B.nown; ++i) local[B.own0 + i] = i;
     for (size_t h = 0; h < halo.size(); ++h) local[halo[h]] = B.nown + (int)h;
-    // edges ordered by (smaller local end, larger local end) for locality,
-    // then spread over the chunks
+    // edges ordered by (smaller local end, larger local end) for locality
     auto& E = bedges[b];
     std::sort(E.begin(), E.end(), [&](int64_t a, int64_t c) {
       int a0 = std::min(local[p[a]], local[q[a]]), a1 = std::max(local[p[a]], local[q[a]]);
@@ -277,24 +280,20 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
       group_entries(ent, B.nloc, L.entries, L.tend);
       L.chunks.push_back(C);
     };
-    const auto parts = spread_chunks(E, chunk_slots, B.nloc, [&](int64_t e, int* node) {
-      int k = 0;
-      for (int m : {local[p[e]], local[q[e]]})
-        if (!gather || m < B.nown) node[k++] = m;
-      return k;
-    });
-    for (const auto& C : parts) {
+    for (size_t i0 = 0; i0 < E.size(); i0 += (size_t)chunk_slots) {
+      const size_t i1 = std::min(E.size(), i0 + (size_t)chunk_slots);
       std::vector<std::pair<int, uint16_t>> ent;
-      for (size_t i = 0; i < C.size(); ++i) {
-        int64_t e = C[i];
-        uint16_t slot = (uint16_t)i;
+      for (size_t i = i0; i < i1; ++i) {
+        int64_t e = E[i];
+        uint16_t slot = (uint16_t)(i - i0);
         // R(p) -= f, R(q) += f (gather: owned ends only)
         if (!gather || local[p[e]] < B.nown)
           ent.emplace_back(local[p[e]], (uint16_t)(slot | 0x8000));
         if (!gather || local[q[e]] < B.nown) ent.emplace_back(local[q[e]], slot);
       }
-      emit(0, (int64_t)L.elpq.size(), (int)C.size(), ent);
-      for (int64_t e : C) {
+      emit(0, (int64_t)L.elpq.size(), (int)(i1 - i0), ent);
+      for (size_t i = i0; i < i1; ++i) {
+        const int64_t e = E[i];
         L.elpq.push_back((uint32_t)local[p[e]] | ((uint32_t)local[q[e]] << 16));
         L.ep.push_back(p[e]);
         L.eq.push_back(q[e]);

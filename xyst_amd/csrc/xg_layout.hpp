@@ -113,8 +113,8 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
 // nodes fills a few of the 256 CUs, and each block walks its chunks alone: so
 // they are cut into about as many blocks as run at once, and where that is
 // the faster, into gather blocks, which need no halo fix-up.  Times of the
-// full blocks and of these when the lines were drawn (chunks not yet spread,
-// the tet kernels' arithmetic heavier), in us:
+// full blocks and of these when the lines were drawn (the tets not yet spread
+// over the chunks, their kernels' arithmetic heavier), in us:
 //  riemann::grad: sixteen nodes, four lanes each (its waves are independent);
 //  riemann::rhs (two workgroups per CU: at most 512 blocks): 12^3 20.6 ->
 //    6.9, 24^3 21.1 -> 9.9, 29^3 (27,000 nodes) 23.7 -> 14.5, with 6
