@@ -849,7 +849,7 @@ int xg_chocg_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
   xg::Layout L;
   const xg::BlockPlan plan = xg::cho_blocks(npoin);
   int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), nosym.data(), plan.nodes,
-                            xg::kBlockCap, xg::kChunkSlots, L, c->err, plan.gather, true);
+                            xg::kBlockCap, xg::kChunkSlots, L, c->err, plan.gather, true, false);
   if (rc) return rc;
   std::vector<double> dwl(L.eidx.size());
   for (size_t e = 0; e < L.eidx.size(); ++e) dwl[e] = w[L.eidx[e]];

@@ -117,15 +117,15 @@ static void group_entries(const std::vector<std::pair<int, uint16_t>>& ent, int 
   for (const auto& e : ent) entries[e0 + pos[e.first]++] = e.second;
 }
 
-// Cuts a block's tets (in local order) into chunks of at most `slots`,
-// spreading the tets of a node over the chunks: a chunk's node sums take as
-// long as the node with the most entries in it.  In local order alone a
-// node's tets fall into one or two chunks (kozak::rhs on 96^3 240 us, 183
-// spread; the KozCG step 1253 -> 1013; its rounding error 7.3e-16 -> 6.9e-16).
-// Edges stay in local order: spread, riemann::rhs on 128^3 took 444 us
-// instead of 470 and chorin::rhs on 64^3 59.7 instead of 62.5, but neighbours
-// that nearly cancel were added apart, and the error against the exact sums
-// grew from 6.9e-16 to 7.5e-16 and from 4.2e-15 to 5.7e-15.
+// Cuts a block's items (edges or tets, in local order) into chunks of at most
+// `slots`, spreading the items of a node over the chunks: a chunk's node sums
+// take as long as the node with the most entries in it.  In local order alone
+// a node's items fall into one or two chunks (kozak::rhs on 96^3 240 us, 183
+// spread; the KozCG step 1253 -> 1013; riemann::rhs on 128^3 470 -> 444).  The
+// chorin operators keep local order (spread = false): chorin::rhs on 64^3 took
+// 59.7 us spread instead of 62.6, but neighbours that nearly cancel were added
+// apart, and the error against exact sums grew from 4.2e-15 to 5.7e-15 (the
+// others' did not).
 // Greedy, in item order: the chunk where the item's nodes have the fewest
 // entries so far, then the emptiest.  ends(i, out): the local nodes that item
 // i adds to; returns how many.  The items of a chunk keep their order.
@@ -172,7 +172,7 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
                  const std::vector<double>& d, int64_t ntri, const int* tri,
                  const uint8_t* besym, int block_nodes, int block_cap,
                  int chunk_slots, Layout& L, std::string& err, bool gather,
-                 bool gather_faces) {
+                 bool gather_faces, bool spread) {
   const int64_t ne = (int64_t)p.size();
   L = Layout();
   if (chunk_slots < 3 || chunk_slots > kChunkSlots) {
@@ -280,20 +280,30 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
       group_entries(ent, B.nloc, L.entries, L.tend);
       L.chunks.push_back(C);
     };
-    for (size_t i0 = 0; i0 < E.size(); i0 += (size_t)chunk_slots) {
-      const size_t i1 = std::min(E.size(), i0 + (size_t)chunk_slots);
+    std::vector<std::vector<int64_t>> parts;
+    if (spread)
+      parts = spread_chunks(E, chunk_slots, B.nloc, [&](int64_t e, int* node) {
+        int k = 0;
+        for (int m : {local[p[e]], local[q[e]]})
+          if (!gather || m < B.nown) node[k++] = m;
+        return k;
+      });
+    else
+      for (size_t i0 = 0; i0 < E.size(); i0 += (size_t)chunk_slots)
+        parts.emplace_back(E.begin() + i0,
+                           E.begin() + std::min(E.size(), i0 + (size_t)chunk_slots));
+    for (const auto& C : parts) {
       std::vector<std::pair<int, uint16_t>> ent;
-      for (size_t i = i0; i < i1; ++i) {
-        int64_t e = E[i];
-        uint16_t slot = (uint16_t)(i - i0);
+      for (size_t i = 0; i < C.size(); ++i) {
+        int64_t e = C[i];
+        uint16_t slot = (uint16_t)i;
         // R(p) -= f, R(q) += f (gather: owned ends only)
         if (!gather || local[p[e]] < B.nown)
           ent.emplace_back(local[p[e]], (uint16_t)(slot | 0x8000));
         if (!gather || local[q[e]] < B.nown) ent.emplace_back(local[q[e]], slot);
       }
-      emit(0, (int64_t)L.elpq.size(), (int)(i1 - i0), ent);
-      for (size_t i = i0; i < i1; ++i) {
-        const int64_t e = E[i];
+      emit(0, (int64_t)L.elpq.size(), (int)C.size(), ent);
+      for (int64_t e : C) {
         L.elpq.push_back((uint32_t)local[p[e]] | ((uint32_t)local[q[e]] << 16));
         L.ep.push_back(p[e]);
         L.eq.push_back(q[e]);

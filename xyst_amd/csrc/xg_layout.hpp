@@ -103,18 +103,19 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
 // is complete in its block: no halo slots (Block::slot0 is -1) and no
 // fix-up lists.  gather_faces: likewise every boundary face that touches one
 // of its nodes; without it a gather layout carries no boundary faces.
+// spread: a node's edges over the chunks of its block (spread_chunks).
 int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                  const std::vector<double>& d, int64_t ntri, const int* tri,
                  const uint8_t* besym, int block_nodes, int block_cap,
                  int chunk_slots, Layout& L, std::string& err, bool gather = false,
-                 bool gather_faces = false);
+                 bool gather_faces = false, bool spread = true);
 
 // Blocks of small meshes.  At the full block sizes a mesh of a few thousand
 // nodes fills a few of the 256 CUs, and each block walks its chunks alone: so
 // they are cut into about as many blocks as run at once, and where that is
 // the faster, into gather blocks, which need no halo fix-up.  Times of the
-// full blocks and of these when the lines were drawn (the tets not yet spread
-// over the chunks, their kernels' arithmetic heavier), in us:
+// full blocks and of these when the lines were drawn (chunks not yet spread,
+// the tet kernels' arithmetic heavier), in us:
 //  riemann::grad: sixteen nodes, four lanes each (its waves are independent);
 //  riemann::rhs (two workgroups per CU: at most 512 blocks): 12^3 20.6 ->
 //    6.9, 24^3 21.1 -> 9.9, 29^3 (27,000 nodes) 23.7 -> 14.5, with 6
