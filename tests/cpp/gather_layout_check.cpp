@@ -5,8 +5,9 @@
 // index and prefetch bound of the kernels must stay inside its list.
 // Input file: int64 npoin, ne, ntri, ntet; int32 p[ne], q[ne], tri[3 ntri],
 // tet[4 ntet].
-// Arguments: FILE KIND(rhs|grad|cho|tet|rows) NODES GATHER, for rows (node rows,
-// xg_rows.hpp) the lanes per node instead of GATHER.
+// Arguments: FILE KIND(rhs|grad|cho|tet|rows|gradrows) NODES GATHER, for rows
+// (node rows, xg_rows.hpp) the lanes per node instead of GATHER, for gradrows
+// (riemann::grad's) the lanes that it has to choose, NODES 0.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -22,14 +23,24 @@ static int64_t val(int64_t item, int corner) { return (item * 7 + corner * 3) % 
 // every edge at both ends with that end's sign, every face at its three nodes,
 // in input order
 static void check_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
-                       const std::vector<int>& tri, int nodes, int lanes) {
+                       const std::vector<int>& tri, int nodes, int lanes, bool grad) {
   std::vector<double> d(3 * p.size());
   for (size_t i = 0; i < d.size(); ++i) d[i] = 1.0 + (double)i;
   xg::RowLayout L;
   std::string err;
-  const int cap = 700, per = 64 / lanes;
-  CHECK(xg::build_rows(npoin, p, q, d, (int64_t)tri.size() / 3, tri.data(), nodes, cap, lanes, L,
-                       err) == 0);
+  int cap = 700;
+  if (grad) {
+    int got = 0;
+    CHECK(xg::build_grad_rows(npoin, p, q, d, (int64_t)tri.size() / 3, tri.data(), L, got, err) ==
+          0);
+    CHECK(got == lanes);
+    nodes = got == 1 ? xg::kGradNodes : 16;
+    cap = got == 1 ? xg::kGradCap : xg::kGradSmallCap;
+  } else {
+    CHECK(xg::build_rows(npoin, p, q, d, (int64_t)tri.size() / 3, tri.data(), nodes, cap, lanes,
+                         L, err) == 0);
+  }
+  const int per = 64 / lanes;
   std::vector<std::vector<int64_t>> edges(npoin), faces(npoin), ge(npoin), gf(npoin);
   for (size_t e = 0; e < p.size(); ++e) {
     edges[p[e]].push_back(-(int64_t)e - 1);
@@ -101,8 +112,8 @@ int main(int argc, char** argv) {
   CHECK(std::fread(tri.data(), 4, tri.size(), f) == tri.size());
   CHECK(std::fread(t32.data(), 4, t32.size(), f) == t32.size());
   std::fclose(f);
-  if (!std::strcmp(kind, "rows")) {
-    check_rows(npoin, p, q, tri, nodes, std::atoi(argv[4]));
+  if (!std::strcmp(kind, "rows") || !std::strcmp(kind, "gradrows")) {
+    check_rows(npoin, p, q, tri, nodes, std::atoi(argv[4]), !std::strcmp(kind, "gradrows"));
     return 0;
   }
   std::string err;

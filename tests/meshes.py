@@ -60,3 +60,23 @@ def smooth_state(coord, seed=7, gamma=1.4):
     U[:, 3] = r * w
     U[:, 4] = p / (gamma - 1.0) + 0.5 * r * (u * u + v * v + w * w)
     return U
+
+
+def hub_mesh(k, hub="last"):
+    """A ball of k surface nodes, each joined to one node at its centre, which
+    has k neighbours and is numbered first or last; as box_mesh's dict."""
+    from scipy.spatial import ConvexHull
+    i = np.arange(k) + 0.5
+    z, t = 1.0 - 2.0 * i / k, np.pi * (1.0 + 5.0 ** 0.5) * i
+    s = np.sqrt(1.0 - z * z)
+    X = np.column_stack([s * np.cos(t), s * np.sin(t), z])
+    tri = ConvexHull(X).simplices.astype(np.int64)
+    a, b, c = X[tri[:, 0]], X[tri[:, 1]], X[tri[:, 2]]
+    inward = np.einsum("ij,ij->i", np.cross(b - a, c - a), a) < 0.0
+    tri[inward] = tri[inward][:, ::-1]
+    centre = k if hub == "last" else 0
+    X = np.vstack([X, np.zeros(3)]) if hub == "last" else np.vstack([np.zeros(3), X])
+    tri = tri + (hub != "last")
+    tet = np.column_stack([np.full(len(tri), centre), tri])
+    return {"coord": np.ascontiguousarray(X.T), "inpoel": tet, "triinpoel": tri,
+            "faceset": np.ones(len(tri), np.int32)}

@@ -437,7 +437,7 @@ int build_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
       }
       W.erows = (int)((most + lanes - 1) / lanes);
       W.frows = (int)((fmost + lanes - 1) / lanes);
-      if (W.erows > 255 || W.frows > 255) {
+      if (W.erows > 65535 || W.frows > 65535) {
         err = "rows: too many edges at a node";
         return XG_EUNSUPPORTED;
       }
@@ -490,6 +490,22 @@ int build_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
     for (int h : halo) local[h] = -1;
   }
   return XG_OK;
+}
+
+int build_grad_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                    const std::vector<double>& d, int64_t ntri, const int* tri, RowLayout& L,
+                    int& lanes, std::string& err) {
+  if (npoin <= kSmallGrad) {
+    std::string why;
+    lanes = 4;
+    const int rc = build_rows(npoin, p, q, d, ntri, tri, 16, kGradSmallCap, lanes, L, why);
+    if (rc != XG_EUNSUPPORTED) {
+      if (rc) err = why;
+      return rc;
+    }
+  }
+  lanes = 1;
+  return build_rows(npoin, p, q, d, ntri, tri, kGradNodes, kGradCap, lanes, L, err);
 }
 
 // kozak::rhs layout: blocks as above on the tets' node graph; a block owns the

@@ -825,16 +825,8 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
   const xg::BlockPlan br = xg::rhs_blocks(npoin);
   xg::RowLayout L;
   xg::Layout LR;
-  int lanes = npoin <= xg::kSmallGrad ? 4 : 1;
-  int rc = XG_EUNSUPPORTED;
-  if (lanes == 4)   // a node with too many neighbours for it: the other
-    rc = xg::build_rows((int)npoin, p, q, d, ntri, tri32.data(), 16, xg::kGradSmallCap, 4, L,
-                        c->err);
-  if (rc == XG_EUNSUPPORTED) {
-    lanes = 1;
-    rc = xg::build_rows((int)npoin, p, q, d, ntri, tri32.data(), xg::kGradNodes, xg::kGradCap,
-                        1, L, c->err);
-  }
+  int lanes = 1;
+  int rc = xg::build_grad_rows((int)npoin, p, q, d, ntri, tri32.data(), L, lanes, c->err);
   if (rc) return rc;
   rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, br.nodes, xg::kRhsCap,
                         xg::kRhsSlots, LR, c->err, br.gather, true);

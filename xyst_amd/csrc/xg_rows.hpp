@@ -31,7 +31,7 @@ struct RowLayout {
   std::vector<RowBlock> blk;
   std::vector<RowWave> wave;
   std::vector<int> halo;
-  std::vector<uint8_t> deg, fdeg;   // per wave and lane: its entries, faces
+  std::vector<uint16_t> deg, fdeg;  // per wave and lane: its entries, faces
   std::vector<uint16_t> nb;         // neighbour, block-local
   std::vector<double> dx, dy, dz;   // signed integrals
   std::vector<int64_t> eidx;        // input edge of each entry (-1: padding)
@@ -39,10 +39,16 @@ struct RowLayout {
   std::vector<int64_t> fidx;        // input face of each face entry (-1: padding)
 };
 
-// XG_EUNSUPPORTED when a node has more neighbours than cap, or more than 255
-// entries or faces per lane
+// XG_EUNSUPPORTED when a node and its neighbours are more than cap nodes, or
+// it has more than 65535 entries or faces per lane
 int build_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                const std::vector<double>& d, int64_t ntri, const int* tri, int block_nodes,
                int cap, int lanes, RowLayout& L, std::string& err);
+
+// riemann::grad's rows (xg_layout.hpp, kGrad*) and their lanes per node: four
+// on small meshes, unless a node has more neighbours than their blocks hold.
+int build_grad_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                    const std::vector<double>& d, int64_t ntri, const int* tri, RowLayout& L,
+                    int& lanes, std::string& err);
 
 }  // namespace xg

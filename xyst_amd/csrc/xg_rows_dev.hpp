@@ -13,8 +13,7 @@ struct RowsDev {
   int* wave0 = nullptr;
   int4* wave = nullptr;     // e0, erows, f0, frows
   int* halo = nullptr;
-  uint8_t *deg = nullptr, *fdeg = nullptr;
-  uint16_t* nb = nullptr;
+  uint16_t *deg = nullptr, *fdeg = nullptr, *nb = nullptr;
   double *dx = nullptr, *dy = nullptr, *dz = nullptr;
   uint32_t *fab = nullptr, *fcs = nullptr;
   double* fn = nullptr;     // normals of the face entries, 3 each
