@@ -7,7 +7,8 @@
 // tet[4 ntet].
 // Arguments: FILE KIND(rhs|grad|cho|tet|rows|gradrows) NODES GATHER, for rows
 // (node rows, xg_rows.hpp) the lanes per node instead of GATHER, for gradrows
-// (riemann::grad's) the lanes that it has to choose, NODES 0.
+// (riemann::grad's) the lanes that it has to choose, NODES 0.  NODES 0 of the
+// others: the operator's own choice of blocks, which has to be GATHER.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -126,8 +127,9 @@ int main(int argc, char** argv) {
     cap = xg::kKozCap;
     slots = xg::kKozPairSlots;
     std::vector<size_t> inp(t32.begin(), t32.end());
-    CHECK(xg::build_tet_layout(npoin, h[3], inp.data(), nodes, cap, T, err,
-                               xg::kTetsPerPairChunk, gather) == 0);
+    CHECK((nodes ? xg::build_tet_layout(npoin, h[3], inp.data(), nodes, cap, T, err,
+                                        xg::kTetsPerPairChunk, gather)
+                 : xg::build_kozak_layout(npoin, h[3], inp.data(), T, err)) == 0);
     for (int64_t e = 0; e < h[3]; ++e)
       for (int a = 0; a < 4; ++a) want[t32[e * 4 + a]] += val(t32[e * 4] + t32[e * 4 + 1], a);
   } else {
@@ -136,8 +138,11 @@ int main(int argc, char** argv) {
     slots = cho ? xg::kChunkSlots : grad ? xg::kGradSlots : xg::kRhsSlots;
     std::vector<double> d(3 * p.size(), 1.0);
     std::vector<uint8_t> sym(3 * h[2], 1);
-    CHECK(xg::build_layout(npoin, p, q, d, h[2], tri.data(), sym.data(), nodes, cap, slots, L,
-                           err, gather, true) == 0);
+    CHECK((nodes ? xg::build_layout(npoin, p, q, d, h[2], tri.data(), sym.data(), nodes, cap,
+                                    slots, L, err, gather, true)
+           : cho ? xg::build_cho_layout(npoin, p, q, d, h[2], tri.data(), L, err)
+                 : xg::build_rhs_layout(npoin, p, q, d, h[2], tri.data(), sym.data(), L, err)) ==
+          0);
     for (size_t e = 0; e < p.size(); ++e) {
       want[p[e]] -= val(e, 0);
       want[q[e]] += val(e, 0);
@@ -157,7 +162,7 @@ int main(int argc, char** argv) {
   if (gather) CHECK(nslot == 0 && fxn.empty());
   std::vector<int64_t> S(nslot, 0);
   for (const auto& B : blk) {
-    CHECK(B.nown > 0 && B.nown <= nodes && B.nloc <= cap && B.nloc <= slots);
+    CHECK(B.nown > 0 && (!nodes || B.nown <= nodes) && B.nloc <= cap && B.nloc <= slots);
     CHECK(gather ? B.slot0 == -1 : B.slot0 + B.nloc - B.nown <= nslot);
     std::vector<int> glob(B.nloc);
     for (int i = 0; i < B.nloc; ++i) {

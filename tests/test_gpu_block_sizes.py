@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from tests.meshes import Case, smooth_state
+from tests.meshes import Case, hub_mesh, smooth_state
 from xyst_amd.meshgen import box_mesh, renumber_mesh
 
 pytestmark = pytest.mark.gpu
@@ -127,4 +127,62 @@ def test_chorin(n):
     _close(X.vgrad(ctx, U, np.zeros((c.npoin, 9))), Go, A)
     Fo, A = O.chorin_flux(se, c.coord, c.tri, U, G9, 0.02, absacc=True)
     _close(X.flux(ctx, 0.02, U, G9, np.zeros((c.npoin, 3))), Fo, A)
+    ctx.close()
+
+
+# a node of more neighbours than the small meshes' blocks hold, numbered last:
+# one lane per node for the gradient (255, 256 around the change), scatter
+# blocks for the rhs, the tet and the chorin operators
+@pytest.mark.parametrize("k", [255, 256, 300, 400, 511])
+def test_riemann_hub(k):
+    from xyst_amd import riemann as X
+    print("hub k=%d" % k, flush=True)
+    m = hub_mesh(k)
+    c = Case(m["coord"], m["inpoel"], m["triinpoel"], m["faceset"], (1,))
+    U = smooth_state(c.coord)
+    ctx = X.Context(0)
+    ctx.upload_mesh(c.coord, c.se.sup, c.se.int, c.tri, c.besym)
+    G = ctx.grad(U)
+    Go, A = O.grad(c.se, c.coord, c.tri, U, absacc=True)
+    _close(G, Go, A)
+    Gv = Go / c.vol[:, None]
+    R = ctx.rhs(Gv, U)
+    Ro, A = O.rhs(O.cfg(), c.se, c.coord, c.tri, c.besym, Gv, U, absacc=True)
+    _close(R, Ro, A)
+    ctx.close()
+
+
+@pytest.mark.parametrize("k", [511, 512, 1500])
+def test_kozak_hub(k):
+    from xyst_amd import kozak as K
+    from xyst_amd import riemann as X
+    print("hub k=%d" % k, flush=True)
+    m = hub_mesh(k)
+    U = smooth_state(m["coord"])
+    ctx = X.Context(0)
+    K.upload(ctx, m["coord"], m["inpoel"])
+    Ro, A = O.kozak_rhs(O.cfg(), m["coord"], m["inpoel"], 1e-3, U, absacc=True)
+    _close(K.rhs(ctx, 1e-3, U), Ro, A)
+    ctx.close()
+
+
+@pytest.mark.parametrize("k", [615, 616, 1500])
+def test_chorin_hub(k):
+    from xyst_amd import chorin as X
+    from xyst_amd import riemann as R
+    print("hub k=%d" % k, flush=True)
+    m = hub_mesh(k)
+    e, d = O.chocg_domint(m["coord"], m["inpoel"])
+    se = O.domsuped(m["inpoel"], e, d)
+    ctx = R.Context(0)
+    X.upload(ctx, m["coord"], se.sup, se.int, m["triinpoel"])
+    rng = np.random.default_rng(k)
+    n = k + 1
+    U, P = rng.standard_normal((n, 3)), rng.standard_normal(n)
+    G9, Gp = rng.standard_normal((n, 9)), rng.standard_normal((n, 3))
+    Ro, A = O.chorin_rhs(O.chocfg(flux="damp4", stab=True, mu=0.05), se, m["coord"],
+                         m["triinpoel"], P, U, G9, absacc=True)
+    _close(X.rhs(ctx, X.config("damp4", stab=True, mu=0.05), P, U, G9), Ro, A)
+    Do, A = O.chorin_div(se, m["coord"], m["triinpoel"], 0.01, P, Gp, U, stab=True, absacc=True)
+    _close(X.div(ctx, 0.01, P, Gp, U, np.zeros(n), stab=True), Do, A)
     ctx.close()

@@ -40,3 +40,18 @@ def _check(exe, tmp_path, k, hub, *args):
 @pytest.mark.parametrize("k,lanes", [(255, 4), (256, 1), (300, 1), (511, 1), (767, 1)])
 def test_gradient_rows(exe, tmp_path, k, lanes, hub):
     _check(exe, tmp_path, k, hub, "gradrows", 0, lanes)
+
+
+# gather blocks (1) as long as one holds the hub's neighbours, then scatter
+# blocks (0), whose nodes need not be with a hub that is numbered last
+@pytest.mark.parametrize("kind,k,gather", [
+    ("rhs", 311, 1), ("rhs", 312, 0), ("rhs", 400, 0), ("rhs", 1500, 0),
+    ("tet", 511, 1), ("tet", 512, 0), ("tet", 1500, 0),
+    ("cho", 615, 1), ("cho", 616, 0), ("cho", 1500, 0)])
+def test_blocks(exe, tmp_path, kind, k, gather):
+    _check(exe, tmp_path, k, "last", kind, 0, gather)
+
+
+@pytest.mark.parametrize("kind,k", [("rhs", 311), ("tet", 511), ("cho", 615)])
+def test_blocks_hub_first(exe, tmp_path, kind, k):
+    _check(exe, tmp_path, k, "first", kind, 0, 1)

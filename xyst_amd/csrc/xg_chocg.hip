@@ -845,11 +845,8 @@ int xg_chocg_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
       return fail(c, XG_EINVAL, "xg_chocg_upload: boundary face node out of range");
   std::vector<int> tri32(ntri * 3);
   for (int64_t f = 0; f < ntri * 3; ++f) tri32[f] = (int)tri[f];
-  std::vector<uint8_t> nosym(ntri * 3 + 1, 0);
   xg::Layout L;
-  const xg::BlockPlan plan = xg::cho_blocks(npoin);
-  int rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), nosym.data(), plan.nodes,
-                            xg::kBlockCap, xg::kChunkSlots, L, c->err, plan.gather, true, false);
+  int rc = xg::build_cho_layout((int)npoin, p, q, d, ntri, tri32.data(), L, c->err);
   if (rc) return rc;
   std::vector<double> dwl(L.eidx.size());
   for (size_t e = 0; e < L.eidx.size(); ++e) dwl[e] = w[L.eidx[e]];

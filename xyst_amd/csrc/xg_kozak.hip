@@ -922,9 +922,7 @@ int xg_kozak_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
     return fail(c, XG_EINVAL, "xg_kozak_upload: bad arguments");
   XG_HIP(c, hipSetDevice(c->device));
   xg::TetLayout L;
-  const xg::BlockPlan plan = xg::tet_blocks(npoin);
-  int rc = xg::build_tet_layout((int)npoin, ntet, inpoel, plan.nodes, xg::kKozCap, L, c->err,
-                                xg::kTetsPerPairChunk, plan.gather);
+  int rc = xg::build_kozak_layout((int)npoin, ntet, inpoel, L, c->err);
   if (rc) return rc;
   auto* k = new KozakMesh;
   k->npoin = (int)npoin;

@@ -667,6 +667,45 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
   return XG_OK;
 }
 
+// build(plan) with the size's plan and, where its gather blocks cannot hold a
+// node's neighbours, with the full scatter blocks.
+template <class Build>
+static int by_plan(const BlockPlan& plan, int full_nodes, std::string& err, Build build) {
+  if (!plan.gather) return build(plan, err);
+  std::string why;
+  const int rc = build(plan, why);
+  if (rc == XG_EUNSUPPORTED) return build(BlockPlan{full_nodes, false}, err);
+  if (rc) err = why;
+  return rc;
+}
+
+int build_rhs_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                     const std::vector<double>& d, int64_t ntri, const int* tri,
+                     const uint8_t* besym, Layout& L, std::string& err) {
+  return by_plan(rhs_blocks(npoin), kRhsNodes, err, [&](const BlockPlan& b, std::string& e) {
+    return build_layout(npoin, p, q, d, ntri, tri, besym, b.nodes, kRhsCap, kRhsSlots, L, e,
+                        b.gather, true);
+  });
+}
+
+int build_kozak_layout(int npoin, int64_t ntet, const size_t* inpoel, TetLayout& L,
+                       std::string& err) {
+  return by_plan(tet_blocks(npoin), kKozNodes, err, [&](const BlockPlan& b, std::string& e) {
+    return build_tet_layout(npoin, ntet, inpoel, b.nodes, kKozCap, L, e, kTetsPerPairChunk,
+                            b.gather);
+  });
+}
+
+int build_cho_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                     const std::vector<double>& d, int64_t ntri, const int* tri, Layout& L,
+                     std::string& err) {
+  const std::vector<uint8_t> nosym(ntri * 3 + 1, 0);
+  return by_plan(cho_blocks(npoin), kBlockNodes, err, [&](const BlockPlan& b, std::string& e) {
+    return build_layout(npoin, p, q, d, ntri, tri, nosym.data(), b.nodes, kBlockCap, kChunkSlots,
+                        L, e, b.gather, true, false);
+  });
+}
+
 // Recursive coordinate bisection into cells of at most `leaf` nodes; the
 // order of nodes inside a cell is their original order.
 static void rcb(std::vector<int>& ids, size_t lo, size_t hi, const double* x,

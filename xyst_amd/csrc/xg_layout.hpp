@@ -154,6 +154,20 @@ inline BlockPlan cho_blocks(int64_t npoin) {
   return {kBlockNodes, false};
 }
 
+// The layouts of riemann::rhs, the tet operators and the chorin operators by
+// these plans.  A gather block holds all neighbours of its nodes, a scatter
+// block those with larger ids only (for tets: the nodes of the tets whose
+// smallest node it owns), so a mesh with a node of too many neighbours for
+// gather blocks takes the full scatter blocks whatever its size.
+int build_rhs_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                     const std::vector<double>& d, int64_t ntri, const int* tri,
+                     const uint8_t* besym, Layout& L, std::string& err);
+int build_kozak_layout(int npoin, int64_t ntet, const size_t* inpoel, TetLayout& L,
+                       std::string& err);
+int build_cho_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
+                     const std::vector<double>& d, int64_t ntri, const int* tri, Layout& L,
+                     std::string& err);
+
 int block_order(int64_t npoin, const double* x, const double* y,
                 const double* z, int leaf, size_t* perm);
 

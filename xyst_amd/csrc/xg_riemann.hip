@@ -822,14 +822,12 @@ int xg_mesh_upload(xg_ctx* c, int64_t npoin, const double* x, const double* y,
       return fail(c, XG_EINVAL, "xg_mesh_upload: boundary face node out of range");
   std::vector<int> tri32(ntri * 3);
   for (int64_t f = 0; f < ntri * 3; ++f) tri32[f] = (int)tri[f];
-  const xg::BlockPlan br = xg::rhs_blocks(npoin);
   xg::RowLayout L;
   xg::Layout LR;
   int lanes = 1;
   int rc = xg::build_grad_rows((int)npoin, p, q, d, ntri, tri32.data(), L, lanes, c->err);
   if (rc) return rc;
-  rc = xg::build_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, br.nodes, xg::kRhsCap,
-                        xg::kRhsSlots, LR, c->err, br.gather, true);
+  rc = xg::build_rhs_layout((int)npoin, p, q, d, ntri, tri32.data(), besym, LR, c->err);
   if (rc) return rc;
   // normals of the rows' boundary faces, (b - a) x (c - a) / 12
   std::vector<double> fn(L.fidx.size() * 3, 0.0);
