@@ -36,6 +36,7 @@
 #include "xg_amg.hpp"
 #include "xg_cg.hpp"
 #include "xg_gnn.hpp"
+#include "xg_stop.hpp"
 #include "xg_tiles_dev.hpp"
 
 using namespace xgd;
@@ -49,11 +50,7 @@ static_assert(kCgThreads == kTileThreads, "the recurrence kernels walk tiles");
 constexpr int kVecParts = 512;    // workgroups of the vector kernels (max)
 constexpr int kBufLen = 2 * kVecParts + 8;   // rz[.], rr[.], finished flag
 
-struct CgState {
-  double normb, rho0, rr;
-  long long it;
-  int done, converged;
-};
+using xg::CgState;
 
 }  // namespace
 
@@ -190,16 +187,13 @@ __device__ inline void record_stop(CgState* st, CgState* pub, int j, double rr, 
                                    double tol_nb) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int conv = !(normr > tol_nb) ? 1 : 0;
-    st->it = j - 1;
-    st->rr = rr;
-    st->converged = conv;
-    st->done = 1;
+    xg::stop_record(*st, j - 1, rr, conv);
     volatile CgState* h = pub;
     h->it = j - 1;
     h->rr = rr;
     h->converged = conv;
     __threadfence_system();
-    h->done = 1;
+    h->found = 1;
   }
 }
 
@@ -263,9 +257,7 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_setup_final(
     st->normb = sqrt(BB);
     st->rho0 = RZ;
     st->rr = RR;
-    st->it = 0;
-    st->done = 0;
-    st->converged = 0;
+    xg::stop_clear(*st);
   }
 }
 
@@ -318,8 +310,8 @@ struct FcgRow {
 // pairs the previous update wrote), q = A p_j, partials of
 // (p_j, q) (ConjugateGradients::next/qAp, :585-635).  The stop test of
 // ConjugateGradients::x after iteration j - 1 runs here: every workgroup
-// takes the same sums and the first one records the stop, which the update
-// kernel of this iteration and all later launches of the batch read.
+// takes the same sums and the first one records the stop for this iteration's
+// update kernel, which passes it on to the later iterations (xg_stop.hpp).
 // An iteration (this and k_cg_update) moves 12 nnz + 44 n bytes of matrix
 // and pairs and 76 n of vectors in FP64: 15 us at 64^3 (274,625 rows) at the
 // copy rate, 26 us measured (37 before the loads were put ahead of the
@@ -331,7 +323,7 @@ __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4)))
     const double* __restrict__ rzb, int nvp, double* __restrict__ pq, CgState* st,
     CgState* pub, long long maxit, double tol_nb) {
   __shared__ TileLds<T> lds;
-  const int done = st->done;
+  const bool past = xg::stop_past(*st);
   PairSource<T> src{reinterpret_cast<const Pair<T>*>(zp), T(0)};
   CgRow<T> row{src, pnew, q, 0.0};
   const bool ran = tiles_spmv<T, false, 3>(
@@ -342,7 +334,7 @@ __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4)))
         const bool finished = cur[2 * kVecParts] != 0.0;
         double v[3] = {part_of(cur, nvp), part_of(cur + kVecParts, nvp),
                        j >= 2 ? part_of(old, nvp) : 0.0};
-        if (done) return false;
+        if (past) return false;
         block_sums_all<3>(v, lds.sm);
         const double normr = sqrt(v[1]);
         if (j >= 2 && (finished || normr < tol_nb || (long long)(j - 1) >= maxit)) {
@@ -373,10 +365,10 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_update(
     int j, int64_t n, const T* __restrict__ q, const T* __restrict__ d,
     const T* __restrict__ p, T* __restrict__ r, T* __restrict__ x,
     T* __restrict__ zp, double* __restrict__ rzb, int nvp, const double* __restrict__ pq,
-    int nsp, const CgState* st, double brk) {
+    int nsp, CgState* st, double brk) {
   constexpr int V = Vec<T>::V;
   __shared__ double sm[2][kCgThreads / 64];
-  const int done = st->done;  // the stop test of this iteration's SpMV
+  const bool found = xg::stop_found(*st);  // the stop test of this iteration's SpMV
   const int64_t nv = n / V, step = (int64_t)gridDim.x * kCgThreads;
   int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
   Vec<T> rv, qv, dv, pv, xv;
@@ -389,7 +381,10 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_update(
   };
   if (i < nv) load(i);
   double v[2] = {part_of(rzb + ((j - 1) & 1) * kBufLen, nvp), part_of(pq, nsp)};
-  if (done) return;
+  if (found) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) xg::stop_pass(*st);
+    return;
+  }
   block_sums_all<2>(v, sm);
   const bool finished = fabs(v[1]) < brk;      // ConjugateGradients.cpp:680-687
   const double alpha = finished ? 0.0 : v[0] / v[1];
@@ -520,11 +515,7 @@ __global__ __launch_bounds__(kCgThreads) void k_residual_norm(
 
 // a new solve on the state: iteration count and flags cleared
 __global__ void k_state_reset(CgState* st) {
-  if (threadIdx.x == 0) {
-    st->it = 0;
-    st->done = 0;
-    st->converged = 0;
-  }
+  if (threadIdx.x == 0) xg::stop_clear(*st);
 }
 
 // st->rr = sum of part[0, n) (one workgroup)
@@ -543,14 +534,14 @@ __global__ __launch_bounds__(kCgThreads) void k_fcg_in(
     int k, const double* __restrict__ part, int npart, long long maxit, double target,
     CgState* st, CgState* pub, const double* __restrict__ r, AmgInput in) {
   __shared__ double sm[1][kCgThreads / 64];
-  const int done = st->done;
+  const bool past = xg::stop_past(*st);
   const int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
   const bool mine = i < in.n;
   const float b = mine ? in.sign[i] * (float)r[i] : 0.f;
   const float wd = mine ? in.w * in.dinv[i] : 0.f;
   if (k > 0) {
     double v[1] = {part_of(part, npart)};
-    if (done) return;
+    if (past) return;
     block_sums_all<1>(v, sm);
     const double nr = sqrt(v[0]);
     if (nr < target || k >= maxit) {
@@ -619,7 +610,7 @@ __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4)))
   __shared__ TileLds<double> lds;
   PairSource<double> src{reinterpret_cast<const Pair<double>*>(zp), 0.0};
   FcgRow row{src, r, pnew, q, 0.0, 0.0};
-  const int done = st ? st->done : 0;
+  const bool found = st && xg::stop_found(*st);
   const bool ran = tiles_spmv<double, false, 2>(
       M, a, src, row,
       [&]() {
@@ -628,7 +619,7 @@ __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4)))
           v[0] = part_of(cur, nvp);
           v[1] = part_of(prev + kMaxParts, nsp);
         }
-        if (done) return false;
+        if (found) return false;
         block_sums_all<2>(v, lds.sm);
         src.bt = v[1] != 0.0 ? -v[0] / v[1] : 0.0;
         return true;
@@ -644,10 +635,10 @@ __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4)))
 __global__ __launch_bounds__(kCgThreads) void k_fcg_update(
     int64_t n, const double* __restrict__ p, const double* __restrict__ q,
     double* __restrict__ r, double* __restrict__ x, double* __restrict__ fb, int nsp,
-    const CgState* st) {
+    CgState* st) {
   constexpr int V = Vec<double>::V;
   __shared__ double sm[2][kCgThreads / 64];
-  const int done = st ? st->done : 0;
+  const bool found = st && xg::stop_found(*st);
   const int64_t nv = n / V, step = (int64_t)gridDim.x * kCgThreads;
   int64_t i = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
   Vec<double> rv, qv, pv, xv;
@@ -659,7 +650,10 @@ __global__ __launch_bounds__(kCgThreads) void k_fcg_update(
   };
   if (i < nv) load(i);
   double v[2] = {part_of(fb + kMaxParts, nsp), part_of(fb + 2 * kMaxParts, nsp)};
-  if (done) return;
+  if (found) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) xg::stop_pass(*st);
+    return;
+  }
   block_sums_all<2>(v, sm);
   const double alpha = v[0] != 0.0 ? v[1] / v[0] : 0.0;
   double rr = 0.0;
@@ -802,7 +796,7 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
   const int batch = 8;
   // the (z, p) pairs of the first SpMV; each update writes the next ones
   T* zp = f32 ? reinterpret_cast<T*>(s->zp32) : reinterpret_cast<T*>(s->zp);
-  s->hpub->done = 0;
+  s->hpub->found = 0;
   hipLaunchKernelGGL(k_pack_zp<T>, dim3((unsigned)((s->nrow + kCgThreads - 1) / kCgThreads)),
                      dim3(kCgThreads), 0, c->stream, s->nrow, z,
                      (jstart - 1) & 1 ? p1 : p0, zp);
@@ -826,7 +820,7 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
   for (;;) {
     XG_HIP(c, hipEventSynchronize(s->ev[waited & 1]));
     ++waited;
-    if (static_cast<volatile CgState*>(s->hpub)->done) break;
+    if (static_cast<volatile CgState*>(s->hpub)->found) break;
     // the stop test holds at the latest in the SpMV of iteration maxit + 1
     while (enq < waited + 2 && jstart + enq * batch <= maxit + 1) {
       if ((rc = enqueue(jstart + enq * batch, (int)(enq & 1)))) return rc;
@@ -838,7 +832,6 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
   s->hst->it = s->hpub->it;
   s->hst->rr = s->hpub->rr;
   s->hst->converged = s->hpub->converged;
-  s->hst->done = 1;
   return XG_OK;
 }
 
@@ -854,7 +847,7 @@ int run_fcg_amg(xg_ctx* c, int64_t maxit, double target) {
   double* P[2] = {s->p0, s->p1};
   double* Q[2] = {s->q, s->q2};
   const AmgInput in = xg_amg_input(c);
-  s->hpub->done = 0;
+  s->hpub->found = 0;
   hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(64), 0, c->stream, s->st);
   auto enqueue = [&](int64_t k) -> int {
     double* Bk = s->fb + (k & 1) * 4 * kMaxParts;
@@ -864,7 +857,7 @@ int run_fcg_amg(xg_ctx* c, int64_t maxit, double target) {
                        in);
     int nzq = 0, rc;
     if ((rc = xg_amg_apply_fcg(c, k > 0 ? P[(k + 1) & 1] : nullptr, Q[(k + 1) & 1],
-                               s->zp, Bk, &s->st->done, &nzq)))
+                               s->zp, Bk, &s->st->found, &nzq)))
       return rc;
     hipLaunchKernelGGL(k_fcg_spmv, dim3(gt), dim3(kCgThreads), 0, c->stream, k == 0 ? 1 : 0,
                        s->tiles(), s->da, s->zp, P[k & 1], Q[k & 1], s->r, Bp, Bk, nzq, gt,
@@ -881,7 +874,7 @@ int run_fcg_amg(xg_ctx* c, int64_t maxit, double target) {
     // iteration maxit only holds the stop test
     if (k < maxit && (rc = enqueue(k + 1))) return rc;
     XG_HIP(c, hipEventSynchronize(s->ev[k & 1]));
-    if (static_cast<volatile CgState*>(s->hpub)->done) break;
+    if (static_cast<volatile CgState*>(s->hpub)->found) break;
     if (k > maxit) return fail(c, XG_EHIP, "flexible CG: stop test not reached on the device");
   }
   XG_HIP(c, hipStreamSynchronize(c->stream));
