@@ -22,7 +22,7 @@
 static int64_t val(int64_t item, int corner) { return (item * 7 + corner * 3) % 1009 - 500; }
 
 // every edge at both ends with that end's sign, every face at its three nodes,
-// in input order
+// in input order (one lane: edges from both ends inward)
 static void check_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                        const std::vector<int>& tri, int nodes, int lanes, bool grad) {
   std::vector<double> d(3 * p.size());
@@ -48,6 +48,15 @@ static void check_rows(int npoin, const std::vector<int>& p, const std::vector<i
     edges[q[e]].push_back((int64_t)e + 1);
   }
   for (size_t k = 0; k < tri.size(); ++k) faces[tri[k]].push_back(k);
+  if (lanes == 1)
+    for (auto& v : edges) {
+      std::vector<int64_t> w;
+      for (size_t a = 0, b = v.size(); a < b;) {
+        w.push_back(v[a++]);
+        if (a < b) w.push_back(v[--b]);
+      }
+      v = w;
+    }
   int next = 0;
   for (const auto& B : L.blk) {
     CHECK(B.own0 == next && B.nown > 0 && B.nown <= nodes && B.nloc <= cap);

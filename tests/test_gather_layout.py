@@ -47,3 +47,30 @@ def test_small_blocks_reach_every_node_once(exe, tmp_path, n, order):
                                    capture_output=True, text=True)
                 assert r.returncode == 0 and r.stdout.startswith("ok"), \
                     (kind, nodes, gather, r.stderr)
+
+
+@pytest.mark.parametrize("n,lanes", [(20, 1), (20, 4), (37, 1)])
+def test_row_sums_round_less_than_in_input_order(tmp_path, n, lanes):
+    """Numbered as bench.py numbers its meshes, the edges of a node ascend by
+    neighbour, and terms that nearly cancel lie far apart in input order: the
+    layout's order has to do better by a fifth (it does by a third)."""
+    from tests.meshes import smooth_state
+    exe = str(tmp_path / "row_sum_check")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", exe,
+                    os.path.join(ROOT, "tests", "cpp", "row_sum_check.cpp"),
+                    os.path.join(ROOT, "xyst_amd", "csrc", "xg_layout.cpp")], check=True)
+    m = box_mesh(n, seed=n)
+    m = renumber_mesh(m, X.mesh_rcm(m["coord"].shape[1], m["inpoel"]))
+    m = renumber_mesh(m, X.mesh_block_order(m["coord"], 1024))
+    e, d = X.mesh_domint(m["coord"], m["inpoel"])
+    u = smooth_state(m["coord"]).T
+    f = tmp_path / "sums.bin"
+    with open(f, "wb") as fh:
+        np.array([u.shape[1], len(e), len(u)], np.int64).tofile(fh)
+        np.ascontiguousarray(e.T, np.int32).tofile(fh)
+        np.ascontiguousarray(d, np.float64).tofile(fh)
+        np.ascontiguousarray(u).tofile(fh)
+    r = subprocess.run([exe, str(f), str(lanes)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    rows, ordered = (float(v) for v in r.stdout.split())
+    assert rows <= 0.8 * ordered, (rows, ordered)

@@ -461,8 +461,15 @@ int build_rows(int npoin, const std::vector<int>& p, const std::vector<int>& q,
       L.fdeg.resize(g0 + 64, 0);
       for (int k = w0; k < std::min(B.nown, w0 + per); ++k) {
         const int i = s + k, l0 = (k - w0) * lanes;
-        for (int64_t j = 0; j < off[i + 1] - off[i]; ++j) {
-          const int64_t ed = inc[off[i] + j];
+        // one lane: from both ends inward (the input's edges ascend by
+        // neighbour), so that opposite neighbours, whose terms nearly cancel,
+        // are added one after the other: the error of the gradient's sums
+        // on 49^3 is 3.5e-16 of the result, ascending 5.5e-16 (four lanes, a
+        // quarter of the terms each: 4.1e-16 so, ascending 3.8e-16)
+        const int64_t ndeg = off[i + 1] - off[i];
+        for (int64_t j = 0; j < ndeg; ++j) {
+          const int64_t o = lanes > 1 ? j : j & 1 ? ndeg - 1 - j / 2 : j / 2;
+          const int64_t ed = inc[off[i] + o];
           const int lane = l0 + (int)(j % lanes);
           const size_t at = W.e0 + 64 * (size_t)(j / lanes) + lane;
           const bool first = p[ed] == i;

@@ -2,14 +2,14 @@
 // to be evaluated at both ends (xg_rows_dev.hpp).
 //
 // Blocks of consecutive owned nodes as in xg_layout.hpp, with every outside
-// neighbour as halo.  The edges of a node lie in the order of the input, each
-// as the neighbour's block-local id and the edge integral with the sign of
-// this end (R(p) -= f, R(q) += f), interleaved over the 64 lanes of a wave, so
-// that a wave reads consecutive addresses and a lane sums its node in
-// registers: no edge records in LDS, no barrier after the block's nodes are
-// staged.  `lanes` lanes share a node (entry k goes to lane k % lanes) where
-// one per node would leave too few waves.  Boundary faces likewise, at each
-// of their nodes.
+// neighbour as halo.  The edges of a node are taken in the order of the input,
+// with one lane per node from both ends inward, each as the neighbour's
+// block-local id and the edge integral with the sign of this end (R(p) -= f,
+// R(q) += f), interleaved over the 64 lanes of a wave, so that a wave reads
+// consecutive addresses and a lane sums its node in registers: no edge records
+// in LDS, no barrier after the block's nodes are staged.  `lanes` lanes share a
+// node (entry k goes to lane k % lanes) where one per node would leave too few
+// waves.  Boundary faces likewise, at each of their nodes, in input order.
 #pragma once
 #include <cstdint>
 #include <string>
