@@ -30,6 +30,7 @@ int main(int argc, char** argv) {
   xg::build_tiles(nrow, ncol, ia.data(), ja.data(), t);
   long next = 0;
   size_t u0 = 0;
+  int64_t nwide = 0;
   for (const xg::Tile& w : t.tile) {
     if (w.row0 != next || w.row1 <= w.row0 || w.k0 != ia[w.row0] ||
         w.nz != ia[w.row1] - ia[w.row0])
@@ -43,6 +44,7 @@ int main(int argc, char** argv) {
     }
     if ((size_t)w.u0 != u0 || w.nu > w.nz) return printf("list of row %d\n", w.row0), 1;
     u0 += w.nu;
+    nwide += w.nu > xg::kTileCols;
     std::set<int32_t> used;
     for (int k = 0; k < w.nz; ++k) {
       if (t.lidx[w.k0 + k] >= w.nu || t.ucol[w.u0 + t.lidx[w.k0 + k]] != ja[w.k0 + k])
@@ -53,6 +55,7 @@ int main(int argc, char** argv) {
     for (int k = 1; k < w.nu; ++k)
       if (t.ucol[w.u0 + k] <= t.ucol[w.u0 + k - 1]) return printf("order\n"), 1;
   }
+  if (nwide != t.nwide) return printf("nwide\n"), 1;
   if (next != nrow || u0 != t.ucol.size() || t.lidx.size() != ja.size())
     return printf("sizes\n"), 1;
   printf("ok\n");

@@ -25,6 +25,22 @@ def _diagonal(n):
     return np.arange(n + 1), np.arange(n), 1.0 + np.arange(n) % 7
 
 
+def _scattered(n, k=7):
+    """Symmetric, k random entries a row and their mirror images of 1/(4 k), 2
+    on the diagonal: rows of less than 4 k entries, so eigenvalues between 1
+    and 3."""
+    rng = np.random.default_rng(n)
+    i, j = np.repeat(np.arange(n), k), rng.integers(0, n, n * k)
+    i, j = i[i != j], j[i != j]
+    key = np.unique(np.concatenate([i * n + j, j * n + i, np.arange(n) * (n + 1)]))
+    r, c = key // n, key % n
+    ia = np.searchsorted(r, np.arange(n + 1))
+    assert np.diff(ia).max() <= 4 * k
+    a = np.full(key.size, 0.25 / k)
+    a[r == c] = 2.0
+    return ia, c, a
+
+
 def _multiply(ia, ja, a, x):
     row = np.repeat(np.arange(ia.size - 1), np.diff(ia))
     return np.bincount(row, a * x[ja], ia.size - 1)
@@ -32,12 +48,15 @@ def _multiply(ia, ja, a, x):
 
 @pytest.mark.parametrize("kind,n", [("arrow", 2047), ("arrow", 2048), ("arrow", 2049),
                                     ("arrow", 5001), ("diagonal", 1), ("diagonal", 255),
-                                    ("diagonal", 257), ("diagonal", 2 ** 19 + 1)])
+                                    ("diagonal", 257), ("diagonal", 2 ** 19 + 1),
+                                    # lists of at most 700, of 768 to 1000 and of more columns
+                                    ("scattered", 700), ("scattered", 1000),
+                                    ("scattered", 5000)])
 def test_cg_at_the_edges_of_tiles(kind, n):
     """Condition at most 7, so a relative residual of 1e-12 (1e-10 with the
     FP32 recurrence) leaves at most seven times that error."""
     from xyst_amd import cg as X
-    ia, ja, a = (_arrow if kind == "arrow" else _diagonal)(n)
+    ia, ja, a = {"arrow": _arrow, "diagonal": _diagonal, "scattered": _scattered}[kind](n)
     print("tiles %s %d" % (kind, n), flush=True)
     x = np.sin(np.arange(n) + 1.0)
     b = _multiply(ia, ja, a, x) * 1e4

@@ -46,6 +46,7 @@ namespace {
 constexpr int kCgThreads = 256;
 constexpr int kLanesPerRow = 8;
 constexpr int kMaxParts = 2048;
+static_assert(xg::kTileCols == 3 * kTileThreads, "three columns a thread");
 static_assert(kCgThreads == kTileThreads, "the recurrence kernels walk tiles");
 constexpr int kVecParts = 512;    // workgroups of the vector kernels (max)
 constexpr int kBufLen = 2 * kVecParts + 8;   // rz[.], rr[.], finished flag
@@ -70,6 +71,7 @@ struct CgSolver {
   std::vector<DevArr> allocs;
   int *dia = nullptr, *dja = nullptr;
   int ntile = 0;                 // SpMV tiles
+  bool wide = false;             // many of them with long column lists
   xg::Tile* dtile = nullptr;
   int* ducol = nullptr;
   uint16_t* dlidx = nullptr;
@@ -316,7 +318,11 @@ struct FcgRow {
 // and pairs and 76 n of vectors in FP64: 15 us at 64^3 (274,625 rows) at the
 // copy rate, 26 us measured (37 before the loads were put ahead of the
 // scalars, 28 before the column lists); 62 us at 100^3, 81 before.
-template <class T>
+// COLS: columns loaded a tile ahead.  Four in FP32 where more than an eighth of
+// the tiles list more than three hold (band numberings from 160^3 on: RCM at
+// 160^3 190 -> 187 us an iteration, at 192^3 320 -> 310); elsewhere three
+// (compact cells at 160^3 190, with four 193).  In FP64 a fourth would spill.
+template <class T, int COLS>
 __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_cg_spmv(
     int j, xg::TileMat M, const T* __restrict__ a, const T* __restrict__ zp,
     T* __restrict__ pnew, T* __restrict__ q,
@@ -326,7 +332,7 @@ __global__ __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(4)))
   const bool past = xg::stop_past(*st);
   PairSource<T> src{reinterpret_cast<const Pair<T>*>(zp), T(0)};
   CgRow<T> row{src, pnew, q, 0.0};
-  const bool ran = tiles_spmv<T, false, 3>(
+  const bool ran = tiles_spmv<T, false, COLS>(
       M, a, src, row,
       [&]() {
         const double* cur = rzb + ((j - 1) & 1) * kBufLen;
@@ -796,6 +802,7 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
   const int batch = 8;
   // the (z, p) pairs of the first SpMV; each update writes the next ones
   T* zp = f32 ? reinterpret_cast<T*>(s->zp32) : reinterpret_cast<T*>(s->zp);
+  auto spmv = f32 && s->wide ? k_cg_spmv<T, sizeof(T) == 4 ? 4 : 3> : k_cg_spmv<T, 3>;
   s->hpub->found = 0;
   hipLaunchKernelGGL(k_pack_zp<T>, dim3((unsigned)((s->nrow + kCgThreads - 1) / kCgThreads)),
                      dim3(kCgThreads), 0, c->stream, s->nrow, z,
@@ -804,7 +811,7 @@ int run_cg(xg_ctx* c, const T* a, T* z, T* p0, T* p1, T* q, const T* d, T* r, T*
     for (int i = 0; i < batch; ++i) {
       const int j = (int)(j0 + i);
       T* pnew = j & 1 ? p1 : p0;
-      hipLaunchKernelGGL(k_cg_spmv<T>, dim3(gr), dim3(kCgThreads), 0, c->stream, j,
+      hipLaunchKernelGGL(spmv, dim3(gr), dim3(kCgThreads), 0, c->stream, j,
                          s->tiles(), a, zp, pnew, q, s->rzb, gv, s->pq, s->st, s->hpub,
                          (long long)maxit, tol_nb);
       hipLaunchKernelGGL(k_cg_update<T>, dim3(gv), dim3(kCgThreads), 0, c->stream, j,
@@ -1027,6 +1034,7 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
   xg::TileSet ts;
   xg::build_tiles(nrow, nrow, s->ia.data(), s->ja.data(), ts);
   s->ntile = (int)ts.tile.size();
+  s->wide = 8 * ts.nwide > (int64_t)ts.tile.size();
   std::vector<float> a32(nnz);
   for (int64_t j = 0; j < nnz; ++j) a32[j] = (float)a[j];
   int rc;

@@ -60,7 +60,10 @@ void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* j
   }
   for (int64_t p = 0; p < npiece; ++p) {
     const int base = (int)t.ucol.size();
-    for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) t.tile[i].u0 += base;
+    for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) {
+      t.tile[i].u0 += base;
+      t.nwide += t.tile[i].nu > kTileCols;
+    }
     t.ucol.insert(t.ucol.end(), cols[p].begin(), cols[p].end());
   }
 }

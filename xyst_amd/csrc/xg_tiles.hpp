@@ -16,6 +16,7 @@ namespace xg {
 
 constexpr int kTileNnz = 2048;
 constexpr int kTileRows = 128;   // two threads of a workgroup per row
+constexpr int kTileCols = 768;   // columns that a workgroup loads a tile ahead
 
 struct alignas(32) Tile {
   int row0, row1;   // rows
@@ -36,6 +37,7 @@ struct TileMat {
 
 struct TileSet {
   bool has_long = false;        // a row is longer than a tile
+  int64_t nwide = 0;            // tiles with more than kTileCols columns
   std::vector<Tile> tile;
   std::vector<int32_t> ucol;    // the tiles' columns
   std::vector<uint16_t> lidx;   // per nonzero: position in its tile's list

@@ -37,7 +37,8 @@ struct TileLds {
 // next tile are in flight during the current one: its source values from the
 // start (their columns were loaded a tile before), the rest from the
 // products on.
-// COLS: columns a thread loads ahead (3: lists of up to 768 columns).
+// COLS: columns a thread loads ahead (3: lists of up to kTileCols columns; a
+// longer list costs its tile a chain of two loads).
 template <class T, bool LANES, int COLS, class Src, class Row, class Coef>
 __device__ inline bool tiles_spmv(const xg::TileMat& M, const T* __restrict__ a, Src& src,
                                   Row& row, Coef coef, TileLds<T>& lds) {
