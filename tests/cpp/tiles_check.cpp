@@ -1,6 +1,6 @@
 // Host check of the SpMV row tiles (xyst_amd/csrc/xg_tiles.cpp) on a seeded
 // random matrix with empty rows and rows longer than a tile:
-// tiles_check NROW NCOL MEAN_NNZ NLONG SEED.  Prints "ok" or the
+// tiles_check NROW NCOL MEAN_NNZ NLONG SEED [ROWS] (default: as the CG).  Prints "ok" or the
 // first mismatch.
 #include <cstdio>
 #include <cstdlib>
@@ -10,9 +10,9 @@
 #include "../../xyst_amd/csrc/xg_tiles.hpp"
 
 int main(int argc, char** argv) {
-  if (argc != 6) return 2;
+  if (argc != 6 && argc != 7) return 2;
   const long nrow = atol(argv[1]), ncol = atol(argv[2]), mean = atol(argv[3]);
-  const long nlong = atol(argv[4]), maxr = xg::kTileRows;
+  const long nlong = atol(argv[4]);
   std::mt19937 g(atoi(argv[5]));
   std::vector<int64_t> ia(1, 0);
   std::vector<int32_t> ja;
@@ -26,8 +26,14 @@ int main(int argc, char** argv) {
     ja.insert(ja.end(), c.begin(), c.end());
     ia.push_back((int64_t)ja.size());
   }
+  const int64_t nnz = (int64_t)ja.size();
+  const int maxr = argc == 7 ? atoi(argv[6]) : xg::tile_rows(nrow, nnz);
+  // at least three quarters of a tile's nonzeros or the most rows
+  if (argc != 7 && maxr != xg::kTileRowsMax &&
+      4 * maxr * nnz < 3 * xg::kTileNnz * nrow)
+    return printf("rows\n"), 1;
   xg::TileSet t;
-  xg::build_tiles(nrow, ncol, ia.data(), ja.data(), t);
+  xg::build_tiles(nrow, ncol, ia.data(), ja.data(), t, maxr);
   long next = 0;
   size_t u0 = 0;
   int64_t nwide = 0;

@@ -41,6 +41,16 @@ def _scattered(n, k=7):
     return ia, c, a
 
 
+def _band(n, k):
+    """Symmetric, k entries of -1/(2 k) on either side of 2 on the diagonal:
+    eigenvalues between 1 and 3."""
+    i = np.arange(n)
+    c = i[:, None] + np.arange(-k, k + 1)
+    ok = (c >= 0) & (c < n)
+    a = np.broadcast_to(np.where(np.arange(-k, k + 1) == 0, 2.0, -0.5 / k), c.shape)
+    return np.concatenate([[0], np.cumsum(ok.sum(1))]), c[ok], a[ok]
+
+
 def _multiply(ia, ja, a, x):
     row = np.repeat(np.arange(ia.size - 1), np.diff(ia))
     return np.bincount(row, a * x[ja], ia.size - 1)
@@ -51,12 +61,16 @@ def _multiply(ia, ja, a, x):
                                     ("diagonal", 257), ("diagonal", 2 ** 19 + 1),
                                     # lists of at most 700, of 768 to 1000 and of more columns
                                     ("scattered", 700), ("scattered", 1000),
-                                    ("scattered", 5000)])
+                                    ("scattered", 5000),
+                                    # 256 rows a tile up to 11 entries a row, 128 from 13 on
+                                    ("band1", 513), ("band5", 4097), ("band6", 4097)])
 def test_cg_at_the_edges_of_tiles(kind, n):
     """Condition at most 7, so a relative residual of 1e-12 (1e-10 with the
     FP32 recurrence) leaves at most seven times that error."""
     from xyst_amd import cg as X
-    ia, ja, a = {"arrow": _arrow, "diagonal": _diagonal, "scattered": _scattered}[kind](n)
+    ia, ja, a = {"arrow": _arrow, "diagonal": _diagonal, "scattered": _scattered,
+                 "band1": lambda n: _band(n, 1), "band5": lambda n: _band(n, 5),
+                 "band6": lambda n: _band(n, 6)}[kind](n)
     print("tiles %s %d" % (kind, n), flush=True)
     x = np.sin(np.arange(n) + 1.0)
     b = _multiply(ia, ja, a, x) * 1e4

@@ -24,3 +24,10 @@ def test_tiles_cover_the_matrix(exe, nrow, ncol, mean, nlong):
         r = subprocess.run([exe] + [str(v) for v in (nrow, ncol, mean, nlong, seed)],
                            capture_output=True, text=True)
         assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout
+
+
+@pytest.mark.parametrize("mean,rows", [(3, 128), (3, 256), (15, 256)])
+def test_tiles_of_given_rows(exe, mean, rows):
+    r = subprocess.run([exe, "5001", "5001", str(mean), "2", "3", str(rows)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout

@@ -46,6 +46,7 @@ namespace {
 constexpr int kCgThreads = 256;
 constexpr int kLanesPerRow = 8;
 constexpr int kMaxParts = 2048;
+static_assert(xg::kTileRowsMax == kTileThreads, "one thread a row");
 static_assert(xg::kTileCols == 3 * kTileThreads, "three columns a thread");
 static_assert(kCgThreads == kTileThreads, "the recurrence kernels walk tiles");
 constexpr int kVecParts = 512;    // workgroups of the vector kernels (max)
@@ -1032,7 +1033,7 @@ int xg_cg_matrix(xg_ctx* c, int ncomp, int64_t npoin, const size_t* ia,
   s->abc = s->a0;
   std::vector<int32_t> ia32(s->ia.begin(), s->ia.end());
   xg::TileSet ts;
-  xg::build_tiles(nrow, nrow, s->ia.data(), s->ja.data(), ts);
+  xg::build_tiles(nrow, nrow, s->ia.data(), s->ja.data(), ts, xg::tile_rows(nrow, nnz));
   s->ntile = (int)ts.tile.size();
   s->wide = 8 * ts.nwide > (int64_t)ts.tile.size();
   std::vector<float> a32(nnz);

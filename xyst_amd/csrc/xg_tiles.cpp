@@ -6,11 +6,12 @@
 
 namespace xg {
 
-void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t) {
+void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t,
+                 int rows) {
   t = TileSet();
   for (int64_t r = 0; r < nrow;) {
     int64_t r1 = r;
-    while (r1 < nrow && r1 - r < kTileRows && ia[r1 + 1] - ia[r] <= kTileNnz) ++r1;
+    while (r1 < nrow && r1 - r < rows && ia[r1 + 1] - ia[r] <= kTileNnz) ++r1;
     if (r1 == r) r1 = r + 1;
     Tile w{};
     w.row0 = (int)r;

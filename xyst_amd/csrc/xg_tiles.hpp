@@ -1,7 +1,8 @@
 // Row tiles of a CSR matrix for SpMV on the device (xg_cg.hip, xg_amg.hip).
 //
 // A tile is a run of consecutive rows with at most kTileNnz nonzeros and
-// kTileRows rows (a longer row is a tile of its own, without a column list).
+// kTileRows or kTileRowsMax rows (a longer row is a tile of its own, without a
+// column list).
 // Neighbouring rows share most of their columns: the matrix of a tet mesh
 // has some 560 different ones among a tile's 2048 nonzeros.  So a tile lists
 // its columns once, ascending, and its nonzeros hold 16-bit positions in
@@ -15,7 +16,8 @@
 namespace xg {
 
 constexpr int kTileNnz = 2048;
-constexpr int kTileRows = 128;   // two threads of a workgroup per row
+constexpr int kTileRows = 128;     // two lanes a row in the V-cycle's kernels
+constexpr int kTileRowsMax = 256;  // a thread a row
 constexpr int kTileCols = 768;   // columns that a workgroup loads a tile ahead
 
 struct alignas(32) Tile {
@@ -44,8 +46,18 @@ struct TileSet {
 };
 
 // Tiles of the matrix with row offsets ia (nrow + 1, from 0) and columns ja
-// below ncol.  Threads work on runs of tiles; the result does not depend on
-// their number.
-void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t);
+// below ncol, of at most `rows` rows.  Threads work on runs of tiles; the
+// result does not depend on their number.
+void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t,
+                 int rows = kTileRows);
+
+// Rows of a tile where one thread sums a row (the CG recurrences): twice
+// kTileRows where these would leave a quarter of a tile's nonzeros unused, as
+// below 12 entries a row.  An iteration on 10^6 rows with 128 and 256 rows a
+// tile: 7 entries a row 56.1 and 49.8 us in FP64, 43.3 and 35.4 in FP32; 3
+// entries 53.7 and 41.6, 41.2 and 30.7.  The matrix of a tet mesh has 15.
+inline int tile_rows(int64_t nrow, int64_t nnz) {
+  return 4 * kTileRows * nnz < 3 * kTileNnz * nrow ? kTileRowsMax : kTileRows;
+}
 
 }  // namespace xg
