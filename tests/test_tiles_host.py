@@ -31,3 +31,14 @@ def test_tiles_of_given_rows(exe, mean, rows):
     r = subprocess.run([exe, "5001", "5001", str(mean), "2", "3", str(rows)],
                        capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout
+
+
+def test_tiles_without_threads(tmp_path):
+    """Where no thread can be created the caller's does all the work."""
+    out = str(tmp_path / "tiles_check")
+    cpp = os.path.join(ROOT, "tests", "cpp")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-pthread", "-o", out,
+                    os.path.join(cpp, "tiles_check.cpp"), os.path.join(cpp, "no_threads.cpp"),
+                    os.path.join(ROOT, "xyst_amd", "csrc", "xg_tiles.cpp")], check=True)
+    r = subprocess.run([out, "200000", "200000", "15", "2", "1"], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", (r.stdout, r.stderr)

@@ -2,9 +2,40 @@
 #include "xg_tiles.hpp"
 
 #include <algorithm>
+#include <atomic>
+#include <exception>
+#include <system_error>
 #include <thread>
 
 namespace xg {
+
+namespace {
+
+// work() on up to nth threads, the caller's among them: as many as can be
+// created.  What one of them throws is thrown again here.
+template <class Work>
+void on_threads(int64_t nth, Work work) {
+  std::vector<std::exception_ptr> bad(std::max<int64_t>(nth, 1));
+  auto guarded = [&](int64_t k) {
+    try {
+      work();
+    } catch (...) {
+      bad[k] = std::current_exception();
+    }
+  };
+  std::vector<std::thread> th;
+  th.reserve(bad.size());
+  try {
+    for (int64_t k = 1; k < nth; ++k) th.emplace_back(guarded, k);
+  } catch (const std::system_error&) {   // no more threads: those there are
+  }
+  guarded(0);
+  for (auto& x : th) x.join();
+  for (const auto& e : bad)
+    if (e) std::rethrow_exception(e);
+}
+
+}  // namespace
 
 void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t,
                  int rows) {
@@ -27,10 +58,11 @@ void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* j
   const int64_t per = 512;   // tiles a piece of work: some million nonzeros
   const int64_t npiece = (nt + per - 1) / per;
   std::vector<std::vector<int32_t>> cols((size_t)npiece);
-  auto work = [&](int64_t p0, int64_t dp) {
+  std::atomic<int64_t> next{0};
+  auto work = [&] {
     std::vector<int32_t> at((size_t)ncol, -1);
     std::vector<int32_t> u;
-    for (int64_t p = p0; p < npiece; p += dp) {
+    for (int64_t p; (p = next++) < npiece;) {
       for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) {
         Tile& w = t.tile[i];
         if (w.nz > kTileNnz) continue;
@@ -52,13 +84,7 @@ void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* j
   };
   const int64_t nth = std::min<int64_t>(
       npiece, std::min(8u, std::max(1u, std::thread::hardware_concurrency())));
-  if (nth <= 1) {
-    work(0, 1);
-  } else {
-    std::vector<std::thread> th;
-    for (int64_t k = 0; k < nth; ++k) th.emplace_back(work, k, nth);
-    for (auto& x : th) x.join();
-  }
+  on_threads(nth, work);
   for (int64_t p = 0; p < npiece; ++p) {
     const int base = (int)t.ucol.size();
     for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) {
