@@ -225,7 +225,7 @@ int up_mat(xg_ctx* c, std::vector<DevArr>& L, const xg::Csr& A, AmgDevMat& D) {
   int rc;
   if ((rc = up(c, L, &ia, to_i32(A.ia))) || (t.has_long && (rc = up(c, L, &ja, A.ja))) ||
       (rc = up(c, L, &D.a, to_f32(A.a))) || (rc = up(c, L, &tile, t.tile)) ||
-      (rc = up(c, L, &ucol, t.ucol)) || (rc = up(c, L, &lidx, t.lidx)))
+      (rc = upload(c, L, &ucol, t.ucol)) || (rc = upload(c, L, &lidx, t.lidx)))
     return rc;
   D.M = xg::TileMat{(int)t.tile.size(), tile, ia, ja, ucol, lidx};
   return XG_OK;

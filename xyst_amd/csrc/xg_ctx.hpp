@@ -133,9 +133,9 @@ int upload(xg_ctx* c, std::vector<DevArr>& list, T** dst, const T* src,
   return XG_OK;
 }
 
-template <class T>
+template <class T, class A>
 int upload(xg_ctx* c, std::vector<DevArr>& list, T** dst,
-           const std::vector<T>& v) {
+           const std::vector<T, A>& v) {
   return upload(c, list, dst, v.data(), v.size());
 }
 

@@ -35,6 +35,50 @@ void on_threads(int64_t nth, Work work) {
     if (e) std::rethrow_exception(e);
 }
 
+// Set of columns as two levels of bits: bit c of `bits`, and bit w of `top`
+// where word w of `bits` is not empty, so that the set is read in order, and
+// emptied, in time of its size and its range / 4096.
+struct ColumnSet {
+  std::vector<uint64_t> bits, top;
+  std::vector<uint16_t> before;   // columns of the set before a word's
+  explicit ColumnSet(int64_t ncol)
+      : bits(ncol / 64 + 1, 0), top(ncol / 4096 + 1, 0), before(ncol / 64 + 1, 0) {}
+  // lidx[k] = position of ja[k] in the ascending list of the nz columns ja,
+  // which is appended to out; returns its length
+  int list(const int32_t* ja, int nz, uint16_t* lidx, std::vector<int32_t>& out) {
+    uint32_t t0 = UINT32_MAX, t1 = 0;
+    for (int k = 0; k < nz; ++k) {
+      const uint32_t c = (uint32_t)ja[k], w = c >> 6, t = w >> 6;
+      bits[w] |= 1ull << (c & 63);
+      top[t] |= 1ull << (w & 63);
+      t0 = std::min(t0, t);
+      t1 = std::max(t1, t);
+    }
+    int n = 0;
+    each_word(t0, t1, [&](uint32_t w) {
+      before[w] = (uint16_t)n;
+      for (uint64_t y = bits[w]; y; y &= y - 1) {
+        out.push_back((int32_t)(w * 64 + (uint32_t)__builtin_ctzll(y)));
+        ++n;
+      }
+    });
+    for (int k = 0; k < nz; ++k) {
+      const uint32_t c = (uint32_t)ja[k], w = c >> 6;
+      const uint64_t lower = bits[w] & ((1ull << (c & 63)) - 1);
+      lidx[k] = (uint16_t)(before[w] + __builtin_popcountll(lower));
+    }
+    each_word(t0, t1, [&](uint32_t w) { bits[w] = 0; });
+    for (uint32_t t = t0; nz && t <= t1; ++t) top[t] = 0;
+    return n;
+  }
+  template <class F>
+  void each_word(uint32_t t0, uint32_t t1, F f) const {
+    if (t0 > t1) return;
+    for (uint32_t t = t0; t <= t1; ++t)
+      for (uint64_t x = top[t]; x; x &= x - 1) f(t * 64 + (uint32_t)__builtin_ctzll(x));
+  }
+};
+
 }  // namespace
 
 void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* ja, TileSet& t,
@@ -53,46 +97,40 @@ void build_tiles(int64_t nrow, int64_t ncol, const int64_t* ia, const int32_t* j
     if (w.nz > kTileNnz) t.has_long = true;
     r = r1;
   }
-  t.lidx.assign((size_t)ia[nrow], 0);
+  t.lidx.resize((size_t)ia[nrow]);
   const int64_t nt = (int64_t)t.tile.size();
-  const int64_t per = 512;   // tiles a piece of work: some million nonzeros
+  const int64_t per = 64;   // tiles a piece of work: some hundred thousand nonzeros
   const int64_t npiece = (nt + per - 1) / per;
+  const int64_t nth = std::min<int64_t>(
+      npiece, std::min(16u, std::max(1u, std::thread::hardware_concurrency())));
   std::vector<std::vector<int32_t>> cols((size_t)npiece);
   std::atomic<int64_t> next{0};
-  auto work = [&] {
-    std::vector<int32_t> at((size_t)ncol, -1);
-    std::vector<int32_t> u;
-    for (int64_t p; (p = next++) < npiece;) {
+  on_threads(nth, [&] {
+    ColumnSet set(ncol);
+    for (int64_t p; (p = next++) < npiece;)
       for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) {
         Tile& w = t.tile[i];
-        if (w.nz > kTileNnz) continue;
-        u.clear();
-        for (int64_t k = w.k0; k < (int64_t)w.k0 + w.nz; ++k)
-          if (at[ja[k]] < 0) {
-            at[ja[k]] = 0;
-            u.push_back(ja[k]);
-          }
-        std::sort(u.begin(), u.end());
-        for (size_t k = 0; k < u.size(); ++k) at[u[k]] = (int32_t)k;
-        for (int64_t k = w.k0; k < (int64_t)w.k0 + w.nz; ++k) t.lidx[k] = (uint16_t)at[ja[k]];
-        for (int32_t c : u) at[c] = -1;
+        uint16_t* l = t.lidx.data() + w.k0;
+        if (w.nz > kTileNnz) {
+          std::fill(l, l + w.nz, (uint16_t)0);
+          continue;
+        }
         w.u0 = (int)cols[p].size();
-        w.nu = (int)u.size();
-        cols[p].insert(cols[p].end(), u.begin(), u.end());
+        w.nu = set.list(ja + w.k0, w.nz, l, cols[p]);
       }
+  });
+  // the pieces' lists after one another
+  std::vector<int64_t> base((size_t)npiece + 1, 0);
+  for (int64_t p = 0; p < npiece; ++p) base[p + 1] = base[p] + (int64_t)cols[p].size();
+  t.ucol.resize((size_t)base[npiece]);
+  next = 0;
+  on_threads(nth, [&] {
+    for (int64_t p; (p = next++) < npiece;) {
+      std::copy(cols[p].begin(), cols[p].end(), t.ucol.begin() + base[p]);
+      for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) t.tile[i].u0 += (int)base[p];
     }
-  };
-  const int64_t nth = std::min<int64_t>(
-      npiece, std::min(8u, std::max(1u, std::thread::hardware_concurrency())));
-  on_threads(nth, work);
-  for (int64_t p = 0; p < npiece; ++p) {
-    const int base = (int)t.ucol.size();
-    for (int64_t i = p * per; i < std::min(nt, (p + 1) * per); ++i) {
-      t.tile[i].u0 += base;
-      t.nwide += t.tile[i].nu > kTileCols;
-    }
-    t.ucol.insert(t.ucol.end(), cols[p].begin(), cols[p].end());
-  }
+  });
+  for (const Tile& w : t.tile) t.nwide += w.nu > kTileCols;
 }
 
 }  // namespace xg

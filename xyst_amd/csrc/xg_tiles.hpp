@@ -11,6 +11,9 @@
 // a nonzero costs 2 bytes of index instead of 4 (with the lists, 3.1).
 #pragma once
 #include <cstdint>
+#include <memory>
+#include <new>
+#include <utility>
 #include <vector>
 
 namespace xg {
@@ -37,12 +40,28 @@ struct TileMat {
   const uint16_t* lidx = nullptr;
 };
 
+// std::vector whose new elements are left as they are: they are written by
+// several threads, which then touch the pages first
+template <class T>
+struct NoInit : std::allocator<T> {
+  template <class U>
+  struct rebind {
+    using other = NoInit<U>;
+  };
+  template <class U>
+  void construct(U* p) noexcept { ::new ((void*)p) U; }
+  template <class U, class... A>
+  void construct(U* p, A&&... a) { ::new ((void*)p) U(std::forward<A>(a)...); }
+};
+template <class T>
+using RawVector = std::vector<T, NoInit<T>>;
+
 struct TileSet {
   bool has_long = false;        // a row is longer than a tile
   int64_t nwide = 0;            // tiles with more than kTileCols columns
   std::vector<Tile> tile;
-  std::vector<int32_t> ucol;    // the tiles' columns
-  std::vector<uint16_t> lidx;   // per nonzero: position in its tile's list
+  RawVector<int32_t> ucol;      // the tiles' columns
+  RawVector<uint16_t> lidx;   // per nonzero: position in its tile's list
 };
 
 // Tiles of the matrix with row offsets ia (nrow + 1, from 0) and columns ja
