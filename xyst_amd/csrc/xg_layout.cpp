@@ -103,6 +103,16 @@ static void full_lists(int npoin, const std::vector<int>& p, const std::vector<i
   }
 }
 
+// Sorts items by key(item), ties by item; the keys are formed once, in `keyed`.
+template <class Key>
+static void sort_by_key(std::vector<int64_t>& items,
+                        std::vector<std::pair<uint64_t, int64_t>>& keyed, Key key) {
+  keyed.clear();
+  for (int64_t i : items) keyed.emplace_back(key(i), i);
+  std::sort(keyed.begin(), keyed.end());
+  for (size_t k = 0; k < items.size(); ++k) items[k] = keyed[k].second;
+}
+
 // Appends a chunk's entries (local node, slot | sign) grouped by node, each
 // node's in the order given, and every local node's entry end.
 static void group_entries(const std::vector<std::pair<int, uint16_t>>& ent, int nloc,
@@ -225,26 +235,38 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     for (int a = 0; a < 3; ++a)
       if ((a < 1 || b[a] != b[0]) && (a < 2 || b[a] != b[1])) bfaces[b[a]].push_back(f);
   }
+  size_t nitem = 0, nface = 0;   // an edge of two gather blocks is in both
+  for (int b = 0; b < nblk; ++b) {
+    nitem += bedges[b].size();
+    nface += bfaces[b].size();
+  }
+  for (auto* v : {&L.dx, &L.dy, &L.dz}) v->reserve(nitem);
+  for (auto* v : {&L.ep, &L.eq}) v->reserve(nitem);
+  L.elpq.reserve(nitem);
+  L.eidx.reserve(nitem);
+  L.entries.reserve(2 * nitem + 3 * nface + 3 * (size_t)chunk_slots);
   L.blk.resize(nblk);
   std::vector<std::vector<std::pair<int,int>>> fix(npoin);   // node -> (block, slot)
   int nslot = 0;
   std::vector<int> local(npoin, -1);
+  std::vector<std::pair<uint64_t, int64_t>> keyed;
   for (int b = 0; b < nblk; ++b) {
     Block& B = L.blk[b];
     B.own0 = bstart[b];
     B.nown = bstart[b + 1] - bstart[b];
     // halo: nodes touched by owned items outside the block, ascending
     std::vector<int> halo;
-    for (int64_t e : bedges[b]) {
-      for (int m : {p[e], q[e]})
-        if (m >= bstart[b + 1] || m < bstart[b]) halo.push_back(m);
-    }
+    auto touch = [&](int m) {
+      if ((m >= bstart[b + 1] || m < bstart[b]) && local[m] != -2) {
+        local[m] = -2;
+        halo.push_back(m);
+      }
+    };
+    for (int64_t e : bedges[b])
+      for (int m : {p[e], q[e]}) touch(m);
     for (int64_t f : bfaces[b])
-      for (int a = 0; a < 3; ++a)
-        if (tri[f * 3 + a] >= bstart[b + 1] || tri[f * 3 + a] < bstart[b])
-          halo.push_back(tri[f * 3 + a]);
+      for (int a = 0; a < 3; ++a) touch(tri[f * 3 + a]);
     std::sort(halo.begin(), halo.end());
-    halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
     B.nloc = B.nown + (int)halo.size();
     if (B.nloc > block_cap) {
       err = "layout: block exceeds LDS capacity";
@@ -261,10 +283,9 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     for (size_t h = 0; h < halo.size(); ++h) local[halo[h]] = B.nown + (int)h;
     // edges ordered by (smaller local end, larger local end) for locality
     auto& E = bedges[b];
-    std::sort(E.begin(), E.end(), [&](int64_t a, int64_t c) {
-      int a0 = std::min(local[p[a]], local[q[a]]), a1 = std::max(local[p[a]], local[q[a]]);
-      int c0 = std::min(local[p[c]], local[q[c]]), c1 = std::max(local[p[c]], local[q[c]]);
-      return a0 != c0 ? a0 < c0 : a1 < c1;
+    sort_by_key(E, keyed, [&](int64_t e) {
+      const uint64_t a = local[p[e]], c = local[q[e]];
+      return (std::min(a, c) << 32) | std::max(a, c);
     });
     B.chunk0 = (int)L.chunks.size();
     // chunk builder: entries (local node, slot | sign) grouped by node, with
@@ -549,17 +570,16 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
     full_lists(npoin, p, q, uoff, up);
   else
     upper_lists(npoin, p, q, uoff, up);
-  for (int i = 0; i < npoin; ++i) {
-    auto b = up.begin() + uoff[i], e = up.begin() + uoff[i + 1];
-    std::sort(b, e);
-  }
   {  // compact duplicates
     std::vector<int64_t> o2(npoin + 1, 0);
-    std::vector<int> u2;
+    std::vector<int> u2, seen(npoin, -1);
     u2.reserve(up.size() / 2);
     for (int i = 0; i < npoin; ++i) {
       for (int64_t k = uoff[i]; k < uoff[i + 1]; ++k)
-        if (k == uoff[i] || up[k] != up[k - 1]) u2.push_back(up[k]);
+        if (seen[up[k]] != i) {
+          seen[up[k]] = i;
+          u2.push_back(up[k]);
+        }
       o2[i + 1] = (int64_t)u2.size();
     }
     uoff.swap(o2);
@@ -591,17 +611,21 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
   std::vector<std::vector<std::pair<int,int>>> fix(npoin);
   int nslot = 0;
   std::vector<int> local(npoin, -1);
+  std::vector<std::pair<uint64_t, int64_t>> keyed;
   for (int b = 0; b < nblk; ++b) {
     Block& B = L.blk[b];
     B.own0 = bstart[b];
     B.nown = bstart[b + 1] - bstart[b];
     std::vector<int> halo;
     for (int64_t e : btets[b])
-      for (int a = 0; a < 4; ++a)
-        if ((int)inpoel[e * 4 + a] >= bstart[b + 1] || (int)inpoel[e * 4 + a] < bstart[b])
-          halo.push_back((int)inpoel[e * 4 + a]);
+      for (int a = 0; a < 4; ++a) {
+        const int m = (int)inpoel[e * 4 + a];
+        if ((m >= bstart[b + 1] || m < bstart[b]) && local[m] != -2) {
+          local[m] = -2;
+          halo.push_back(m);
+        }
+      }
     std::sort(halo.begin(), halo.end());
-    halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
     B.nloc = B.nown + (int)halo.size();
     if (B.nloc > block_cap) {
       err = "kozak layout: block exceeds LDS capacity";
@@ -617,15 +641,14 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
     for (int i = 0; i < B.nown; ++i) local[B.own0 + i] = i;
     for (size_t h = 0; h < halo.size(); ++h) local[halo[h]] = B.nown + (int)h;
     auto& T = btets[b];
-    auto key = [&](int64_t e) {
+    sort_by_key(T, keyed, [&](int64_t e) {
       int l[4];
       for (int a = 0; a < 4; ++a) l[a] = local[inpoel[e * 4 + a]];
-      std::sort(l, l + 4);
+      for (auto o : {std::pair<int, int>{0, 1}, {2, 3}, {0, 2}, {1, 3}, {1, 2}})
+        if (l[o.first] > l[o.second]) std::swap(l[o.first], l[o.second]);
       return ((uint64_t)l[0] << 48) | ((uint64_t)l[1] << 32) | ((uint64_t)l[2] << 16) |
              (uint64_t)l[3];
-    };
-    std::stable_sort(T.begin(), T.end(),
-                     [&](int64_t a, int64_t c) { return key(a) < key(c); });
+    });
     B.chunk0 = (int)L.chunks.size();
     const auto parts = spread_chunks(T, tets_per_chunk, B.nloc, [&](int64_t e, int* node) {
       int k = 0;
