@@ -5,7 +5,7 @@
 // index and prefetch bound of the kernels must stay inside its list.
 // Input file: int64 npoin, ne, ntri, ntet; int32 p[ne], q[ne], tri[3 ntri],
 // tet[4 ntet].
-// Arguments: FILE KIND(rhs|grad|cho|tet|rows|gradrows) NODES GATHER, for rows
+// Arguments: FILE KIND(rhs|cho|tet|rows|gradrows) NODES GATHER, for rows
 // (node rows, xg_rows.hpp) the lanes per node instead of GATHER, for gradrows
 // (riemann::grad's) the lanes that it has to choose, NODES 0.  NODES 0 of the
 // others: the operator's own choice of blocks, which has to be GATHER.
@@ -142,13 +142,13 @@ int main(int argc, char** argv) {
     for (int64_t e = 0; e < h[3]; ++e)
       for (int a = 0; a < 4; ++a) want[t32[e * 4 + a]] += val(t32[e * 4] + t32[e * 4 + 1], a);
   } else {
-    const bool cho = !std::strcmp(kind, "cho"), grad = !std::strcmp(kind, "grad");
-    cap = cho ? xg::kBlockCap : grad ? xg::kGradCap : xg::kRhsCap;
-    slots = cho ? xg::kChunkSlots : grad ? xg::kGradSlots : xg::kRhsSlots;
+    const bool cho = !std::strcmp(kind, "cho");
+    cap = cho ? xg::kBlockCap : xg::kRhsCap;
+    slots = cho ? xg::kChunkSlots : xg::kRhsSlots;
     std::vector<double> d(3 * p.size(), 1.0);
     std::vector<uint8_t> sym(3 * h[2], 1);
     CHECK((nodes ? xg::build_layout(npoin, p, q, d, h[2], tri.data(), sym.data(), nodes, cap,
-                                    slots, L, err, gather, true)
+                                    slots, L, err, gather, !cho)
            : cho ? xg::build_cho_layout(npoin, p, q, d, h[2], tri.data(), L, err)
                  : xg::build_rhs_layout(npoin, p, q, d, h[2], tri.data(), sym.data(), L, err)) ==
           0);

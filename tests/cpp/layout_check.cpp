@@ -3,11 +3,11 @@
 // direct scatter, bounds-checking every index the device kernels use.
 // Input file (raw little-endian): int64 npoin, ne, ntri; int32 p[ne], q[ne];
 // int32 tri[3*ntri]; uint8 besym[3*ntri].  Optional arguments: owned nodes,
-// block capacity and chunk slots (default: the ChoCG blocks; the rhs blocks
-// are kRhsNodes kRhsCap kRhsSlots), then 1 for a gather layout (the grad
-// blocks: kGradNodes kGradCap kGradSlots 1), whose halo nodes must receive
-// nothing and whose owned sums must be complete without a fix-up.  Prints
-// "ok <stats>" or exits 1.
+// block capacity and chunk slots of blocks whose edges are spread over the
+// chunks (the rhs blocks are kRhsNodes kRhsCap kRhsSlots; default: the ChoCG
+// blocks, whose edges are not), then 1 for a gather layout, whose halo nodes
+// must receive nothing and whose owned sums must be complete without a fix-up.
+// Prints "ok <stats>" or exits 1.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -47,7 +47,7 @@ int main(int argc, char** argv) {
   xg::Layout L;
   std::string err;
   CHECK(xg::build_layout(npoin, p, q, d, ntri, tri.data(), besym.data(), nodes, cap,
-                         slots, L, err, gather) == 0);
+                         slots, L, err, gather, argc >= 5) == 0);
   // direct scatter
   std::vector<double> Rref((size_t)npoin * 5, 0.0), R((size_t)npoin * 5, -1e300);
   for (int64_t e = 0; e < ne; ++e)
@@ -55,14 +55,14 @@ int main(int argc, char** argv) {
       Rref[p[e] * 5 + c] -= eflux(p[e], q[e], c);
       Rref[q[e] * 5 + c] += eflux(p[e], q[e], c);
     }
-  for (int64_t t = 0; t < (gather ? 0 : ntri); ++t)   // gather layouts carry no faces
+  for (int64_t t = 0; t < ntri; ++t)
     for (int a = 0; a < 3; ++a)
       for (int c = 0; c < 5; ++c)
         Rref[tri[t * 3 + a] * 5 + c] += fflux(tri[t * 3], tri[t * 3 + 1], tri[t * 3 + 2], a, c);
   // emulate k_rhs_blocks: local node data, per-thread node accumulators
   std::vector<double> S((size_t)L.nslot * 5, -1e300);
-  if (gather)   // edges between blocks twice, no faces, no halo partials
-    CHECK((int64_t)L.elpq.size() >= ne && L.fab.empty() && L.nslot == 0 &&
+  if (gather)   // edges and faces of several blocks in each, no halo partials
+    CHECK((int64_t)L.elpq.size() >= ne && (int64_t)L.fab.size() >= ntri && L.nslot == 0 &&
           L.fx_node.empty());
   else
     CHECK((int64_t)L.elpq.size() == ne && (int64_t)L.fab.size() == ntri);
@@ -97,7 +97,7 @@ int main(int argc, char** argv) {
           for (int c = 0; c < 5; ++c) F[t * 5 + c] = eflux(glob[lp], glob[lq], c);
         } else {
           int ff = C.first + t;
-          CHECK(ff >= 0 && ff < ntri);
+          CHECK(ff >= 0 && ff < (int64_t)L.fab.size());
           int la = L.fab[ff] & 0xffff, lb = L.fab[ff] >> 16, lc = L.fcs[ff] & 0xffff;
           CHECK(la < B.nloc && lb < B.nloc && lc < B.nloc);
           CHECK((int)(L.fcs[ff] >> 16) < 8);

@@ -315,10 +315,11 @@ struct FcgRow {
 // ConjugateGradients::x after iteration j - 1 runs here: every workgroup
 // takes the same sums and the first one records the stop for this iteration's
 // update kernel, which passes it on to the later iterations (xg_stop.hpp).
-// An iteration (this and k_cg_update) moves 12 nnz + 44 n bytes of matrix
-// and pairs and 76 n of vectors in FP64: 15 us at 64^3 (274,625 rows) at the
-// copy rate, 26 us measured (37 before the loads were put ahead of the
-// scalars, 28 before the column lists); 62 us at 100^3, 81 before.
+// An iteration (this and k_cg_update) moves in FP64 10 nnz bytes of values
+// and ids, 4 a listed column (0.2 nnz in compact cells), 36 n of offsets, pairs
+// and results and 72 n in the update: 73 MB at 64^3 (274,625 rows), 14 us at
+// the copy rate (5.1 TB/s), 26 us measured (37 before the loads were put ahead
+// of the scalars, 28 before the column lists); 62 us at 100^3, 81 before.
 // COLS: columns loaded a tile ahead.  Four in FP32 where more than an eighth of
 // the tiles list more than three hold (band numberings from 160^3 on: RCM at
 // 160^3 190 -> 187 us an iteration, at 192^3 320 -> 310); elsewhere three

@@ -558,8 +558,9 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
 // Limit coefficients C+/- (KozCG.cpp:1005-1024) from the owners' bounds Q and
 // the halo bounds S of the node's slots (max for Q+, min for Q-), one thread
 // per node and component (neighbouring threads read neighbouring words).
-// Bound by memory: 320 bytes a node, 64 us on 96^3 (4.6 TB/s); 35 + 48 us
-// while a pass of its own merged the bounds first.
+// Bound by memory: 292 bytes a node and 84 a halo slot, 0.68 a node on 96^3:
+// 318 MB, 64 us (5.0 TB/s); 35 + 48 us while a pass of its own merged the
+// bounds first.
 template <int NC>
 __global__ __launch_bounds__(kBlock) void k_kozcg_coef(
     int npoin, const double* __restrict__ W, const double* __restrict__ vol,
@@ -711,9 +712,9 @@ __global__ __launch_bounds__(kKozThreads) __attribute__((amdgpu_waves_per_eu(4))
 // new solution (KozCG.cpp:1144-1160), NC components per node; Un receives
 // the old one.  A: the owners' limited contributions (without FCT the rhs),
 // S the halo partials of the node's slots, added in block order.  Bound by
-// memory: 200 bytes a node, 51 us on 96^3 (19 + 30 us and a launch with a
-// fix-up pass of its own).  dtp (nullable): the nodes' local time steps
-// without FCT.
+// memory: 212 bytes a node and 44 a halo slot, 221 MB on 96^3: 51 us (4.3
+// TB/s; 19 + 30 us and a launch with a fix-up pass of its own).  dtp
+// (nullable): the nodes' local time steps without FCT.
 template <bool FCT, int NC>
 __global__ __launch_bounds__(kBlock) void k_kozcg_solve(
     int npoin, double dt, const double* __restrict__ dtp, const double* __restrict__ UL,

@@ -18,9 +18,10 @@
 // The chorin operators use blocks of up to kBlockCap nodes with 1024-slot
 // chunks (each node thread gathers the terms of the chunk edges that touch
 // it); riemann::rhs builds its own layout of kRhsCap-node blocks and 512-slot
-// chunks, two workgroups per CU.  riemann::grad, whose per-edge work is
-// small, uses a gather layout (see build_layout): edges between two blocks
-// are evaluated in both, so no block leaves partial sums behind.
+// chunks, two workgroups per CU.  On small meshes both use gather blocks (see
+// build_layout): edges and faces between two blocks are evaluated in both, so
+// no block leaves partial sums behind.  riemann::grad, whose per-edge work is
+// small, uses node rows (build_rows).
 //
 // The layout is fastest when node ids are block-contiguous and spatially
 // compact (xg_mesh_block_order), but is correct for any numbering.
@@ -181,8 +182,7 @@ static std::vector<std::vector<int64_t>> spread_chunks(const std::vector<int64_t
 int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                  const std::vector<double>& d, int64_t ntri, const int* tri,
                  const uint8_t* besym, int block_nodes, int block_cap,
-                 int chunk_slots, Layout& L, std::string& err, bool gather,
-                 bool gather_faces, bool spread) {
+                 int chunk_slots, Layout& L, std::string& err, bool gather, bool spread) {
   const int64_t ne = (int64_t)p.size();
   L = Layout();
   if (chunk_slots < 3 || chunk_slots > kChunkSlots) {
@@ -194,7 +194,7 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
   // lies beyond it), or both ways for a gather layout
   std::vector<int64_t> uoff;
   std::vector<int> up;
-  if (gather && gather_faces && ntri) {
+  if (gather) {
     // the faces' edges too: a block holds the nodes of every face it takes
     std::vector<int> pf(p), qf(q);
     for (int64_t f = 0; f < ntri; ++f)
@@ -203,8 +203,6 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
         qf.push_back(tri[f * 3 + (a + 1) % 3]);
       }
     full_lists(npoin, pf, qf, uoff, up);
-  } else if (gather) {
-    full_lists(npoin, p, q, uoff, up);
   } else {
     upper_lists(npoin, p, q, uoff, up);
   }
@@ -225,7 +223,7 @@ int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q
     bedges[b0].push_back(e);
     if (gather && b1 != b0) bedges[b1].push_back(e);
   }
-  for (int64_t f = 0; f < (gather && !gather_faces ? 0 : ntri); ++f) {
+  for (int64_t f = 0; f < ntri; ++f) {
     const int* N = tri + f * 3;
     if (!gather) {
       bfaces[blk_of[std::min(N[0], std::min(N[1], N[2]))]].push_back(f);
@@ -714,7 +712,7 @@ int build_rhs_layout(int npoin, const std::vector<int>& p, const std::vector<int
                      const uint8_t* besym, Layout& L, std::string& err) {
   return by_plan(rhs_blocks(npoin), kRhsNodes, err, [&](const BlockPlan& b, std::string& e) {
     return build_layout(npoin, p, q, d, ntri, tri, besym, b.nodes, kRhsCap, kRhsSlots, L, e,
-                        b.gather, true);
+                        b.gather);
   });
 }
 
@@ -732,7 +730,7 @@ int build_cho_layout(int npoin, const std::vector<int>& p, const std::vector<int
   const std::vector<uint8_t> nosym(ntri * 3 + 1, 0);
   return by_plan(cho_blocks(npoin), kBlockNodes, err, [&](const BlockPlan& b, std::string& e) {
     return build_layout(npoin, p, q, d, ntri, tri, nosym.data(), b.nodes, kBlockCap, kChunkSlots,
-                        L, e, b.gather, true, false);
+                        L, e, b.gather, false);
   });
 }
 

@@ -19,10 +19,8 @@ constexpr int kBlockNodes = 432;
 // riemann::grad blocks (node rows, xg_rows.hpp): one thread per owned node,
 // the primitive state of the local ones in LDS (30,720 bytes: five
 // workgroups share a CU); small meshes: 16 nodes, four lanes each.
-// kGradSlots: chunk slots where a gather layout is built at these sizes.
 constexpr int kGradNodes = 384;
 constexpr int kGradCap = 768;
-constexpr int kGradSlots = 1024;
 constexpr int kGradSmallCap = 256;
 // riemann::rhs has blocks of its own, small enough that two 512-thread
 // workgroups share a CU: 23 doubles per local node, 512 flux slots of 5
@@ -69,7 +67,7 @@ struct Layout {
 // KozCG blocks: a block stages U (5) and coordinates (3) of up to kKozCap
 // nodes in LDS beside one chunk's corner values (5 doubles per slot); a
 // chunk holds kKozPairSlots / 4 tets, two threads per tet.  At 1024 slots
-// and 512 nodes the largest of the KozCG block kernels takes 78,848 bytes of
+// and 512 nodes the largest of the KozCG block kernels takes 80,896 bytes of
 // LDS, so two share a CU.
 constexpr int kKozCap = 512;
 constexpr int kKozNodes = 384;
@@ -101,14 +99,13 @@ int build_tet_layout(int npoin, int64_t ntet, const size_t* inpoel,
 // between two blocks are in both), its halo is every outside end of those,
 // and its entries add each edge to its owned ends only, so every owned sum
 // is complete in its block: no halo slots (Block::slot0 is -1) and no
-// fix-up lists.  gather_faces: likewise every boundary face that touches one
-// of its nodes; without it a gather layout carries no boundary faces.
+// fix-up lists.  Likewise every boundary face that touches one of its nodes.
 // spread: a node's edges over the chunks of its block (spread_chunks).
 int build_layout(int npoin, const std::vector<int>& p, const std::vector<int>& q,
                  const std::vector<double>& d, int64_t ntri, const int* tri,
                  const uint8_t* besym, int block_nodes, int block_cap,
                  int chunk_slots, Layout& L, std::string& err, bool gather = false,
-                 bool gather_faces = false, bool spread = true);
+                 bool spread = true);
 
 // Blocks of small meshes.  At the full block sizes a mesh of a few thousand
 // nodes fills a few of the 256 CUs, and each block walks its chunks alone: so

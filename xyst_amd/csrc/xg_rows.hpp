@@ -35,7 +35,7 @@ struct RowLayout {
   std::vector<uint16_t> nb;         // neighbour, block-local
   std::vector<double> dx, dy, dz;   // signed integrals
   std::vector<int64_t> eidx;        // input edge of each entry (-1: padding)
-  std::vector<uint32_t> fab, fcs;   // a | b << 16; c | this corner << 16
+  std::vector<uint32_t> fab, fcs;   // a | b << 16; c | this corner << 16 (checks)
   std::vector<int64_t> fidx;        // input face of each face entry (-1: padding)
 };
 
