@@ -160,7 +160,9 @@ int xg_mesh_neumann(int64_t npoin, const double* x, const double* y,
  * the three superedge groups (dsupedge[k], dsupint[k]: nsup[k] tets (4 ids,
  * 6x3 D), triangles (3 ids, 3x3 D), edges (2 ids, 3 D)), boundary triangles
  * and their per-node symmetry flags besym.  The device layout (edge list,
- * deterministic scatter order, boundary gather lists) is built here once. */
+ * deterministic scatter order, boundary gather lists) is built here once.
+ * XG_EUNSUPPORTED for a node of more than 767 neighbours, or of more than 311
+ * with larger ids. */
 int xg_mesh_upload(xg_ctx* ctx, int64_t npoin,
                    const double* x, const double* y, const double* z,
                    const int64_t nsup[3],
@@ -277,7 +279,8 @@ int xg_mesh_device_bytes(const xg_ctx* ctx, int64_t* bytes);
 
 /* The mesh arguments of kozak::rhs (Kozak.hpp:19-27): tet connectivity
  * inpoel (4 ids per tet) and coordinates.  The device layout (node blocks,
- * tets by block, deterministic scatter order) is built here once. */
+ * tets by block, deterministic scatter order) is built here once.
+ * XG_EUNSUPPORTED for a node of more than 511 neighbours with larger ids. */
 int xg_kozak_upload(xg_ctx* ctx, int64_t npoin, const double* x,
                     const double* y, const double* z, int64_t ntet,
                     const size_t* inpoel);
@@ -370,7 +373,8 @@ typedef struct {
 /* The mesh arguments of the chorin:: operators (Chorin.hpp:19-70): the
  * superedges of ChoCG::domsuped with 5 values per edge integral
  * (ChoCG.cpp:398-445, 687-813: normal components, J/120,
- * dot(grad_p,grad_q)/J/6), coordinates and boundary triangles. */
+ * dot(grad_p,grad_q)/J/6), coordinates and boundary triangles.
+ * XG_EUNSUPPORTED for a node of more than 615 neighbours with larger ids. */
 int xg_chocg_upload(xg_ctx* ctx, int64_t npoin, const double* x,
                     const double* y, const double* z, const int64_t nsup[3],
                     const size_t* dsupedge0, const double* dsupint0,
