@@ -12,8 +12,8 @@
 // CG's SpMV and beta read it.  Every kernel has a fixed summation order, so
 // applications are bitwise reproducible.
 //
-// What bounds it: bytes on the finest level (B twice, P and R: some 90 MB at
-// 64^3 in FP32, 18 us at the copy rate) and the latency of a launch and of
+// What bounds it: bytes on the finest level (B twice, P and R: 82 MB at 64^3
+// in FP32, 16 us at the copy rate) and the latency of a launch and of
 // its chain of loads on the others (4 to 6 us each).
 #include <hip/hip_runtime.h>
 
